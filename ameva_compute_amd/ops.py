@@ -43,6 +43,8 @@ Q8_0_MMA = 1008
 # the same layouts with f16 q * d in place of f16 q: the scaled batched MUL_MAT (AMV_ACT_Q8_K_DEQ / AMV_ACT_Q8_0_DEQ)
 Q8_K_DEQ = 1115
 Q8_0_DEQ = 1108
+# Q8_0 activations with the scratch in which the batched Q4_0 MUL_MAT keeps their 6-bit digits (AMV_ACT_Q8_0_F6)
+Q8_0_F6 = 1208
 
 
 # The batched MUL_MAT's arithmetic above MMQ16_MIN_M tokens: "exact" (the default: exact per-block integer sums and
@@ -65,6 +67,14 @@ def act_type(wtype: int, m: int = 1, exact: bool | None = None) -> int:
     if wtype == Q4_K and MMQ_MIN_M <= m <= MMQ16_MIN_M:
         return Q8_K_MMA
     return Q8_K if wtype in (Q4_K, Q6_K) else Q8_0
+
+
+def gemm_act_type(wtype: int, m: int) -> int:
+    """The activation layout the fastest MUL_MAT of m tokens in MMQ_FORM's arithmetic takes: act_type's, with the digits'
+    scratch for Q4_0 above MMQ16_MIN_M tokens in the exact form (the same results from the 6-bit matrix instruction)."""
+    if wtype == Q4_0 and m > MMQ16_MIN_M and MMQ_FORM == "exact":
+        return Q8_0_F6
+    return act_type(wtype, m)
 
 
 def act_layout(wtype: int, act: torch.Tensor, m: int, k: int) -> int:
@@ -124,7 +134,7 @@ def quantize_act(x: torch.Tensor, atype: int = Q8_0, rule: int = Q8_X86, ggml: b
     if n < 0:
         raise ValueError(f"quantize_act: type {atype} cannot hold rows of {k}")
     act = torch.empty(n, dtype=torch.uint8, device=x.device)
-    gt = Q8_K if atype in (Q8_K_MMA, Q8_K_DEQ) else Q8_0 if atype in (Q8_0_MMA, Q8_0_DEQ) else atype
+    gt = Q8_K if atype in (Q8_K_MMA, Q8_K_DEQ) else Q8_0 if atype in (Q8_0_MMA, Q8_0_DEQ, Q8_0_F6) else atype
     g = torch.empty((m, ggml_row_bytes(gt, k)), dtype=torch.uint8, device=x.device) if ggml else None
     check(lib().amv_quantize_act(atype, x2.data_ptr(), m, k, rule, _ptr(g), act.data_ptr(), _stream()),
           "amv_quantize_act")
@@ -270,7 +280,7 @@ def mul_mat(w: QWeight, x: torch.Tensor, rule: int = Q8_X86) -> torch.Tensor:
     x2 = x.reshape(-1, x.shape[-1])
     if x2.shape[1] != w.k:
         raise ValueError(f"mul_mat: k mismatch {x2.shape[1]} != {w.k}")
-    at = act_type(w.type, x2.shape[0])
+    at = gemm_act_type(w.type, x2.shape[0])
     act, _ = quantize_act(x2, at, rule)
     return mul_mat_q(w, act, x2.shape[0], act_t=at)
 
