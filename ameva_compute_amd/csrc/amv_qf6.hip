@@ -258,6 +258,7 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2))) v
         F6_STEP(3, sw3, sw0, b, a)
     }
 #undef F6_STEP
+    F6_WAIT(0);  // the last step's prefetch may still write LDS
     if constexpr (KG == 2 && !SUMS) {  // the second group's sums join the first's, 4 BM x 4 floats at a time
         float* red = reinterpret_cast<float*>(sA16a);
         constexpr int PER = 2 * 4 * BM * 4 / 256;
