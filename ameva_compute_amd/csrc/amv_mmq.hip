@@ -473,42 +473,32 @@ static void mmq_launch(const uint8_t* wq, const uint16_t* wd, int N, int nb, con
 template <int WT, bool SUMS>
 static void mmq_dispatch(const uint8_t* wq, const uint16_t* wd, int N, int nb, const int8_t* aq, const int2* ameta,
                          int M, float* dst, int64_t ldd, int32_t* sums, hipStream_t st) {
-    const int64_t row_tiles = (N + 127) / 128;
     if (mmq_sb_launch<WT, SUMS>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st)) return;
-    if (M <= 32) {
-        // small batches: one 16 TI x 16 TJ tile per workgroup, its 4 waves splitting k; the largest row tile that
-        // still gives >= 224 workgroups (M = 16: 14336 x 4096 28 us with TI = 4, 4096 x 14336 41 us with TI = 1)
-        const int ti = N / 64 >= 224 ? 4 : (N / 32 >= 224 ? 2 : 1);
-        if (M <= 16) {
-            if (ti == 4) mmq_launch<WT, SUMS, 4, 1, 2, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
-            else if (ti == 2) mmq_launch<WT, SUMS, 2, 1, 4, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
-            else mmq_launch<WT, SUMS, 1, 1, 4, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
-        } else {
-            if (ti == 4) mmq_launch<WT, SUMS, 4, 2, 2, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
-            else if (ti == 2) mmq_launch<WT, SUMS, 2, 2, 2, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
-            else mmq_launch<WT, SUMS, 1, 2, 4, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
-        }
-    } else if (M <= 64 || row_tiles * ((M + 127) / 128) < 192)
-        mmq_launch<WT, SUMS, 4, 2, 2>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
-    else mmq_launch<WT, SUMS, 4, 4, 1>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
+    // one 16 TI x 16 TJ tile per workgroup, its 4 waves splitting k; the largest row tile that still gives >= 224
+    // workgroups (M = 16: 14336 x 4096 28 us with TI = 4, 4096 x 14336 41 us with TI = 1)
+    const int ti = N / 64 >= 224 ? 4 : (N / 32 >= 224 ? 2 : 1);
+    if (M <= 16) {
+        if (ti == 4) mmq_launch<WT, SUMS, 4, 1, 2, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
+        else if (ti == 2) mmq_launch<WT, SUMS, 2, 1, 4, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
+        else mmq_launch<WT, SUMS, 1, 1, 4, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
+    } else {
+        if (ti == 4) mmq_launch<WT, SUMS, 4, 2, 2, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
+        else if (ti == 2) mmq_launch<WT, SUMS, 2, 2, 2, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
+        else mmq_launch<WT, SUMS, 1, 2, 4, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
+    }
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// Q4_K x Q8_K for many tokens on the f16 matrix cores (v_mfma_f32_32x32x16_f16), with ggml's integer structure kept
-// exactly: per 256-weight super-block ggml forms I1 = sum_u sc_u * dot_u (dot_u the int dot of 32-weight unit u) and
-// I2 = sum_u m_u * bsum_u, then adds d_a * (d * I1 - dmin * I2). Here the weight operand carries sc_u * q (<= 945)
-// and the activation operand q_a (<= 127), both exact in f16, so the MFMA's f32 sums are exact integers while they
-// stay below 2^24: each super-block is summed in two accumulators of 128 products (<= 15.4 M each), whose f32 sum
-// rounds exactly as ggml's conversion of the int32 I1. I2 is one more exact MFMA per super-block (m_u against the
-// f16 sums per 16 of the activations). The f32 epilogue thus runs once per 256 weights instead of per 32.
-// Roles: A = activations (32 tokens x 16 k), B = weights (16 k x 32 rows), so lane l's output column is weight row
-// l % 32 (its own scales) and its 16 outputs are tokens 8 (r / 4) + 4 (l / 32) + r % 4. k slots: lane half h owns
-// the weights 128 h .. 128 h + 127 of a super-block (bytes 64 h .. 64 h + 63 of its 128 qs bytes); step s (0..15)
-// takes weights 128 h + 8 s .. + 7 (chunk 2 h + s / 8, nibble (s / 4) % 2, bytes 32 (s / 8) + 8 (s % 4) .. + 7).
+// Q4_K x Q8_K of up to 32 tokens on the f16 matrix cores, with ggml's integer structure kept exactly: per 256-weight
+// super-block ggml forms I1 = sum_u sc_u * dot_u (dot_u the int dot of 32-weight unit u) and I2 = sum_u m_u * bsum_u,
+// then adds d_a * (d * I1 - dmin * I2). Here the weight operand carries sc_u * q (<= 945) and the activation operand q_a
+// (<= 127), both exact in f16, so the MFMA's f32 sums are exact integers while they stay below 2^24: each super-block is
+// summed in two accumulators of 128 products (<= 15.4 M each), whose f32 sum rounds exactly as ggml's conversion of the
+// int32 I1. I2 is one more exact MFMA per super-block (m_u against the f16 sums per 16 of the activations). The f32
+// epilogue thus runs once per 256 weights instead of per 32.
 // ---------------------------------------------------------------------------------------------------------------
 typedef _Float16 k4_h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 k4_h2 __attribute__((ext_vector_type(2)));
-typedef float k4_f16v __attribute__((ext_vector_type(16)));
 typedef _Float16 k4_h4 __attribute__((ext_vector_type(4)));
 typedef float k4_f16v4 __attribute__((ext_vector_type(4)));
 
@@ -522,135 +512,6 @@ __device__ __forceinline__ k4_h8 k4_nib_f16(uint32_t x0, uint32_t x1, k4_h2 sc2)
     const k4_h2 p3 = __builtin_bit_cast(k4_h2, __builtin_amdgcn_perm(x1, m64, 0x00070006u));
     const k4_h2 v0 = (p0 - off) * sc2, v1 = (p1 - off) * sc2, v2 = (p2 - off) * sc2, v3 = (p3 - off) * sc2;
     return k4_h8{v0.x, v0.y, v1.x, v1.y, v2.x, v2.y, v3.x, v3.y};
-}
-
-// 33..64 tokens: a workgroup of 2 x 2 waves on 64 rows x 64 TT tokens, each wave one 32 x 32 TT tile over all the
-// super-blocks (smaller batches run k_mmq_q4k_sb).
-template <bool SUMS, int TT>
-__global__ __launch_bounds__(256) void k_mmq_q4k(const uint4* __restrict__ wq, const uint4* __restrict__ wh, int N,
-                                                int nsb, const uint16_t* __restrict__ a16,
-                                                const uint16_t* __restrict__ bs16, const float* __restrict__ dt, int M,
-                                                float* __restrict__ dst, int64_t ldd, int32_t* __restrict__ sums) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, c = lane & 31, h = lane >> 5;
-    const int row0 = blockIdx.x * 64 + 32 * (w & 1);
-    const int tok0 = blockIdx.y * (64 * TT) + 32 * TT * (w >> 1);
-    const int K = nsb * 256;
-    const int row = min(row0 + c, N - 1);
-    const uint4* qrow = wq + (size_t)row * nsb * 8 + 4 * h;  // 8 uint4 of qs per super-block; this half's 4
-    const uint4* hrow = wh + (size_t)row * nsb;
-    const uint16_t* arow[TT];
-    const uint16_t* brow[TT];
-#pragma unroll
-    for (int t = 0; t < TT; ++t) {
-        const int tok = min(tok0 + 32 * t + c, M - 1);
-        arow[t] = a16 + (size_t)tok * K + 128 * h;
-        brow[t] = bs16 + (size_t)tok * (K / 16) + 8 * h;
-    }
-    k4_f16v acc[TT];
-#pragma unroll
-    for (int t = 0; t < TT; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[t][r] = 0.0f;
-
-    // the weights of the next super-block are loaded while this one computes
-    uint4 nq4[4], nhd;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) nq4[i] = qrow[i];
-    nhd = hrow[0];
-    for (int j = 0; j < nsb; ++j) {
-        uint4 q4[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) q4[i] = nq4[i];
-        const uint4 hd = nhd;
-        const int jn = min(j + 1, nsb - 1);  // the last super-block reloads itself (unused)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) nq4[i] = qrow[(size_t)jn * 8 + i];
-        nhd = hrow[jn];
-        // scales and mins of units 4 h .. 4 h + 3 (get_scale_min_k4 on the 12 packed bytes)
-        int scv[4], mv[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) k4_scale_min(4 * h + e, hd.y, hd.z, hd.w, scv[e], mv[e]);
-        k4_f16v C0[TT], C1[TT], I2[TT];
-#pragma unroll
-        for (int t = 0; t < TT; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) C0[t][r] = C1[t][r] = 0.0f;
-#pragma unroll
-        for (int st = 0; st < 16; ++st) {
-            const int jj = st >> 3, nib = (st >> 2) & 1, seg = st & 3;
-            const uint4 v = q4[2 * jj + (seg >> 1)];
-            uint32_t x0 = (seg & 1) ? v.z : v.x, x1 = (seg & 1) ? v.w : v.y;
-            x0 = (x0 >> (4 * nib)) & 0x0F0F0F0Fu;
-            x1 = (x1 >> (4 * nib)) & 0x0F0F0F0Fu;
-            const _Float16 scf = (_Float16)(float)scv[2 * jj + nib];
-            const k4_h8 B = k4_nib_f16(x0, x1, k4_h2{scf, scf});
-#pragma unroll
-            for (int t = 0; t < TT; ++t) {
-                const k4_h8 A = *reinterpret_cast<const k4_h8*>(arow[t] + (size_t)j * 256 + 8 * st);
-                if (st < 8) C0[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A, B, C0[t], 0, 0, 0);
-                else C1[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A, B, C1[t], 0, 0, 0);
-            }
-        }
-        // I2: m of the lane's units against the activation sums per 16 (slot e <-> sum 8 h + e <-> unit 4 h + e / 2)
-        {
-            k4_h8 Bm;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) Bm[e] = (_Float16)(float)mv[e >> 1];
-#pragma unroll
-            for (int t = 0; t < TT; ++t) {
-                const k4_h8 A = *reinterpret_cast<const k4_h8*>(brow[t] + (size_t)j * 16);
-                k4_f16v z;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) z[r] = 0.0f;
-                I2[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A, Bm, z, 0, 0, 0);
-            }
-        }
-        const float d = amv_h2f(hd.x), dmin = amv_h2f(hd.x >> 16);
-#pragma unroll
-        for (int t = 0; t < TT; ++t) {
-#pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4) {
-                const int tk = tok0 + 32 * t + 8 * r4 + 4 * h;  // tokens tk .. tk + 3 of outputs 4 r4 .. 4 r4 + 3
-                float da[4];
-                if (!SUMS) {
-                    if (tk + 3 < M && (M & 3) == 0) {
-                        const float4 d4 = *reinterpret_cast<const float4*>(dt + (size_t)j * M + tk);
-                        da[0] = d4.x; da[1] = d4.y; da[2] = d4.z; da[3] = d4.w;
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) da[e] = dt[(size_t)j * M + min(tk + e, M - 1)];
-                    }
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int r = 4 * r4 + e;
-                    if (SUMS) {
-                        const int tok = tk + e, n = row0 + c;
-                        if (tok < M && n < N) {
-                            int32_t* o = sums + (((size_t)tok * N + n) * nsb + j) * 2;
-                            o[0] = (int)C0[t][r] + (int)C1[t][r];
-                            o[1] = (int)I2[t][r];
-                        }
-                    } else {
-                        const float i1 = C0[t][r] + C1[t][r];
-                        acc[t][r] = fmaf(da[e], fmaf(d, i1, -dmin * I2[t][r]), acc[t][r]);
-                    }
-                }
-            }
-        }
-    }
-    if (!SUMS) {
-        const int n = row0 + c;
-        if (n < N) {
-#pragma unroll
-            for (int t = 0; t < TT; ++t)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int tok = tok0 + 32 * t + 8 * (r >> 2) + 4 * h + (r & 3);
-                    if (tok < M) dst[(size_t)tok * ldd + n] = acc[t][r];
-                }
-        }
-    }
 }
 
 // Small batches (m <= 32) of Q4_K, streamed like k_mmq_sb (k_mmq_q4k_sb). A wave owns TI 16-row weight tiles and
@@ -1113,34 +974,25 @@ static int mmq_q4k(const void* w, int64_t n_rows, int64_t k, const void* act, in
     const uint16_t* a16 = (const uint16_t*)((const uint8_t*)act + L.a16);
     const uint16_t* bs16 = (const uint16_t*)((const uint8_t*)act + L.bs16);
     const float* dt = (const float*)((const uint8_t*)act + L.dt);
-    const unsigned gx = (unsigned)((n_rows + 63) / 64);
-    if (m <= 32) {
-        // small batches, streamed: two 16-row tiles per wave and 4 waves while that leaves >= 256 workgroups, else one
-        // tile and 8 waves splitting the super-blocks (4 for two token tiles)
-        const bool two = (n_rows + 31) / 32 >= 256;
-        const dim3 G((unsigned)(two ? (n_rows + 31) / 32 : (n_rows + 15) / 16));
+    // small batches, streamed: two 16-row tiles per wave and 4 waves while that leaves >= 256 workgroups, else one
+    // tile and 8 waves splitting the super-blocks (4 for two token tiles)
+    const bool two = (n_rows + 31) / 32 >= 256;
+    const dim3 G((unsigned)(two ? (n_rows + 31) / 32 : (n_rows + 15) / 16));
 #define Q4K_SB(TI, TJ, NW)                                                                                           \
     do {                                                                                                              \
-        if (sums) hipLaunchKernelGGL((k_mmq_q4k_sb<TI, TJ, NW, true>), G, dim3(64 * NW), 0, st, wq, wh, (int)n_rows, \
-                                     nsb, a16, bs16, dt, (int)m, dst, ldd, sums);                                     \
-        else hipLaunchKernelGGL((k_mmq_q4k_sb<TI, TJ, NW, false>), G, dim3(64 * NW), 0, st, wq, wh, (int)n_rows, nsb, \
-                                a16, bs16, dt, (int)m, dst, ldd, sums);                                               \
+    if (sums) hipLaunchKernelGGL((k_mmq_q4k_sb<TI, TJ, NW, true>), G, dim3(64 * NW), 0, st, wq, wh, (int)n_rows, \
+                                 nsb, a16, bs16, dt, (int)m, dst, ldd, sums);                                     \
+    else hipLaunchKernelGGL((k_mmq_q4k_sb<TI, TJ, NW, false>), G, dim3(64 * NW), 0, st, wq, wh, (int)n_rows, nsb, \
+                            a16, bs16, dt, (int)m, dst, ldd, sums);                                               \
     } while (0)
-        if (m <= 16) {
-            if (two) Q4K_SB(2, 1, 4);
-            else Q4K_SB(1, 1, 8);
-        } else {
-            if (two) Q4K_SB(2, 2, 4);
-            else Q4K_SB(1, 2, 4);  // 8 waves of this tile would spill registers
-        }
-#undef Q4K_SB
-    } else {  // 33..64 tokens: 64-row x 64-token tiles of 2 x 2 waves
-        const dim3 G(gx, (unsigned)((m + 63) / 64));
-        if (sums) hipLaunchKernelGGL((k_mmq_q4k<true, 1>), G, dim3(256), 0, st, wq, wh, (int)n_rows, nsb, a16, bs16, dt,
-                                     (int)m, dst, ldd, sums);
-        else hipLaunchKernelGGL((k_mmq_q4k<false, 1>), G, dim3(256), 0, st, wq, wh, (int)n_rows, nsb, a16, bs16, dt,
-                                (int)m, dst, ldd, sums);
+    if (m <= 16) {
+        if (two) Q4K_SB(2, 1, 4);
+        else Q4K_SB(1, 1, 8);
+    } else {
+        if (two) Q4K_SB(2, 2, 4);
+        else Q4K_SB(1, 2, 4);  // 8 waves of this tile would spill registers
     }
+#undef Q4K_SB
     return amv_check_launch("amv_mul_mat_q");
 }
 
@@ -1153,9 +1005,11 @@ int amv_qgemm(int wtype, const void* w, int64_t n_rows, int64_t k, const void* a
 int amv_qgemm_f6(const void* w, int64_t n_rows, int64_t k, void* act, int64_t m, float* dst, int64_t ldd, int32_t* sums,
                  hipStream_t st, const float* add);
 
-// Batches above this many tokens go to the tiled kernels (amv_qgemm for the exact layouts and the plain ones, the f16
-// kernels for the scaled DEQ layouts); smaller ones to the k_mmq kernels of this file, which read the plain Q8_0
-// prefix (Q4_0 / Q8_0) or the f16 copies of AMV_ACT_Q8_K_MMA (Q4_K).
+// Batches above QGEMM_MIN_M tokens go to the tiled int8 kernels (amv_qgemm, the plain prefix of every layout; with a DEQ
+// layout from MMQ16_MIN_M tokens to the scaled f16 kernels); smaller ones to the k_mmq kernels of this file, which read the
+// plain Q8_0 prefix (Q4_0 / Q8_0) or the f16 copies of AMV_ACT_Q8_K_MMA (Q4_K). At 32 tokens the latter take 10 (4096 x
+// 4096) to 22 us (14336 x 4096), the tiled ones 16 to 22 from 33 tokens on.
+#define QGEMM_MIN_M 32
 #define MMQ16_MIN_M 64
 
 // q4k_mma: act is AMV_ACT_Q8_K_MMA (the small-batch Q4_K kernels read its f16 copies); with a plain Q8_K act every
@@ -1172,7 +1026,7 @@ static int mmq_impl(int wtype, const void* w, int64_t n_rows, int64_t k, const v
     // Q6_K up to 32 tokens: the streamed small-batch kernel (the plain Q8_K prefix of either layout)
     if (wtype == AMV_T_Q6_K && m <= 32) return mmq_q6k_sb(w, n_rows, k, act, m, dst, ldd, sums, amv_stream(stream));
     // the tiled int8 kernel reads the plain prefix of any layout
-    if (m > MMQ16_MIN_M || wtype == AMV_T_Q6_K || (wtype == AMV_T_Q4_K && !q4k_mma)) {
+    if (m > QGEMM_MIN_M || wtype == AMV_T_Q6_K || (wtype == AMV_T_Q4_K && !q4k_mma)) {
         AMV_REQUIRE((wtype != AMV_T_Q4_K && wtype != AMV_T_Q6_K) || k % 256 == 0,
                     "amv_mul_mat_q: K-quants need k %% 256 == 0");
         AMV_REQUIRE(m * k <= INT32_MAX && m <= 65535LL * 128, "amv_mul_mat_q: too large");
@@ -1223,7 +1077,7 @@ static int mmq_act_impl(const char* fn, int wtype, const void* w, int64_t n_rows
     const bool q80x = act_type == AMV_ACT_Q8_0_MMA || act_type == AMV_ACT_Q8_0_DEQ;
     const bool q8kx = act_type == AMV_ACT_Q8_K_MMA || act_type == AMV_ACT_Q8_K_DEQ;
     // Q6_K batches above 32 tokens run the tiled int8 kernel (up to 32 the streamed k_mmq_q6k_sb)
-    const bool tiled = (m > MMQ16_MIN_M && (((q80x || act_type == AMV_T_Q8_0) && (wtype == AMV_T_Q4_0 || wtype == AMV_T_Q8_0)) ||
+    const bool tiled = (m > (deq ? MMQ16_MIN_M : QGEMM_MIN_M) && (((q80x || act_type == AMV_T_Q8_0) && (wtype == AMV_T_Q4_0 || wtype == AMV_T_Q8_0)) ||
                                             ((q8kx || act_type == AMV_T_Q8_K) && wtype == AMV_T_Q4_K))) ||
                        ((q8kx || act_type == AMV_T_Q8_K) && wtype == AMV_T_Q6_K && m > 32);
     if (add && !(tiled && !deq)) {  // only the exact tiled kernels add the residual in their epilogue

@@ -19,9 +19,8 @@
 // unpacked at staging: 16 nibbles (two dwords) spread to 16 6-bit fields (three dwords) in 10 operations, in an order
 // that the digits follow (f6_elem).
 //
-// Tiling: KG groups of 4 waves, WM x WN, on BM = 32 WM tokens x BN = 32 TW WN weight rows; a wave owns 32 tokens x TW
-// tiles of 32 rows, so the C operand (16 moves) serves TW tiles. The groups take consecutive parts of k and add their
-// sums at the end. A = weight rows, B = tokens: lane l of the result holds token l % 32 and rows 8 (r / 4) + 4 (l / 32)
+// Tiling: 4 waves on 128 tokens x 128 weight rows; a wave owns 32 tokens x 4 tiles of 32 rows, so the C operand (16 moves)
+// serves 4 tiles. A = weight rows, B = tokens: lane l of the result holds token l % 32 and rows 8 (r / 4) + 4 (l / 32)
 // + r % 4. Steps of 64 k, double-buffered in LDS. A workgroup alone on its CU spends its time waiting for loads (1.1 us a
 // step of 2600 cycles with both operands one step ahead in registers, 0.7 with the scheme below), so the weights run
 // four steps ahead in registers and the digits, which need no unpacking, go to LDS directly. Grid order and the split
@@ -35,6 +34,9 @@ typedef unsigned int f6_v4u __attribute__((ext_vector_type(4)));
 typedef float f6_v16 __attribute__((ext_vector_type(16)));
 typedef float f6_v32 __attribute__((ext_vector_type(32)));
 
+#define BM 128  // tokens and weight rows of a tile
+#define BN 128
+#define TW 4    // 32-row tiles of a wave
 #define F6_FMT 2  // E2M3
 // block exponents: a code unit is 2^-3, the high digit counts 16
 #define F6_EXP_LO (127 + 3)
@@ -106,29 +108,25 @@ typedef __attribute__((address_space(3))) void f6_lds;
 // wait until at most n vector memory loads are outstanding (n < 16; the other counters are left alone)
 #define F6_WAIT(n) __builtin_amdgcn_s_waitcnt(0x0f70 | (n))
 
-template <int WM, int WN, int TW, int KG, bool SUMS, bool ADD>
-__global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2))) void k_qgemm_f6(
+template <bool SUMS, bool ADD>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_qgemm_f6(
     const uint8_t* __restrict__ wq, const uint16_t* __restrict__ wd, int N, int nb, const uint4* __restrict__ d16,
     const uint2* __restrict__ d8, const float2* __restrict__ meta, int mp, int M, float* __restrict__ dst, int64_t ldd,
     const float* add, int32_t* __restrict__ sums, int vec, int kb_per, int64_t zstride, int n_tw, int n_tt, int n_z) {
-    constexpr int BM = 32 * WM, BN = 32 * TW * WN;
-    static_assert(BN % 128 == 0 && BM % 64 == 0 && TW % 2 == 0, "staging and outer-product shapes");
     // the two buffers of a step are variables of their own, so that the compiler sees that reads of one do not wait for
     // the loads into the other
-    __shared__ __align__(16) uint4 sA16a[KG][4 * BM], sA16b[KG][4 * BM], sW16a[KG][2 * BN], sW16b[KG][2 * BN];
-    __shared__ __align__(16) uint2 sA8a[KG][4 * BM], sA8b[KG][4 * BM], sW8a[KG][2 * BN], sW8b[KG][2 * BN];
-    __shared__ __align__(16) float2 sMta[KG][2 * BM], sMtb[KG][2 * BM];
-    __shared__ __align__(16) float sDwa[KG][2 * BN], sDwb[KG][2 * BN];
-    const int t = threadIdx.x & 255, kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), c = lane & 31, h = lane >> 5;
-    const int wm = wv % WM, wn = wv / WM;
+    __shared__ __align__(16) uint4 sA16a[4 * BM], sA16b[4 * BM], sW16a[2 * BN], sW16b[2 * BN];
+    __shared__ __align__(16) uint2 sA8a[4 * BM], sA8b[4 * BM], sW8a[2 * BN], sW8b[2 * BN];
+    __shared__ __align__(16) float2 sMta[2 * BM], sMtb[2 * BM];
+    __shared__ __align__(16) float sDwa[2 * BN], sDwb[2 * BN];
+    const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), c = lane & 31, h = lane >> 5;
+    const int wm = wv;
     // tile index: token tile fastest, then the split of k, then the weight tile
     const int T = amv_xcd_tile(blockIdx.x, n_tw * n_z * n_tt);
     const int tt = T % n_tt, tw = (T / n_tt) % n_tw, z = T / (n_tt * n_tw);
     const int n0 = tw * BN, m0 = tt * BM;
-    // this split's blocks, dealt to the KG groups of 4 waves (a group's steps past its blocks have weight scale 0)
-    const int z0 = z * kb_per, z_end = min(nb, z0 + kb_per);
-    const int nsteps = ((z_end - z0 + 1) / 2 + KG - 1) / KG;
-    const int b0 = z0 + 2 * nsteps * kg, b_end = min(z_end, b0 + 2 * nsteps);
+    const int b0 = z * kb_per, b_end = min(nb, b0 + kb_per);
+    const int nsteps = (b_end - b0 + 1) / 2;
     dst += (size_t)z * zstride;
 
     f6_v16 acc[TW];
@@ -140,7 +138,6 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2))) v
     // Weights run four steps ahead in registers (a row's 32 bytes of a step are a quarter of a line, so this is the line
     // being fetched once, early); digits go to LDS without registers, one step ahead. Buffer loads: the per-thread
     // offsets are fixed, the step is a scalar, and rows past N read as zero.
-    static_assert(BN == 128, "one weight block per thread");
     F6W sw0, sw1, sw2, sw3;
     const int blk = t & 1, wrow = t >> 1;
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
@@ -165,20 +162,16 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2))) v
     const auto load_d = [&](uint4* a16, uint2* a8, float2* mt, int step) {
         const int s = min(step, nsteps - 1);
         const uint32_t at = (uint32_t)(b0 + 2 * s) * (uint32_t)mp + (uint32_t)m0;  // (block, token) index
-        if (BM == 128 || wv < BM / 32) {
 #pragma unroll
-            for (int bl = 0; bl < 2; ++bl) {
-                const uint32_t ab = at + bl * (uint32_t)mp;
-                // BM * 32 bytes of a block, 1 KB per wave; BM * 8, 256 per wave
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(r16, (f6_lds*)(a16 + bl * 2 * BM + 64 * wv), 16, 16 * t,
-                                                         ab * 32u, 0, 0);
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rm, (f6_lds*)(mt + bl * BM + 32 * wv), 4, 4 * t, ab * 8u, 0, 0);
-            }
-            // BM * 16 bytes per block: the two blocks' 1 KB pieces dealt to the waves
-            constexpr int PB = BM / 64;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r8, (f6_lds*)(a8 + 128 * wv), 16, 16 * lane + 1024 * (wv % PB),
-                                                     (at + (wv / PB) * (uint32_t)mp) * 16u, 0, 0);
+        for (int bl = 0; bl < 2; ++bl) {
+            const uint32_t ab = at + bl * (uint32_t)mp;
+            // BM * 32 bytes of a block, 1 KB per wave; BM * 8, 256 per wave
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r16, (f6_lds*)(a16 + bl * 2 * BM + 64 * wv), 16, 16 * t, ab * 32u, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rm, (f6_lds*)(mt + bl * BM + 32 * wv), 4, 4 * t, ab * 8u, 0, 0);
         }
+        // BM * 16 bytes per block: the two blocks' 1 KB pieces dealt to the waves
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r8, (f6_lds*)(a8 + 128 * wv), 16, 16 * lane + 1024 * (wv & 1),
+                                                 (at + (wv >> 1) * (uint32_t)mp) * 16u, 0, 0);
         __builtin_amdgcn_sched_barrier(0);  // these before the step's weight loads: the wait below counts on it
     };
     const auto store = [&](const F6W& g, int step, uint4* w16, uint2* w8, float* dw) {
@@ -193,7 +186,7 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2))) v
     const int ea = F6_EXP_LO, eb = h ? F6_EXP_LO : F6_EXP_HI;  // half 0: the high digits
     const auto compute = [&](int step, const uint4* a16, const uint2* a8, const float2* mt,
                              const uint4* w16, const uint2* w8, const float* dw) {
-#pragma unroll KG  // (both blocks at once where one workgroup has the CU: the registers are there)
+#pragma unroll 1
         for (int bl = 0; bl < 2; ++bl) {
             const int tok = 32 * wm + c;
             const uint4 b4 = a16[(bl * BM + tok) * 2 + h];
@@ -208,11 +201,11 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2))) v
                 f6_v32 o;
                 if constexpr (!SUMS) {
                     const f6_v32 zero = {};
-                    o = __builtin_amdgcn_mfma_f32_32x32x1f32(dw[bl * BN + 32 * TW * wn + 64 * p + lane], ms.x, zero, 0, 0, 0);
+                    o = __builtin_amdgcn_mfma_f32_32x32x1f32(dw[bl * BN + 64 * p + lane], ms.x, zero, 0, 0, 0);
                 }
 #pragma unroll
                 for (int jj = 0; jj < 2; ++jj) {
-                    const int j = 2 * p + jj, rl = 32 * (TW * wn + j) + c;
+                    const int j = 2 * p + jj, rl = 32 * j + c;
                     const uint4 a4 = w16[bl * BN + rl];
                     const uint2 a2 = w8[bl * BN + rl];
                     const f6_v8i A = {(int)a4.x, (int)a4.y, (int)a4.z, (int)a4.w, (int)a2.x, (int)a2.y, 0, 0};
@@ -222,7 +215,7 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2))) v
                         const int b = b0 + 2 * step + bl, m = m0 + tok;
 #pragma unroll
                         for (int r = 0; r < 16; ++r) {
-                            const int n = n0 + 32 * (TW * wn + j) + 8 * (r >> 2) + 4 * h + (r & 3);
+                            const int n = n0 + 32 * j + 8 * (r >> 2) + 4 * h + (r & 3);
                             if (b < b_end && m < M && n < N) sums[((size_t)m * N + n) * nb + b] = (int32_t)P[r];
                         }
                     } else {
@@ -233,22 +226,22 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2))) v
             }
         }
     };
-    load_d(sA16a[kg], sA8a[kg], sMta[kg], 0);
+    load_d(sA16a, sA8a, sMta, 0);
     load_w(sw0, 0);
     load_w(sw1, 1);
     load_w(sw2, 2);
     load_w(sw3, 3);
-    store(sw0, 0, sW16a[kg], sW8a[kg], sDwa[kg]);
+    store(sw0, 0, sW16a, sW8a, sDwa);
     F6_WAIT(6);  // the digits; the three later weight blocks (two loads each) may be out
     __syncthreads();
     // step u of four: digits of step + 1 to the other buffer, weights of step + 4 to the registers just free; then
     // step + 1's weights to LDS. At the wait the two weight loads of this step may be out, the digits before them not.
 #define F6_STEP(u, W, WN1, X, Y)                                                       \
-    load_d(sA16##Y[kg], sA8##Y[kg], sMt##Y[kg], s0 + u + 1);                           \
+    load_d(sA16##Y, sA8##Y, sMt##Y, s0 + u + 1);                           \
     load_w(W, s0 + u + 4);                                                             \
-    compute(s0 + u, sA16##X[kg], sA8##X[kg], sMt##X[kg], sW16##X[kg], sW8##X[kg], sDw##X[kg]); \
+    compute(s0 + u, sA16##X, sA8##X, sMt##X, sW16##X, sW8##X, sDw##X); \
     if (s0 + u + 1 >= nsteps) break;                                                   \
-    store(WN1, s0 + u + 1, sW16##Y[kg], sW8##Y[kg], sDw##Y[kg]);                       \
+    store(WN1, s0 + u + 1, sW16##Y, sW8##Y, sDw##Y);                       \
     F6_WAIT(2);                                                                        \
     __syncthreads();
     for (int s0 = 0;; s0 += 4) {
@@ -259,22 +252,6 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2))) v
     }
 #undef F6_STEP
     F6_WAIT(0);  // the last step's prefetch may still write LDS
-    if constexpr (KG == 2 && !SUMS) {  // the second group's sums join the first's, 4 BM x 4 floats at a time
-        float* red = reinterpret_cast<float*>(sA16a);
-        constexpr int PER = 2 * 4 * BM * 4 / 256;
-#pragma unroll
-        for (int i = 0; i < TW * 16 / PER; ++i) {
-            __syncthreads();
-            if (kg)
-#pragma unroll
-                for (int r = 0; r < PER; ++r) red[r * 256 + t] = acc[(i * PER + r) / 16][(i * PER + r) % 16];
-            __syncthreads();
-            if (!kg)
-#pragma unroll
-                for (int r = 0; r < PER; ++r) acc[(i * PER + r) / 16][(i * PER + r) % 16] += red[r * 256 + t];
-        }
-        if (kg) return;
-    }
     if constexpr (!SUMS) {
         const int m = m0 + 32 * wm + c;
         if (m >= M) return;
@@ -284,7 +261,7 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2))) v
         for (int j = 0; j < TW; ++j)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const int n = n0 + 32 * (TW * wn + j) + 8 * q + 4 * h;
+                const int n = n0 + 32 * j + 8 * q + 4 * h;
                 float4 v = make_float4(acc[j][4 * q], acc[j][4 * q + 1], acc[j][4 * q + 2], acc[j][4 * q + 3]);
                 if (vec && n + 3 < N) {
                     if constexpr (ADD) {
@@ -305,15 +282,13 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2))) v
 // ---------------------------------------------------------------------------------------------------------------
 // host
 // ---------------------------------------------------------------------------------------------------------------
-float* amv_splitk_workspace(size_t bytes, hipStream_t st);
+float* amv_splitk_workspace(size_t bytes, hipStream_t st, bool optional = false);
 int amv_splitk_count(int64_t tiles, int steps);
 void amv_splitk_reduce(const float* part, int S, int64_t zstride, int64_t m, int64_t n, float* dst, int64_t ldd,
                        hipStream_t st, const float* add = nullptr);
 
-template <int WM, int WN, int TW, int KG>
 static int f6_launch(const void* w, int64_t n_rows, int64_t k, uint8_t* act, int64_t m, float* dst, int64_t ldd,
                      int32_t* sums, hipStream_t st, const float* add) {
-    constexpr int BM = 32 * WM, BN = 32 * TW * WN;
     const int nb = (int)(k / 32);
     const int n_tw = (int)((n_rows + BN - 1) / BN), n_tt = (int)((m + BM - 1) / BM);
     const int64_t tiles = (int64_t)n_tw * n_tt;
@@ -342,7 +317,7 @@ static int f6_launch(const void* w, int64_t n_rows, int64_t k, uint8_t* act, int
     const int vec = ldo % 4 == 0 && ((uintptr_t)out & 15) == 0 && ((uintptr_t)kadd & 15) == 0;
     const dim3 grid((unsigned)(tiles * S));
 #define F6_GO(SU, AD)                                                                                              \
-    hipLaunchKernelGGL((k_qgemm_f6<WM, WN, TW, KG, SU, AD>), grid, dim3(256 * KG), 0, st, wq, wd, (int)n_rows, nb, d16, d8, meta, \
+    hipLaunchKernelGGL((k_qgemm_f6<SU, AD>), grid, dim3(256), 0, st, wq, wd, (int)n_rows, nb, d16, d8, meta, \
                        (int)L.mp, (int)m, out, ldo, kadd, sums, vec, per, zstride, n_tw, n_tt, S)
     if (sums) F6_GO(true, false);
     else if (kadd) F6_GO(false, true);
@@ -352,27 +327,26 @@ static int f6_launch(const void* w, int64_t n_rows, int64_t k, uint8_t* act, int
     return AMV_OK;
 }
 
+int amv_qgemm(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int64_t m, float* dst, int64_t ldd,
+              int32_t* sums, hipStream_t st, const float* add);
+
 // Q4_0 weights with an AMV_ACT_Q8_0_F6 activation of m rows: its plain Q8_0 prefix is packed into its scratch part, then
 // the product
 int amv_qgemm_f6(const void* w, int64_t n_rows, int64_t k, void* act, int64_t m, float* dst, int64_t ldd, int32_t* sums,
                  hipStream_t st, const float* add) {
     const int nb = (int)(k / 32);
+    const int64_t tiles = ((m + BM - 1) / BM) * ((n_rows + BN - 1) / BN);
+    // fewer than 1.5 workgroups per CU: the int8 kernel, whose smaller tiles share k between groups of waves (6144 x 4096 x
+    // 512 57 us against 73, 4096 x 4096 x 96 21 against 69). Measured here against it (us): 28672 x 4096 x 512 184 (195),
+    // 14336 x 4096 x 512 97 (98), 4096 x 14336 x 512 106 (114).
+    if (tiles * (sums ? 1 : amv_splitk_count(tiles, (nb + 1) / 2)) < 384)
+        return amv_qgemm(AMV_T_Q4_0, w, n_rows, k, act, m, dst, ldd, sums, st, add);
     uint8_t* a = (uint8_t*)act;
     const AmvQ80F6 L = amv_q8_0_f6_layout(m, k);
     hipLaunchKernelGGL(k_f6_pack, dim3((unsigned)((L.mp + 63) / 64), (unsigned)((nb + 3) / 4)), dim3(256), 0, st,
                        (const int8_t*)a, (const int2*)(a + m * k), (int)m, (int)L.mp, nb, (uint4*)(a + L.d16),
                        (uint2*)(a + L.d8), (float2*)(a + L.meta));
-    const auto wgs = [&](int bm, int bn) {  // workgroups with the split of k
-        const int64_t t = ((m + bm - 1) / bm) * ((n_rows + bn - 1) / bn);
-        return t * (sums ? 1 : amv_splitk_count(t, (nb + 1) / 2));
-    };
-    // 128 x 128 from 384 workgroups (1.5 per CU, as k_qgemm), else 64 x 128; where that leaves at most one workgroup per
-    // CU, two groups of 4 waves share its k. Measured (us, k = 4096 unless noted, against the int8 kernel): 28672 rows x
-    // 512 tokens 184 (229), 14336 x 512 97 (110), 14336 x 300 77 (108), 6144 x 512 60 (62), 4096 x 512 38 (51; one group
-    // 51), 14336 x 128 35 (53; one group 48), 4096 x 96 33 (42), k = 14336: 4096 x 512 106 (136), 4096 x 128 40 (48).
-    const int rc = wgs(128, 128) >= 384  ? f6_launch<4, 1, 4, 1>(w, n_rows, k, a, m, dst, ldd, sums, st, add)
-                   : wgs(64, 128) <= 256 ? f6_launch<2, 2, 2, 2>(w, n_rows, k, a, m, dst, ldd, sums, st, add)
-                                         : f6_launch<2, 2, 2, 1>(w, n_rows, k, a, m, dst, ldd, sums, st, add);
+    const int rc = f6_launch(w, n_rows, k, a, m, dst, ldd, sums, st, add);
     if (rc) return rc;
     return amv_check_launch("amv_mul_mat_q_act");
 }

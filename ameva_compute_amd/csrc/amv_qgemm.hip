@@ -8,22 +8,15 @@
 //                             I1 = sum_u sc_u sum_k q_k a_k, I2 = sum_u m_u sum_k a_k,
 //                             dst += d_a * (d * I1 - dmin * I2)
 // One v_mfma_i32_32x32x32_i8 is one 32-block (or one Q4_K unit) of a 32 x 32 tile, so S comes out of the matrix core
-// as an int32, exact. The per-block epilogue is VALU work beside the matrix core: Q4_0 / Q8_0 take three operations
-// per output and block (convert, scale by d_a, fma by d_w), Q4_K one integer multiply-add per unit (I1 += sc_u S_u)
-// and four per super-block (I2 is one f16 MFMA of the units' mins against the activation sums per 16, exact in f32).
+// as an int32, exact. The per-block epilogue is VALU work beside the matrix core and bounds these kernels: Q4_0 / Q8_0 take
+// two operations per output and block (convert, fma), Q4_K one integer multiply-add per unit (I1 += sc_u S_u) and four
+// per super-block (I2 is one f16 MFMA of the units' mins against the activation sums per 16, exact in f32).
 // The inputs are the plain activation layouts (int8 q with {f32 d, i32 sum} per 32, or Q8_K's f32 d per 256 and i32
 // sums per 16): no f16 copies are read.
 //
-// Tiling: workgroup of 4 waves (2 x 2) on BM = 64 TT tokens x BN = 64 TW weight rows; wave (wt, ww) owns tokens
-// 32 TT wt .. and rows 32 TW ww .. as TT x TW tiles of 32 x 32. MFMA operands: A = tokens, B = weight rows; lane l
-// supplies token (row of A) / weight row (column of B) l % 32 and the 16 bytes 16 (l / 32) .. + 15 of the 32-block
-// (any assignment of k to byte slots works as long as A and B share it); the result D of lane l holds weight row
-// l % 32 and tokens 8 (r / 4) + 4 (l / 32) + r % 4, r = 0..15, so the weight scale of an output is one value per lane
-// and the token scales are four float4 reads.
-// Pipeline steps of 64 k (two 32-blocks, or one 32-byte Q4_K chunk = units 2c, 2c + 1): the global loads of step
-// s + 1 are issued before step s computes from LDS; at staging the weights are expanded to int8 once per workgroup
-// (Q4_0: n - 8 per byte with integer tricks, Q4_K: the unsigned nibbles) and the activations copied. LDS rows are
-// 80 bytes (64 + 16 of padding): the 16-byte fragment reads of 32 consecutive rows hit distinct banks.
+// MFMA operands: A = tokens, B = weight rows; lane l supplies token (row of A) / weight row (column of B) l % 32 and the 16
+// bytes 16 (l / 32) .. + 15 of the 32-block (any assignment of k to byte slots works as long as A and B share it); the
+// result D of lane l holds weight row l % 32 and tokens 8 (r / 4) + 4 (l / 32) + r % 4, r = 0..15.
 // The grid is one dimension, mapped so that the workgroups sharing a weight tile (its token tiles) are dispatched to
 // the same XCD, one after another, and with a split of k each k range goes to its own group of XCDs (range z to
 // XCDs 8 z / n_z ..): MI355X hands workgroup i to XCD i % 8, and each XCD has its own L2, so an XCD reads the weight
@@ -46,421 +39,406 @@ __device__ __forceinline__ uint32_t qg_m8(uint32_t v) { return (v + 0x78787878u)
 
 
 // ---------------------------------------------------------------------------------------------------------------
-// Q4_0 / Q8_0
+// Q4_0 / Q8_0 x Q8_0. Bytes go from memory to LDS without registers (buffer_load .. lds), one step of four blocks (128 k)
+// ahead; Q4_0 weights stay packed there and a lane unpacks its operand bytes (n - 8 per byte) for both its token tiles.
+// Per wave 64 tokens x 32 rows: WM x WN waves on BM = 64 WM tokens x BN = 32 WN rows, KG such groups in a workgroup on
+// consecutive parts of k, their sums added at the end: where the tiles alone leave at most one workgroup per CU, a group by
+// itself waits for its loads most of the time. The registers stay within 128, so four waves share a SIMD.
+// Epilogue of a block: the scale products d_a d_w of both token tiles are one outer product on the matrix core
+// (v_mfma_f32_32x32x1_2b_f32: each one f32 product), which leaves the conversion and the fma.
+// LDS rows are unpadded (the loads write them as they come): the 16-byte pieces of a row are exchanged by an XOR with the
+// row index on the memory side, so that the fragment reads of 16 consecutive rows hit all banks once.
 // ---------------------------------------------------------------------------------------------------------------
-template <int WT>
-struct QgRegs {  // one thread's share of a step: weight block (row t / 2, block t % 2), activation block (token t / 2)
-    uint4 w0, w1;  // Q4_0: w0 = the 16 nibble bytes; Q8_0: the 32 bytes
-    uint4 a0, a1;  // 32 int8 of the token's block
-    uint32_t dw;   // the weight block's f16 scale bits
-    float da;
-    bool past;     // a block past the split's end: weight scale 0
-};
+typedef __attribute__((address_space(3))) void qg_lds;
+#define QG_RSRC(p, bytes) __builtin_amdgcn_make_buffer_rsrc((void*)(p), 0, (uint32_t)(bytes), 0x00027000)
+// wait for every vector memory load (the other counters are left alone)
+#define QG_WAIT_LOADS() __builtin_amdgcn_s_waitcnt(0x0f70)
 
-template <int WT, int TT, int TW>
-__device__ __forceinline__ QgRegs<WT> qg_load(int step, const uint8_t* __restrict__ wq,
-                                        const uint16_t* __restrict__ wd, int N, int nb, int n0,
-                                        const int8_t* __restrict__ aq, const int2* __restrict__ am, int M, int m0,
-                                        int K, int b0, int b_end) {
-    constexpr int BN = 64 * TW, BM = 64 * TT;
-    const int t = threadIdx.x, blk = t & 1;
-    const int b = b0 + 2 * step + blk, bc = min(b, b_end - 1);  // a block past the split's end: weight scale 0
-    // the loaded values stay untouched until qg_store (any arithmetic on them here makes the compiler wait for the
-    // whole prefetch at the load); the fields of a role the thread does not have are not read
-    QgRegs<WT> s;
-    s.past = b >= b_end;
-    if (2 * BN >= 256 || t < 2 * BN) {  // (every thread of the 256 when BN = 128)
-        const int row = min(n0 + (t >> 1), N - 1);
-        const size_t bi = (size_t)row * nb + bc;
-        if constexpr (WT == AMV_T_Q4_0) {
-            s.w0 = *reinterpret_cast<const uint4*>(wq + bi * 16);
-            s.dw = wd[amv_q4_0_didx(row, bc, nb, N)];
-        } else {
-            const uint4* p = reinterpret_cast<const uint4*>(wq + bi * 32);
-            s.w0 = p[0];
-            s.w1 = p[1];
-            s.dw = wd[bi];
+// The end of a product: the KG groups' sums joined in the first group, in order of k, through the first A buffers (gA: KG
+// x BM * 8 pieces, free), 8 registers of a thread at a time, then stored. A lane holds weight row n and tokens
+// m + 32 i + 8 (r / 4) + r % 4: for each r the 32 lanes of a half store 32 consecutive floats of one token row.
+template <bool SUMS, int BM, int NT, int KG, bool ADD>
+__device__ __forceinline__ void qg_finish(qg_f16v (&acc)[2], uint4 (*gA)[BM * 8], int kg, int t, int n, int m, int M, int N,
+                                          float* __restrict__ dst, int64_t ldd, const float* add) {
+    if constexpr (SUMS) return;
+    if constexpr (KG > 1) {
+        constexpr int PER = BM * 8 * 4 / NT;
+        float* const red = reinterpret_cast<float*>(gA[kg]);
+#pragma unroll
+        for (int q = 0; q < 32 / PER; ++q) {
+            __syncthreads();
+            if (kg)
+#pragma unroll
+                for (int r = 0; r < PER; ++r) red[r * NT + t] = acc[(q * PER + r) / 16][(q * PER + r) % 16];
+            __syncthreads();
+            if (!kg)
+#pragma unroll
+                for (int g = 1; g < KG; ++g)
+#pragma unroll
+                    for (int r = 0; r < PER; ++r)
+                        acc[(q * PER + r) / 16][(q * PER + r) % 16] += reinterpret_cast<const float*>(gA[g])[r * NT + t];
         }
+        if (kg) return;
     }
-    if (2 * BM >= 256 || t < 2 * BM) {
-        const int tok = min(m0 + (t >> 1), M - 1);
-        const uint4* p = reinterpret_cast<const uint4*>(aq + (size_t)tok * K + 32 * bc);
-        s.a0 = p[0];
-        s.a1 = p[1];
-        s.da = __int_as_float(am[(size_t)tok * nb + bc].x);
-    }
-    return s;
+    if (n >= N) return;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int mm = m + 32 * i + 8 * (r >> 2) + (r & 3);
+            if (mm < M) {
+                const size_t o = (size_t)mm * ldd + n;
+                if constexpr (ADD) dst[o] = acc[i][r] + add[o];
+                else dst[o] = acc[i][r];
+            }
+        }
 }
 
-template <int WT, int TT, int TW>
-__device__ __forceinline__ void qg_store(const QgRegs<WT>& s, int8_t* __restrict__ sW, int8_t* __restrict__ sA,
-                                         float* __restrict__ sDw, float* __restrict__ sDa) {
-    constexpr int BN = 64 * TW, BM = 64 * TT;
-    const int t = threadIdx.x, blk = t & 1;
-    if (t < 2 * BN) {
-        uint4* d = reinterpret_cast<uint4*>(sW + (t >> 1) * QG_LD + 32 * blk);
-        if constexpr (WT == AMV_T_Q4_0) {  // element e < 16: low nibble of byte e; 16 + e: its high nibble
-            const uint4 x = s.w0;
-            d[0] = make_uint4(qg_m8(x.x & 0x0F0F0F0Fu), qg_m8(x.y & 0x0F0F0F0Fu), qg_m8(x.z & 0x0F0F0F0Fu),
-                              qg_m8(x.w & 0x0F0F0F0Fu));
-            d[1] = make_uint4(qg_m8((x.x >> 4) & 0x0F0F0F0Fu), qg_m8((x.y >> 4) & 0x0F0F0F0Fu),
-                              qg_m8((x.z >> 4) & 0x0F0F0F0Fu), qg_m8((x.w >> 4) & 0x0F0F0F0Fu));
-        } else {
-            d[0] = s.w0;
-            d[1] = s.w1;
-        }
-        sDw[blk * BN + (t >> 1)] = s.past ? 0.0f : amv_h2f((uint16_t)s.dw);
-    }
-    if (t < 2 * BM) {
-        uint4* d = reinterpret_cast<uint4*>(sA + (t >> 1) * QG_LD + 32 * blk);
-        d[0] = s.a0;
-        d[1] = s.a1;
-        sDa[blk * BM + (t >> 1)] = s.da;
-    }
-}
-
-template <int WT, bool SUMS, int TT, int TW, bool ADD = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_qgemm(const uint8_t* __restrict__ wq, const uint16_t* __restrict__ wd,
-                                              int N, int nb, const int8_t* __restrict__ aq,
-                                              const int2* __restrict__ am, int M, float* __restrict__ dst,
-                                              int64_t ldd, const float* add, int32_t* __restrict__ sums, int kb_per,
-                                              int64_t zstride, int n_tw, int n_tt, int n_z) {
-    constexpr int BN = 64 * TW, BM = 64 * TT;
-    __shared__ __align__(16) int8_t sW[2][BN * QG_LD];
-    __shared__ __align__(16) int8_t sA[2][BM * QG_LD];
-    __shared__ __align__(16) float sDw[2][2 * BN];
-    __shared__ __align__(16) float sDa[2][2 * BM];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int wt = w & 1, ww = w >> 1, c = lane & 31, h = lane >> 5;
+template <int WT, bool SUMS, int WM, int WN, int KG, bool ADD = false>
+__global__ __launch_bounds__(64 * WM * WN * KG) __attribute__((amdgpu_waves_per_eu(4))) void k_qgemm(
+    const uint8_t* __restrict__ wq, const uint16_t* __restrict__ wd, int N, int nb, const int8_t* __restrict__ aq,
+    const int2* __restrict__ am, int M, float* __restrict__ dst, int64_t ldd, const float* add,
+    int32_t* __restrict__ sums, int kb_per, int64_t zstride, int n_tw, int n_tt, int n_z) {
+    constexpr int BN = 32 * WN, BM = 64 * WM, NT = 64 * WM * WN;
+    constexpr bool Q4 = WT == AMV_T_Q4_0;
+    constexpr int WB = Q4 ? 16 : 32, WP = 4 * WB / 16;            // bytes of a weight block, 16-byte pieces of a step's row
+    constexpr int RA = BM * 8 / NT, RW = BN * WP / NT;            // rounds of the threads over a step's pieces
+    constexpr int RDA = BM * 4 / NT, RDW = BN * 4 / NT;           // and over its scales
+    // the buffers of even and odd steps are variables of their own: reads of one do not wait for the loads into the other
+    __shared__ __align__(16) uint4 gAa[KG][BM * 8], gAb[KG][BM * 8], gWa[KG][BN * WP], gWb[KG][BN * WP];
+    __shared__ __align__(16) float gDa[KG][2][4 * BM], gDw[KG][2][4 * BN];
+    const int t = threadIdx.x & (NT - 1), lane = t & 63, c32 = lane & 31, h = lane >> 5;
+    const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT);
+    uint4 *const sAa = gAa[kg], *const sAb = gAb[kg], *const sWa = gWa[kg], *const sWb = gWb[kg];
+    const int wv = __builtin_amdgcn_readfirstlane(t >> 6), wm = wv / WN, wn = wv % WN;
     // tile index: token tile fastest, then the split of k, then the weight tile
-    const int T = amv_xcd_tile(blockIdx.x, n_tw * n_z * n_tt);  // token tiles, weight tiles, k ranges
+    const int T = amv_xcd_tile(blockIdx.x, n_tw * n_z * n_tt);
     const int tt = T % n_tt, tw = (T / n_tt) % n_tw, z = T / (n_tt * n_tw);
     const int n0 = tw * BN, m0 = tt * BM;
     const int K = nb * 32;
-    const int b0 = z * kb_per, b_end = min(nb, b0 + kb_per);
-    const int nsteps = (b_end - b0 + 1) / 2;
+    // the split's blocks, dealt to the KG groups of waves in runs of steps
+    const int z0 = z * kb_per, z_end = min(nb, z0 + kb_per), nsteps = ((z_end - z0 + 3) / 4 + KG - 1) / KG;
+    const int b0 = z0 + 4 * nsteps * kg, b_end = min(z_end, b0 + 4 * nsteps);
     dst += (size_t)z * zstride;
 
-    qg_f16v acc[TT][TW];
+    const int mr = min(BM, M - m0), nr = min(BN, N - n0);  // rows past N and tokens past M read as zero
+    const __amdgpu_buffer_rsrc_t ra = QG_RSRC(aq + (size_t)m0 * K, mr * K);
+    const __amdgpu_buffer_rsrc_t rw = QG_RSRC(wq + (size_t)n0 * nb * WB, (uint32_t)(nr * nb) * WB);
+    const __amdgpu_buffer_rsrc_t rm = QG_RSRC(am + (size_t)m0 * nb, (uint32_t)(mr * nb) * 8u);
+    const uint32_t oa = (uint32_t)(t >> 3) * K + 16 * ((t & 7) ^ ((t >> 4) & 7));
+    const uint32_t ow = Q4 ? (uint32_t)(t >> 2) * (nb * 16) + 16 * ((t & 3) ^ ((t >> 4) & 3))
+                           : (uint32_t)(t >> 3) * (nb * 32) + 16 * ((t & 7) ^ ((t >> 4) & 7));
+    const auto load = [&](uint4* sA, uint4* sW, int b) {
 #pragma unroll
-    for (int i = 0; i < TT; ++i)
+        for (int i = 0; i < RA; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (qg_lds*)(sA + NT * i + 64 * wv), 16,
+                                                     oa + (uint32_t)(NT / 8 * i) * K, 32 * b, 0, 0);
 #pragma unroll
-        for (int j = 0; j < TW; ++j)
+        for (int i = 0; i < RW; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (qg_lds*)(sW + NT * i + 64 * wv), 16,
+                                                     ow + (uint32_t)(NT / WP * i) * (nb * WB), WB * b, 0, 0);
+    };
+    // scales, through registers: token x / 4 (row x / 4) of the block x % 4 of the step; 0 past the group's blocks
+    float da[RDA];
+    uint32_t dw[RDW];
+    const auto load_s = [&](int b) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-    // global loads run two steps ahead of the compute: the registers of step s + 2 are loaded while step s computes
-    // and step s + 1's (loaded during step s - 1) go to LDS at its end
-    QgRegs<WT> st0, st1;
-    st0 = qg_load<WT, TT, TW>(0, wq, wd, N, nb, n0, aq, am, M, m0, K, b0, b_end);
-    qg_store<WT, TT, TW>(st0, sW[0], sA[0], sDw[0], sDa[0]);
-    st1 = qg_load<WT, TT, TW>(min(1, nsteps - 1), wq, wd, N, nb, n0, aq, am, M, m0, K, b0, b_end);
-    __syncthreads();
-    const auto compute = [&](int step) {
-        const int buf = step & 1;
-#pragma unroll 1
-        for (int bl = 0; bl < 2; ++bl) {  // one block's MFMA results live at a time
-            qg_v4i A[TT], B[TW];
+        for (int i = 0; i < RDA; ++i) {
+            const int x = t + NT * i, bb = b + (x & 3);
+            da[i] = __int_as_float(
+                __builtin_amdgcn_raw_buffer_load_b32(rm, ((uint32_t)(x >> 2) * nb + (bb < b_end ? bb : 0)) * 8u, 0, 0));
+        }
 #pragma unroll
-            for (int i = 0; i < TT; ++i)
-                A[i] = *reinterpret_cast<const qg_v4i*>(sA[buf] + (32 * (TT * wt + i) + c) * QG_LD + 32 * bl + 16 * h);
-#pragma unroll
-            for (int j = 0; j < TW; ++j)
-                B[j] = *reinterpret_cast<const qg_v4i*>(sW[buf] + (32 * (TW * ww + j) + c) * QG_LD + 32 * bl + 16 * h);
-            const int b = b0 + 2 * step + bl;
-#pragma unroll
-            for (int i = 0; i < TT; ++i) {
-                const int tl = 32 * (TT * wt + i) + 4 * h;  // first token of the lane in this token tile
-                float da[16];
-                if constexpr (!SUMS) {
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const float4 v = *reinterpret_cast<const float4*>(&sDa[buf][bl * BM + tl + 8 * q]);
-                        da[4 * q] = v.x;
-                        da[4 * q + 1] = v.y;
-                        da[4 * q + 2] = v.z;
-                        da[4 * q + 3] = v.w;
-                    }
-                }
-#pragma unroll
-                for (int j = 0; j < TW; ++j) {
-                    const qg_v16i zero = {};
-                    const qg_v16i C = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[i], B[j], zero, 0, 0, 0);
-                    const int rl = 32 * (TW * ww + j) + c;  // the lane's weight row in the tile
-                    if constexpr (SUMS) {
-                        const int n = n0 + rl;
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            const int m = m0 + tl + 8 * (r >> 2) + (r & 3);
-                            if (b < b_end && m < M && n < N) sums[((size_t)m * N + n) * nb + b] = C[r];
-                        }
-                    } else {
-                        const float dw = sDw[buf][bl * BN + rl];
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) acc[i][j][r] = fmaf((float)C[r], dw * da[r], acc[i][j][r]);
-                    }
-                }
-            }
+        for (int i = 0; i < RDW; ++i) {
+            const int x = t + NT * i, bb = min(b + (x & 3), z_end - 1), row = min(n0 + (x >> 2), N - 1);
+            dw[i] = wd[Q4 ? amv_q4_0_didx(row, bb, nb, N) : (size_t)row * nb + bb];
         }
     };
-    // the prefetches are unconditional (past the last step they read the last step again) so that the wait before
-    // each store covers only the registers it stores, not the prefetch issued after them
-    for (int step = 0; step < nsteps; step += 2) {
-        st0 = qg_load<WT, TT, TW>(min(step + 2, nsteps - 1), wq, wd, N, nb, n0, aq, am, M, m0, K, b0, b_end);
-        compute(step);
-        if (step + 1 >= nsteps) break;
-        qg_store<WT, TT, TW>(st1, sW[1], sA[1], sDw[1], sDa[1]);
-        __syncthreads();
-        st1 = qg_load<WT, TT, TW>(min(step + 3, nsteps - 1), wq, wd, N, nb, n0, aq, am, M, m0, K, b0, b_end);
-        compute(step + 1);
-        if (step + 2 >= nsteps) break;
-        qg_store<WT, TT, TW>(st0, sW[0], sA[0], sDw[0], sDa[0]);
-        __syncthreads();
-    }
-    if constexpr (!SUMS) {
-        // lane: weight row n, tokens 8 (r / 4) + 4 h + r % 4: for each r the 32 lanes of a half store 32 consecutive
-        // floats of one token row
+    const auto store_s = [&](int b, int buf) {
 #pragma unroll
-        for (int j = 0; j < TW; ++j) {
-            const int n = n0 + 32 * (TW * ww + j) + c;
-            if (n >= N) continue;
+        for (int i = 0; i < RDA; ++i) {
+            const int x = t + NT * i;
+            gDa[kg][buf][(x & 3) * BM + (x >> 2)] = b + (x & 3) < b_end ? da[i] : 0.0f;
+        }
 #pragma unroll
-            for (int i = 0; i < TT; ++i)
+        for (int i = 0; i < RDW; ++i) {
+            const int x = t + NT * i;
+            gDw[kg][buf][(x & 3) * BN + (x >> 2)] = b + (x & 3) < b_end ? amv_h2f((uint16_t)dw[i]) : 0.0f;
+        }
+    };
+
+    qg_f16v acc[2];
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int m = m0 + 32 * (TT * wt + i) + 8 * (r >> 2) + 4 * h + (r & 3);
-                    if (m < M) {
-                        const size_t o = (size_t)m * ldd + n;
-                        if constexpr (ADD) dst[o] = acc[i][j][r] + add[o];
-                        else dst[o] = acc[i][j][r];
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
+    const int ar = 64 * wm + c32, wr = 32 * wn + c32;
+    const int ax = (c32 >> 1) & 7, wx = Q4 ? (c32 >> 2) & 3 : ax;  // the rows' XOR (64 wm, 32 i, 32 wn do not change them)
+    const auto compute = [&](const uint4* sA, const uint4* sW, int b, int buf) {
+#pragma unroll
+        for (int bl = 0; bl < 4; ++bl) {
+            typedef float f32v __attribute__((ext_vector_type(32)));
+            f32v o;
+            if constexpr (!SUMS) {
+                const f32v zero = {};
+                o = __builtin_amdgcn_mfma_f32_32x32x1f32(gDa[kg][buf][bl * BM + 64 * wm + lane], gDw[kg][buf][bl * BN + wr],
+                                                         zero, 0, 0, 0);
+            }
+            qg_v4i B;
+            if constexpr (Q4) {  // element e < 16: low nibble of byte e (lane half 0); 16 + e: its high nibble (half 1)
+                const uint4 x = sW[wr * 4 + (bl ^ wx)];
+                const int s = 4 * h;
+                B = qg_v4i{(int)qg_m8((x.x >> s) & 0x0F0F0F0Fu), (int)qg_m8((x.y >> s) & 0x0F0F0F0Fu),
+                           (int)qg_m8((x.z >> s) & 0x0F0F0F0Fu), (int)qg_m8((x.w >> s) & 0x0F0F0F0Fu)};
+            } else {
+                const uint4 x = sW[wr * 8 + ((2 * bl + h) ^ wx)];
+                B = qg_v4i{(int)x.x, (int)x.y, (int)x.z, (int)x.w};
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const uint4 a = sA[(ar + 32 * i) * 8 + ((2 * bl + h) ^ ax)];
+                const qg_v16i zero = {};
+                const qg_v16i C = __builtin_amdgcn_mfma_i32_32x32x32_i8(
+                    qg_v4i{(int)a.x, (int)a.y, (int)a.z, (int)a.w}, B, zero, 0, 0, 0);
+                if constexpr (SUMS) {
+                    const int n = n0 + wr;
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int m = m0 + 64 * wm + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
+                        if (b + bl < b_end && m < M && n < N) sums[((size_t)m * N + n) * nb + b + bl] = C[r];
                     }
-                }
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------------------------------------------
-// Q4_K x Q8_K. Step = chunk c (0..3) of super-block j: the 32 qs bytes whose low nibbles are unit 2c and high nibbles
-// unit 2c + 1. Per super-block values (unit scales and mins, d, dmin, the activation sums per 16 and d_a) are staged
-// at its chunk 0 into a slot of their own, double-buffered by super-block parity.
-// ---------------------------------------------------------------------------------------------------------------
-struct QgKRegs {
-    uint4 q;       // weight bytes 16 hf .. + 15 of the chunk (row t / 2, hf = t % 2)
-    uint4 hd;      // the row's 16-byte head (d, dmin, 12 scale bytes), at chunk 0
-    uint4 a0, a1;  // 32 activation int8 (token t / 2, k 64 c + 32 hf ..)
-    int s[8];      // at chunk 0: the token's sums per 16, 8 hf .. 8 hf + 7
-    float da;      // at chunk 0: the token's super-block scale
-};
-
-template <int TT, int TW>
-__device__ __forceinline__ void qgk_load(QgKRegs& s, int step, const uint4* __restrict__ wq,
-                                         const uint4* __restrict__ wh, int N, int nsb, int n0,
-                                         const int8_t* __restrict__ aq, const float* __restrict__ ad,
-                                         const int32_t* __restrict__ as16, int M, int m0, int K, int sb0) {
-    constexpr int BN = 64 * TW, BM = 64 * TT;
-    const int t = threadIdx.x, hf = t & 1;
-    const int j = sb0 + (step >> 2), c = step & 3;
-    if (t < 2 * BN) {
-        const int row = min(n0 + (t >> 1), N - 1);
-        const size_t sb = (size_t)row * nsb + j;
-        s.q = wq[sb * 8 + 2 * c + hf];
-        if (c == 0) s.hd = wh[sb];
-    }
-    if (t < 2 * BM) {
-        const int tok = min(m0 + (t >> 1), M - 1);
-        const uint4* p = reinterpret_cast<const uint4*>(aq + (size_t)tok * K + 256 * j + 64 * c + 32 * hf);
-        s.a0 = p[0];
-        s.a1 = p[1];
-        if (c == 0) {
-            const int32_t* q = as16 + (size_t)tok * (K / 16) + 16 * j + 8 * hf;  // 4-byte aligned only
+                } else {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) s.s[e] = q[e];
-            s.da = ad[(size_t)tok * nsb + j];
+                    for (int r = 0; r < 16; ++r) acc[i][r] = fmaf((float)C[r], o[16 * i + r], acc[i][r]);
+                }
+            }
+            // one block's results at a time (more do not fit the registers), added up here (the compiler would move the
+            // additions behind the next barrier and keep the results until then)
+            asm volatile("" : "+v"(acc[0]), "+v"(acc[1]));
+            __builtin_amdgcn_sched_barrier(0);
         }
+    };
+
+    load(sAa, sWa, b0);
+    load_s(b0);
+    store_s(b0, 0);
+    QG_WAIT_LOADS();
+    __syncthreads();
+    for (int s = 0;; s += 2) {
+        load(sAb, sWb, b0 + 4 * (s + 1));
+        load_s(b0 + 4 * (s + 1));
+        if (b0 + 4 * s < b_end) compute(sAa, sWa, b0 + 4 * s, 0);
+        if (s + 1 >= nsteps) break;
+        store_s(b0 + 4 * (s + 1), 1);
+        QG_WAIT_LOADS();
+        __syncthreads();
+        load(sAa, sWa, b0 + 4 * (s + 2));
+        load_s(b0 + 4 * (s + 2));
+        if (b0 + 4 * (s + 1) < b_end) compute(sAb, sWb, b0 + 4 * (s + 1), 1);
+        if (s + 2 >= nsteps) break;
+        store_s(b0 + 4 * (s + 2), 0);
+        QG_WAIT_LOADS();
+        __syncthreads();
     }
+    QG_WAIT_LOADS();  // the last step's prefetch may still write LDS
+    qg_finish<SUMS, BM, NT, KG, ADD>(acc, gAa, kg, t, n0 + wr, m0 + 64 * wm + 4 * h, M, N, dst, ldd, add);
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// Q4_K x Q8_K. All operands go from memory to LDS without registers (buffer_load .. lds), one step ahead, and the
+// weights stay packed there: the 16 bytes a lane reads of a 32-byte chunk are its operand bytes of two units (low and
+// high nibbles), unpacked in 12 operations for both token tiles. Waves, groups and LDS rows as k_qgemm above: with the loads staged
+// through registers and two waves of 64 x 64 on a SIMD, half the cycles went by with no instruction issued.
+// Step = half a super-block (128 k).
+// Per super-block: the 16-byte heads go to LDS with the first half; every lane decodes its row's 8 scales and mins from
+// the head (bytes, 8 operations). The activation sums per 16 (f16) and d_a are staged through registers.
+// ---------------------------------------------------------------------------------------------------------------
 __device__ __forceinline__ uint32_t qg_h2(int a, int b) {
     return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(float)a) |
            ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(float)b) << 16);
 }
 
-template <int TT, int TW>
-__device__ __forceinline__ void qgk_store(const QgKRegs& s, int step, int8_t* __restrict__ sW,
-                                          int8_t* __restrict__ sA, uint8_t* __restrict__ sSc,
-                                          float* __restrict__ sD, float* __restrict__ sDm, uint16_t* __restrict__ sMn,
-                                          uint16_t* __restrict__ sBs, float* __restrict__ sDa) {
-    constexpr int BN = 64 * TW, BM = 64 * TT;
-    const int t = threadIdx.x, hf = t & 1, c = step & 3;
-    if (t < 2 * BN) {
-        const int rl = t >> 1;
-        uint4* d = reinterpret_cast<uint4*>(sW + rl * QG_LD);
-        const uint4 x = s.q;  // unit 2c: low nibbles (elements 16 hf ..), unit 2c + 1: high nibbles
-        d[hf] = make_uint4(x.x & 0x0F0F0F0Fu, x.y & 0x0F0F0F0Fu, x.z & 0x0F0F0F0Fu, x.w & 0x0F0F0F0Fu);
-        d[2 + hf] = make_uint4((x.x >> 4) & 0x0F0F0F0Fu, (x.y >> 4) & 0x0F0F0F0Fu, (x.z >> 4) & 0x0F0F0F0Fu,
-                               (x.w >> 4) & 0x0F0F0F0Fu);
-        if (c == 0) {  // units 4 hf .. 4 hf + 3: scales (bytes) and mins (f16, on the two 16-sum slots of each unit)
-            uint32_t mm[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                int sc, mn;
-                k4_scale_min(4 * hf + e, s.hd.y, s.hd.z, s.hd.w, sc, mn);
-                sSc[(4 * hf + e) * BN + rl] = (uint8_t)sc;
-                mm[e] = qg_h2(mn, mn);
-            }
-            *reinterpret_cast<uint4*>(sMn + rl * 16 + 8 * hf) = make_uint4(mm[0], mm[1], mm[2], mm[3]);
-            if (hf == 0) {
-                sD[rl] = amv_h2f(s.hd.x);
-                sDm[rl] = amv_h2f(s.hd.x >> 16);
-            }
-        }
-    }
-    if (t < 2 * BM) {
-        const int tl = t >> 1;
-        uint4* d = reinterpret_cast<uint4*>(sA + tl * QG_LD + 32 * hf);
-        d[0] = s.a0;
-        d[1] = s.a1;
-        if (c == 0) {  // the 16-sums as f16 (|sum| <= 2032: exact)
-            *reinterpret_cast<uint4*>(sBs + tl * 16 + 8 * hf) =
-                make_uint4(qg_h2(s.s[0], s.s[1]), qg_h2(s.s[2], s.s[3]), qg_h2(s.s[4], s.s[5]), qg_h2(s.s[6], s.s[7]));
-            if (hf == 0) sDa[tl] = s.da;
-        }
-    }
-}
-
-template <bool SUMS, int TT, int TW, bool ADD = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_qgemm_q4k(const uint4* __restrict__ wq, const uint4* __restrict__ wh, int N,
-                                                  int nsb, const int8_t* __restrict__ aq, const float* __restrict__ ad,
-                                                  const int32_t* __restrict__ as16, int M, float* __restrict__ dst,
-                                                  int64_t ldd, const float* add, int32_t* __restrict__ sums, int sb_per,
-                                                  int64_t zstride, int n_tw, int n_tt, int n_z) {
-    constexpr int BN = 64 * TW, BM = 64 * TT;
-    __shared__ __align__(16) int8_t sW[2][BN * QG_LD];
-    __shared__ __align__(16) int8_t sA[2][BM * QG_LD];
-    __shared__ __align__(16) uint8_t sSc[2][8 * BN];
-    __shared__ __align__(16) float sD[2][BN], sDm[2][BN], sDa[2][BM];
-    __shared__ __align__(16) uint16_t sMn[2][BN * 16], sBs[2][BM * 16];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int wt = w & 1, ww = w >> 1, c32 = lane & 31, h = lane >> 5;
+template <bool SUMS, int WM, int WN, int KG, bool ADD = false>
+__global__ __launch_bounds__(64 * WM * WN * KG) __attribute__((amdgpu_waves_per_eu(4))) void k_qgemm_q4k(
+    const uint4* __restrict__ wq, const uint4* __restrict__ wh, int N, int nsb, const int8_t* __restrict__ aq,
+    const float* __restrict__ ad, const int32_t* __restrict__ as16, int M, float* __restrict__ dst, int64_t ldd,
+    const float* add, int32_t* __restrict__ sums, int sb_per, int64_t zstride, int n_tw, int n_tt, int n_z) {
+    constexpr int BN = 32 * WN, BM = 64 * WM, NT = 64 * WM * WN;
+    constexpr int RA = BM * 8 / NT, RW = BN * 4 / NT, RS = BM * 4 / NT;  // rounds of the threads over a step's pieces
+    // the buffers of the two halves are variables of their own: reads of one do not wait for the loads into the other
+    __shared__ __align__(16) uint4 gAa[KG][BM * 8], gAb[KG][BM * 8], gWa[KG][BN * 4], gWb[KG][BN * 4], gHd[KG][BN];
+    __shared__ __align__(16) uint2 gBs[KG][BM * 4];
+    __shared__ __align__(16) float gDa[KG][BM];
+    const int t = threadIdx.x & (NT - 1), lane = t & 63, c32 = lane & 31, h = lane >> 5;
+    const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT);
+    uint4 *const sAa = gAa[kg], *const sAb = gAb[kg], *const sWa = gWa[kg], *const sWb = gWb[kg], *const sHd = gHd[kg];
+    uint2* const sBs = gBs[kg];
+    float* const sDa = gDa[kg];
+    const int wv = __builtin_amdgcn_readfirstlane(t >> 6), wm = wv / WN, wn = wv % WN;
     const int T = amv_xcd_tile(blockIdx.x, n_tw * n_z * n_tt);  // token tiles, weight tiles, k ranges
     const int tt = T % n_tt, tw = (T / n_tt) % n_tw, z = T / (n_tt * n_tw);
     const int n0 = tw * BN, m0 = tt * BM;
     const int K = nsb * 256;
-    const int sb0 = z * sb_per, sb_end = min(nsb, sb0 + sb_per);
-    const int nsteps = (sb_end - sb0) * 4;
+    // the split's super-blocks, dealt to the KG groups of waves in runs of `run`; a group's turns past the end (or past the
+    // split's) compute on the last super-block and add nothing
+    const int z0 = z * sb_per, z_end = min(nsb, z0 + sb_per), run = (z_end - z0 + KG - 1) / KG;
+    const int sb0 = z0 + run * kg, sb_end = min(z_end, sb0 + run), sb_last = z_end - 1;
     dst += (size_t)z * zstride;
 
-    qg_f16v acc[TT][TW];
-    qg_v16i I1[TT][TW];
+    // rows past N and tokens past M read as zero
+    const int mr = min(BM, M - m0), nr = min(BN, N - n0);
+    const __amdgpu_buffer_rsrc_t ra = QG_RSRC(aq + (size_t)m0 * K, mr * K);
+    const __amdgpu_buffer_rsrc_t rw = QG_RSRC(wq + (size_t)n0 * nsb * 8, nr * nsb * 128);
+    const __amdgpu_buffer_rsrc_t rh = QG_RSRC(wh + (size_t)n0 * nsb, nr * nsb * 16);
+    const __amdgpu_buffer_rsrc_t rs = QG_RSRC(as16 + (size_t)m0 * (K / 16), mr * (K / 4));
+    const __amdgpu_buffer_rsrc_t rd = QG_RSRC(ad + (size_t)m0 * nsb, mr * nsb * 4);
+    const uint32_t oa = (uint32_t)(t >> 3) * K + 16 * ((t & 7) ^ ((t >> 4) & 7));
+    const uint32_t ow = (uint32_t)(t >> 2) * (nsb * 128) + 16 * ((t & 3) ^ ((t >> 4) & 3));
+    const auto load = [&](uint4* sA, uint4* sW, int j, int half) {
 #pragma unroll
-    for (int i = 0; i < TT; ++i)
+        for (int i = 0; i < RA; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (qg_lds*)(sA + NT * i + 64 * wv), 16,
+                                                     oa + (uint32_t)(NT / 8 * i) * K, 256 * j + 128 * half, 0, 0);
 #pragma unroll
-        for (int j = 0; j < TW; ++j)
+        for (int i = 0; i < RW; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (qg_lds*)(sW + NT * i + 64 * wv), 16,
+                                                     ow + (uint32_t)(NT / 4 * i) * (nsb * 128), 128 * j + 64 * half, 0, 0);
+    };
+    const auto load_head = [&](int j) {
+        if (wv < BN / 64)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rh, (qg_lds*)(sHd + 64 * wv), 16, (uint32_t)t * (nsb * 16), 16 * j, 0,
+                                                     0);
+    };
+    // activation sums (thread: token t / 4, 4 of the 16) and scale of super-block j, through registers
+    typedef int v4i __attribute__((ext_vector_type(4)));
+    v4i bs[RS];
+    int da0;
+    const auto load_sb = [&](int j) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                acc[i][j][r] = 0.0f;
-                I1[i][j][r] = 0;
-            }
+        for (int i = 0; i < RS; ++i)
+            bs[i] = (v4i)__builtin_amdgcn_raw_buffer_load_b128(rs, (uint32_t)((t >> 2) + NT / 4 * i) * (K / 4) + 16 * (t & 3),
+                                                               64 * j, 0);
+        da0 = __builtin_amdgcn_raw_buffer_load_b32(rd, (uint32_t)min(t, BM - 1) * (nsb * 4), 4 * j, 0);
+    };
+    const auto store_sb = [&]() {
+#pragma unroll
+        for (int i = 0; i < RS; ++i)
+            sBs[t + NT * i] = make_uint2(qg_h2(bs[i].x, bs[i].y), qg_h2(bs[i].z, bs[i].w));
+        if (t < BM) sDa[t] = __int_as_float(da0);
+    };
 
-    QgKRegs st;
-    qgk_load<TT, TW>(st, 0, wq, wh, N, nsb, n0, aq, ad, as16, M, m0, K, sb0);
-    qgk_store<TT, TW>(st, 0, sW[0], sA[0], sSc[0], sD[0], sDm[0], sMn[0], sBs[0], sDa[0]);
-    __syncthreads();
-    for (int step = 0; step < nsteps; ++step) {
-        const int buf = step & 1, j = sb0 + (step >> 2), c = step & 3, jp = (step >> 2) & 1;
-        if (step + 1 < nsteps) qgk_load<TT, TW>(st, step + 1, wq, wh, N, nsb, n0, aq, ad, as16, M, m0, K, sb0);
+    qg_f16v acc[2];
+    qg_v16i I1[2];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {  // unit 2c + u
-            qg_v4i A[TT], B[TW];
-            int sc[TW];
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int i = 0; i < TT; ++i)
-                A[i] = *reinterpret_cast<const qg_v4i*>(sA[buf] + (32 * (TT * wt + i) + c32) * QG_LD + 32 * u + 16 * h);
+        for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
+
+    const int ar = 64 * wm + c32, wr = 32 * wn + c32;
+    const int ax = (c32 >> 1) & 7, wx = (c32 >> 2) & 3;  // the rows' XOR (64 wm, 32 i, 32 wn do not change them)
+    const auto half_step = [&](const uint4* sA, const uint4* sW, uint32_t scw, bool first) {
 #pragma unroll
-            for (int jj = 0; jj < TW; ++jj) {
-                const int rl = 32 * (TW * ww + jj) + c32;
-                B[jj] = *reinterpret_cast<const qg_v4i*>(sW[buf] + rl * QG_LD + 32 * u + 16 * h);
-                sc[jj] = sSc[jp][(2 * c + u) * BN + rl];
-            }
+        for (int cp = 0; cp < 2; ++cp) {
+            const uint4 x = sW[wr * 4 + ((2 * cp + h) ^ wx)];
 #pragma unroll
-            for (int i = 0; i < TT; ++i)
+            for (int v = 0; v < 2; ++v) {
+                const int u = 2 * cp + v;
+                const qg_v4i B = v == 0 ? qg_v4i{(int)(x.x & 0x0F0F0F0Fu), (int)(x.y & 0x0F0F0F0Fu), (int)(x.z & 0x0F0F0F0Fu),
+                                                 (int)(x.w & 0x0F0F0F0Fu)}
+                                        : qg_v4i{(int)((x.x >> 4) & 0x0F0F0F0Fu), (int)((x.y >> 4) & 0x0F0F0F0Fu),
+                                                 (int)((x.z >> 4) & 0x0F0F0F0Fu), (int)((x.w >> 4) & 0x0F0F0F0Fu)};
+                const int sc = (int)((scw >> (8 * u)) & 0xFFu);
 #pragma unroll
-                for (int jj = 0; jj < TW; ++jj) {
+                for (int i = 0; i < 2; ++i) {
+                    const uint4 a = sA[(ar + 32 * i) * 8 + ((2 * u + h) ^ ax)];
                     const qg_v16i zero = {};
-                    const qg_v16i C = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[i], B[jj], zero, 0, 0, 0);
+                    const qg_v16i C = __builtin_amdgcn_mfma_i32_32x32x32_i8(
+                        qg_v4i{(int)a.x, (int)a.y, (int)a.z, (int)a.w}, B, zero, 0, 0, 0);
+                    if (first && u == 0) {
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) I1[i][jj][r] += __mul24(C[r], sc[jj]);
-                }
-        }
-        if (c == 3) {  // end of super-block j: I2 (mins against the 16-sums) and the f32 epilogue
-#pragma unroll
-            for (int i = 0; i < TT; ++i) {
-                const int tl = 32 * (TT * wt + i) + 4 * h;
-                const qg_h8 Abs = *reinterpret_cast<const qg_h8*>(sBs[jp] + (32 * (TT * wt + i) + c32) * 16 + 8 * h);
-                float da[16];
-                if constexpr (!SUMS) {
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const float4 v = *reinterpret_cast<const float4*>(&sDa[jp][tl + 8 * q]);
-                        da[4 * q] = v.x;
-                        da[4 * q + 1] = v.y;
-                        da[4 * q + 2] = v.z;
-                        da[4 * q + 3] = v.w;
-                    }
-                }
-#pragma unroll
-                for (int jj = 0; jj < TW; ++jj) {
-                    const int rl = 32 * (TW * ww + jj) + c32;
-                    const qg_h8 Bmn = *reinterpret_cast<const qg_h8*>(sMn[jp] + rl * 16 + 8 * h);
-                    const qg_f16v zf = {};
-                    const qg_f16v I2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(Abs, Bmn, zf, 0, 0, 0);
-                    if constexpr (SUMS) {
-                        const int n = n0 + rl;
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            const int m = m0 + tl + 8 * (r >> 2) + (r & 3);
-                            if (m < M && n < N) {
-                                int32_t* o = sums + (((size_t)m * N + n) * nsb + j) * 2;
-                                o[0] = I1[i][jj][r];
-                                o[1] = (int)I2[r];
-                            }
-                        }
+                        for (int r = 0; r < 16; ++r) I1[i][r] = __mul24(C[r], sc);
                     } else {
-                        const float d = sD[jp][rl], dm = sDm[jp][rl];
 #pragma unroll
-                        for (int r = 0; r < 16; ++r)
-                            acc[i][jj][r] = fmaf(fmaf(d, (float)I1[i][jj][r], -(dm * I2[r])), da[r], acc[i][jj][r]);
+                        for (int r = 0; r < 16; ++r) I1[i][r] += __mul24(C[r], sc);
                     }
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) I1[i][jj][r] = 0;
                 }
+                // one unit's results at a time (more do not fit the registers), added up here (the compiler would move
+                // the additions behind the next barrier and keep the results until then)
+                asm volatile("" : "+v"(I1[0]), "+v"(I1[1]));
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if (step + 1 < nsteps) {
-            const int sp = ((step + 1) >> 2) & 1;
-            qgk_store<TT, TW>(st, step + 1, sW[buf ^ 1], sA[buf ^ 1], sSc[sp], sD[sp], sDm[sp], sMn[sp], sBs[sp],
-                              sDa[sp]);
-            __syncthreads();
-        }
-    }
-    if constexpr (!SUMS) {
+    };
+
+    load_head(min(sb0, sb_last));
+    load(sAa, sWa, min(sb0, sb_last), 0);
+    load_sb(min(sb0, sb_last));
+    QG_WAIT_LOADS();
+    __syncthreads();
+    for (int j = sb0; j < sb0 + run; ++j) {
+        const int jn = min(j + 1, sb_last);
+        load(sAb, sWb, min(j, sb_last), 1);
+        const uint4 hd = sHd[wr];
+        // scales and mins of units 0-3 and 4-7, one per byte
+        const uint32_t sc0 = hd.y & 0x3F3F3F3Fu, sc1 = (hd.w & 0x0F0F0F0Fu) | ((hd.y >> 2) & 0x30303030u);
+        const uint32_t mw = h ? ((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u) : hd.z & 0x3F3F3F3Fu;
+        half_step(sAa, sWa, sc0, true);
+        store_sb();
+        QG_WAIT_LOADS();
+        __syncthreads();
+        load(sAa, sWa, jn, 0);
+        load_head(jn);
+        load_sb(jn);
+        half_step(sAb, sWb, sc1, false);
+        // end of super-block j: I2 (mins, each on its unit's two 16-sum slots, against the sums) and the f32 epilogue
+        const qg_h8 Bmn = [&] {
+            const uint32_t off = 0xE400E400u;  // -1024, -1024: 0x6400 | m is the f16 1024 + m
+            typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+            qg_h8 r;
 #pragma unroll
-        for (int jj = 0; jj < TW; ++jj) {
-            const int n = n0 + 32 * (TW * ww + jj) + c32;
-            if (n >= N) continue;
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t p = __builtin_amdgcn_perm(0x64646464u, mw, 0x04000400u + 0x00010001u * e);
+                const h2 q = __builtin_bit_cast(h2, p) + __builtin_bit_cast(h2, off);
+                r[2 * e] = q.x;
+                r[2 * e + 1] = q.y;
+            }
+            return r;
+        }();
+        const float d = amv_h2f(hd.x), dm = amv_h2f(hd.x >> 16);
+        if (KG == 1 || j < sb_end)
 #pragma unroll
-            for (int i = 0; i < TT; ++i)
+        for (int i = 0; i < 2; ++i) {
+            const int tl = 64 * wm + 32 * i;
+            const qg_h8 Abs = *reinterpret_cast<const qg_h8*>(&sBs[(tl + c32) * 4 + 2 * h]);
+            const qg_f16v zf = {};
+            const qg_f16v I2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(Abs, Bmn, zf, 0, 0, 0);
+            if constexpr (SUMS) {
+                const int n = n0 + wr;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const int m = m0 + 32 * (TT * wt + i) + 8 * (r >> 2) + 4 * h + (r & 3);
-                    if (m < M) {
-                        const size_t o = (size_t)m * ldd + n;
-                        if constexpr (ADD) dst[o] = acc[i][jj][r] + add[o];
-                        else dst[o] = acc[i][jj][r];
+                    const int m = m0 + tl + 4 * h + 8 * (r >> 2) + (r & 3);
+                    if (m < M && n < N) {
+                        int32_t* o = sums + (((size_t)m * N + n) * nsb + j) * 2;
+                        o[0] = I1[i][r];
+                        o[1] = (int)I2[r];
                     }
                 }
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float4 v = *reinterpret_cast<const float4*>(&sDa[tl + 4 * h + 8 * q]);
+                    const float da[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        acc[i][4 * q + r] = fmaf(fmaf(d, (float)I1[i][4 * q + r], -(dm * I2[4 * q + r])), da[r],
+                                                 acc[i][4 * q + r]);
+                }
+            }
         }
+        QG_WAIT_LOADS();
+        __syncthreads();
     }
+    qg_finish<SUMS, BM, NT, KG, ADD>(acc, gAa, kg, t, n0 + wr, m0 + 64 * wm + 4 * h, M, N, dst, ldd, add);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -687,108 +665,166 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // host
 // ---------------------------------------------------------------------------------------------------------------
 // split of k shared with the f16 kernels (amv_mmq16.hip): workspace per device and the in-order partial sum
-float* amv_splitk_workspace(size_t bytes, hipStream_t st);
+float* amv_splitk_workspace(size_t bytes, hipStream_t st, bool optional = false);
 int amv_splitk_count(int64_t tiles, int steps);
 void amv_splitk_reduce(const float* part, int S, int64_t zstride, int64_t m, int64_t n, float* dst, int64_t ldd,
                        hipStream_t st, const float* add = nullptr);
 
-template <int TT, int TW>
-static int qgemm_launch(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int64_t m, float* dst,
-                         int64_t ldd, int32_t* sums, hipStream_t st, const float* add) {
-    constexpr int BM = 64 * TT, BN = 64 * TW;
-    const int8_t* aq = (const int8_t*)act;
-    const int n_tw = (int)((n_rows + BN - 1) / BN), n_tt = (int)((m + BM - 1) / BM);
-    const int64_t tiles = (int64_t)n_tw * n_tt;
-    const bool q4k = wtype == AMV_T_Q4_K, q6k = wtype == AMV_T_Q6_K, kq = q4k || q6k;
-    const int nb = (int)(k / 32), nsb = (int)(k / 256);
-    const int steps = q4k ? 4 * nsb : q6k ? 4 * nsb : (nb + 1) / 2;  // in units of 64 k
-    // split of k when the tiles leave CUs idle (partials in the library's workspace, summed in order of k)
-    int S = sums ? 1 : amv_splitk_count(tiles, steps);
-    int per = kq ? nsb : nb;
-    float* out = dst;
-    int64_t ldo = ldd, zstride = 0;
-    if (S > 1) {
-        per = kq ? (nsb + S - 1) / S : (((nb + S - 1) / S + 1) & ~1);
-        S = kq ? (nsb + per - 1) / per : (nb + per - 1) / per;
-        float* ws = S > 1 ? amv_splitk_workspace((size_t)S * m * n_rows * 4, st) : nullptr;
-        if (S > 1 && !ws) return AMV_ERR_HIP;  // never unsplit: the summation order would change
+// a launch's tiles and split of k (partials in the library's workspace, summed in order of k): k in units of `unit`
+// blocks, `n_unit` of them
+struct QgPlan {
+    int n_tw, n_tt, S, per;
+    float* out;
+    int64_t ldo, zstride;
+};
+static int qg_plan(QgPlan& p, int bm, int bn, int64_t n_rows, int64_t m, int64_t k, int n_blk, int align, float* dst,
+                   int64_t ldd, bool split, hipStream_t st) {
+    p.n_tw = (int)((n_rows + bn - 1) / bn);
+    p.n_tt = (int)((m + bm - 1) / bm);
+    p.S = split ? amv_splitk_count((int64_t)p.n_tw * p.n_tt, (int)(k / 64)) : 1;
+    p.per = n_blk;
+    p.out = dst;
+    p.ldo = ldd;
+    p.zstride = 0;
+    if (p.S > 1) {
+        p.per = ((n_blk + p.S - 1) / p.S + align - 1) / align * align;
+        p.S = (n_blk + p.per - 1) / p.per;
+    }
+    if (p.S > 1) {
+        // Never unsplit above 64 tokens: the summation order would change. Up to 64 tokens a capture that runs before any
+        // such call has no workspace and must not fail: it keeps k whole.
+        float* ws = amv_splitk_workspace((size_t)p.S * m * n_rows * 4, st, m <= 64);
+        if (!ws && m > 64) return AMV_ERR_HIP;
         if (ws) {
-            out = ws;
-            ldo = n_rows;
-            zstride = m * n_rows;
+            p.out = ws;
+            p.ldo = n_rows;
+            p.zstride = m * n_rows;
         } else {
-            S = 1;
-            per = kq ? nsb : nb;
+            p.S = 1;
+            p.per = n_blk;
         }
     }
-    const dim3 grid((unsigned)(tiles * S));
-    const float* kadd = S > 1 ? nullptr : add;  // with a split of k the residual joins in the sum of the partials
-    if (q6k) {  // ql [n][nsb][128] | qh [n][nsb][64] | scales [n][nsb][16] | d [n][nsb]
-        const int64_t nblk = n_rows * nsb;
-        const uint8_t* base = (const uint8_t*)w;
-        const uint4* wl = (const uint4*)base;
-        const uint4* wqh = (const uint4*)(base + nblk * 128);
-        const uint4* wsc = (const uint4*)(base + nblk * 192);
-        const uint16_t* wd = (const uint16_t*)(base + nblk * 208);
-        const float* ad = (const float*)(aq + m * k);
-        if (sums)
-            hipLaunchKernelGGL((k_qgemm_q6k<true, TT, TW>), grid, dim3(256), 0, st, wl, wqh, wsc, wd, (int)n_rows, nsb,
-                               aq, ad, (int)m, out, ldo, kadd, sums, per, zstride, n_tw, n_tt, S);
-        else if (kadd)
-            hipLaunchKernelGGL((k_qgemm_q6k<false, TT, TW, true>), grid, dim3(256), 0, st, wl, wqh, wsc, wd,
-                               (int)n_rows, nsb, aq, ad, (int)m, out, ldo, kadd, sums, per, zstride, n_tw, n_tt, S);
-        else
-            hipLaunchKernelGGL((k_qgemm_q6k<false, TT, TW>), grid, dim3(256), 0, st, wl, wqh, wsc, wd, (int)n_rows,
-                               nsb, aq, ad, (int)m, out, ldo, kadd, sums, per, zstride, n_tw, n_tt, S);
-    } else if (q4k) {
-        const int64_t nblk = n_rows * nsb;
-        const uint4* wq = (const uint4*)w;
-        const uint4* wh = (const uint4*)((const uint8_t*)w + nblk * 128);
-        const float* ad = (const float*)(aq + m * k);
-        const int32_t* as16 = (const int32_t*)(aq + m * k + m * nsb * 4);
-        if (sums)
-            hipLaunchKernelGGL((k_qgemm_q4k<true, TT, TW>), grid, dim3(256), 0, st, wq, wh, (int)n_rows, nsb, aq, ad,
-                               as16, (int)m, out, ldo, kadd, sums, per, zstride, n_tw, n_tt, S);
-        else if (kadd)
-            hipLaunchKernelGGL((k_qgemm_q4k<false, TT, TW, true>), grid, dim3(256), 0, st, wq, wh, (int)n_rows, nsb,
-                               aq, ad, as16, (int)m, out, ldo, kadd, sums, per, zstride, n_tw, n_tt, S);
-        else
-            hipLaunchKernelGGL((k_qgemm_q4k<false, TT, TW>), grid, dim3(256), 0, st, wq, wh, (int)n_rows, nsb, aq, ad,
-                               as16, (int)m, out, ldo, kadd, sums, per, zstride, n_tw, n_tt, S);
-    } else {
-        const int64_t nblk = n_rows * nb;
-        const uint8_t* wq = (const uint8_t*)w;
-        const uint16_t* wd = (const uint16_t*)(wq + nblk * (wtype == AMV_T_Q4_0 ? 16 : 32));
-        const int2* am = (const int2*)(aq + m * k);
-#define QG_LAUNCH(WT, SU, AD)                                                                                     \
-    hipLaunchKernelGGL((k_qgemm<WT, SU, TT, TW, AD>), grid, dim3(256), 0, st, wq, wd, (int)n_rows, nb, aq, am, (int)m, \
-                       out, ldo, kadd, sums, per, zstride, n_tw, n_tt, S)
-        if (wtype == AMV_T_Q4_0) {
-            if (sums) QG_LAUNCH(AMV_T_Q4_0, true, false);
-            else if (kadd) QG_LAUNCH(AMV_T_Q4_0, false, true);
-            else QG_LAUNCH(AMV_T_Q4_0, false, false);
-        } else {
-            if (sums) QG_LAUNCH(AMV_T_Q8_0, true, false);
-            else if (kadd) QG_LAUNCH(AMV_T_Q8_0, false, true);
-            else QG_LAUNCH(AMV_T_Q8_0, false, false);
-        }
-#undef QG_LAUNCH
-    }
-    if (S > 1) amv_splitk_reduce(out, S, zstride, m, n_rows, dst, ldd, st, add);
     return AMV_OK;
 }
 
-// Q4_0 / Q8_0 weights with plain Q8_0 activations (int8 [m][k], {f32 d, i32 sum} [m][k/32]); Q4_K weights with plain
-// Q8_K activations (int8 [m][k], f32 d [m][k/256], i32 sums per 16 [m][k/16]). The prefixes of the MMA / DEQ layouts
-// are these layouts. Tile: 128 x 128 while that gives at least 384 workgroups (1.5 per CU), else 64 x 64 (a split
-// of k then fills the GPU where the tiles alone cannot). Measured on MI355X (Q4_K, exact): 14336 x 4096 at 512
-// tokens 104 us with 128 x 128 against 115 us with 64 x 64; 6144 x 4096 at 512 tokens 55 us with 64 x 64 against
-// 65 us (64 x 128) and 76 us (128 x 128); 14336 x 4096 at 128 tokens 47 us with 64 x 64 against 52 and 75 us.
-int amv_qgemm(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int64_t m, float* dst,
-              int64_t ldd, int32_t* sums, hipStream_t st, const float* add) {
+struct QgCall {
+    const void* w;
+    int64_t n_rows, k;
+    const void* act;
+    int64_t m;
+    float* dst;
+    int64_t ldd;
+    int32_t* sums;
+    hipStream_t st;
+    const float* add;
+    bool split;  // k may be split over workgroups
+};
+
+// launches kernel<sums / plain / ADD> of a plan; A: the arguments after M
+#define QG_GO(KERNEL, THREADS, ...)                                                                                       \
+    do {                                                                                                                  \
+        const dim3 grid((unsigned)((int64_t)p.n_tw * p.n_tt * p.S));                                                      \
+        const float* kadd = p.S > 1 ? nullptr : c.add; /* with a split of k the residual joins in the partials' sum */    \
+        const auto fn = c.sums ? KERNEL(true, false) : kadd ? KERNEL(false, true) : KERNEL(false, false);                 \
+        hipLaunchKernelGGL(fn, grid, dim3(THREADS), 0, c.st, __VA_ARGS__, (int)c.m, p.out, p.ldo, kadd, c.sums, p.per,    \
+                           p.zstride, p.n_tw, p.n_tt, p.S);                                                               \
+        if (p.S > 1) amv_splitk_reduce(p.out, p.S, p.zstride, c.m, c.n_rows, c.dst, c.ldd, c.st, c.add);                  \
+    } while (0)
+
+template <int WT, int WM, int WN, int KG>
+static int qg_block(const QgCall& c) {
+    const int nb = (int)(c.k / 32);
+    QgPlan p;
+    const int rc = qg_plan(p, 64 * WM, 32 * WN, c.n_rows, c.m, c.k, nb, 4, c.dst, c.ldd, c.split, c.st);
+    if (rc) return rc;
+    const int8_t* aq = (const int8_t*)c.act;
+    const int2* am = (const int2*)(aq + c.m * c.k);
+    const uint8_t* wq = (const uint8_t*)c.w;
+    const uint16_t* wd = (const uint16_t*)(wq + c.n_rows * nb * (WT == AMV_T_Q4_0 ? 16 : 32));
+#define QG_K(SU, AD) k_qgemm<WT, SU, WM, WN, KG, AD>
+    QG_GO(QG_K, 64 * WM * WN * KG, wq, wd, (int)c.n_rows, nb, aq, am);
+#undef QG_K
+    return AMV_OK;
+}
+
+template <int WM, int WN, int KG>
+static int qg_q4k(const QgCall& c) {
+    const int nsb = (int)(c.k / 256);
+    QgPlan p;
+    const int rc = qg_plan(p, 64 * WM, 32 * WN, c.n_rows, c.m, c.k, nsb, 1, c.dst, c.ldd, c.split, c.st);
+    if (rc) return rc;
+    const int8_t* aq = (const int8_t*)c.act;
+    const uint4* wq = (const uint4*)c.w;
+    const uint4* wh = (const uint4*)((const uint8_t*)c.w + c.n_rows * nsb * 128);
+    const float* ad = (const float*)(aq + c.m * c.k);
+    const int32_t* as16 = (const int32_t*)(aq + c.m * c.k + c.m * nsb * 4);
+#define QG_K(SU, AD) k_qgemm_q4k<SU, WM, WN, KG, AD>
+    QG_GO(QG_K, 64 * WM * WN * KG, wq, wh, (int)c.n_rows, nsb, aq, ad, as16);
+#undef QG_K
+    return AMV_OK;
+}
+
+template <int TT, int TW>
+static int qg_q6k(const QgCall& c) {  // ql [n][nsb][128] | qh [n][nsb][64] | scales [n][nsb][16] | d [n][nsb]
+    const int nsb = (int)(c.k / 256);
+    QgPlan p;
+    const int rc = qg_plan(p, 64 * TT, 64 * TW, c.n_rows, c.m, c.k, nsb, 1, c.dst, c.ldd, c.split, c.st);
+    if (rc) return rc;
+    const int64_t nblk = c.n_rows * nsb;
+    const uint8_t* base = (const uint8_t*)c.w;
+    const uint4* wl = (const uint4*)base;
+    const uint4* wqh = (const uint4*)(base + nblk * 128);
+    const uint4* wsc = (const uint4*)(base + nblk * 192);
+    const uint16_t* wd = (const uint16_t*)(base + nblk * 208);
+    const int8_t* aq = (const int8_t*)c.act;
+    const float* ad = (const float*)(aq + c.m * c.k);
+#define QG_K(SU, AD) k_qgemm_q6k<SU, TT, TW, AD>
+    QG_GO(QG_K, 256, wl, wqh, wsc, wd, (int)c.n_rows, nsb, aq, ad);
+#undef QG_K
+    return AMV_OK;
+}
+#undef QG_GO
+
+int amv_qgemm(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int64_t m, float* dst, int64_t ldd,
+              int32_t* sums, hipStream_t st, const float* add) {
+    const QgCall c{w, n_rows, k, act, m, dst, ldd, sums, st, add, !sums};
     const auto tiles = [&](int bm, int bn) { return ((m + bm - 1) / bm) * ((n_rows + bn - 1) / bn); };
-    const int rc = tiles(128, 128) >= 384 ? qgemm_launch<2, 2>(wtype, w, n_rows, k, act, m, dst, ldd, sums, st, add)
-                                          : qgemm_launch<1, 1>(wtype, w, n_rows, k, act, m, dst, ldd, sums, st, add);
+    const auto wgs = [&](int bm, int bn) {  // workgroups with the split of k
+        return tiles(bm, bn) * (c.split ? amv_splitk_count(tiles(bm, bn), (int)(k / 64)) : 1);
+    };
+    // 64 x 64 tiles with four groups sharing k while that leaves at most one workgroup per CU, then 64 x 128 with four (two
+    // where LDS holds no more, or from one to two workgroups per CU), then a group to a workgroup on 128 x 128 (Q4_K below 384
+    // of them: 64 x 128; Q4_0 below that and without a split of k: 64 x 128, two groups). Measured (us; before: tiles staged through registers, 4 waves each,
+    // m <= 64 on 16 x 16 tiles):
+    //   rows x k, tokens     Q4_K           Q8_0           Q4_0
+    //   14336 x 4096,  48    18 (48)        22 (111)       22 (116)
+    //   4096 x 14336,  48    22 (173)       24 (373)       24 (395)
+    //   4096 x 4096,   96    16 (38)        19 (39)        21 (42)
+    //   14336 x 4096, 128    27 (46)        35 (51)        33 (52)
+    //   4096 x 4096,  512    29 (47)        39 (56)        39 (56)
+    //   14336 x 4096, 331    61 (94)        82 (122)       79 (114)
+    //   4096 x 14336, 331    67 (96)        76 (120)       81 (111)
+    //   14336 x 4096, 512    78 (97)        93 (117)       98 (110)
+    //   28672 x 4096, 512    158 (199)      187 (228)      195 (225)
+    // The neighbours of a choice: 14336 x 128 rows of Q4_K 35 with 64 x 64 tiles (448 of them), 6144 x 128 24 with 64 x 128
+    // (17 with 64 x 64), 4096 x 512 41 with one group (29 with four).
+    const bool t64 = wgs(64, 64) <= 256, t128 = wgs(64, 128) <= 256, two = wgs(64, 128) <= 512, big = tiles(128, 128) >= 384;
+    int rc;
+    if (wtype == AMV_T_Q4_K)
+        rc = t64    ? qg_q4k<1, 2, 4>(c)
+             : t128 ? qg_q4k<1, 4, 4>(c)
+             : two  ? qg_q4k<1, 4, 2>(c)
+             : big  ? qg_q4k<2, 4, 1>(c)
+                    : qg_q4k<1, 4, 1>(c);
+    else if (wtype == AMV_T_Q4_0)
+        rc = t64                ? qg_block<AMV_T_Q4_0, 1, 2, 4>(c)
+             : t128             ? qg_block<AMV_T_Q4_0, 1, 4, 4>(c)
+             : big || k >= 6144 ? qg_block<AMV_T_Q4_0, 2, 4, 1>(c)
+                                : qg_block<AMV_T_Q4_0, 1, 4, 2>(c);
+    else if (wtype == AMV_T_Q8_0)
+        rc = t64 ? qg_block<AMV_T_Q8_0, 1, 2, 4>(c) : t128 ? qg_block<AMV_T_Q8_0, 1, 4, 2>(c) : qg_block<AMV_T_Q8_0, 2, 4, 1>(c);
+    else
+        rc = big ? qg_q6k<2, 2>(c) : qg_q6k<1, 1>(c);
     if (rc) return rc;
     return amv_check_launch("amv_mul_mat_q_act");
 }

@@ -659,13 +659,13 @@ struct Engine {
         // batched (M >= 8) MUL_MATs run on the matrix cores for Q4_0 / Q8_0 / Q4_K / Q6_K (the reference's switch at
         // AMEVA_QGEMM_MIN_M). Above 64 tokens the exact form (exact per-block integer sums, ggml's f32 epilogue: the
         // reference's MMQ arithmetic) reads the plain Q8_0 / Q8_K layout (Q4_0: with room for its 6-bit digits); Q4_K
-        // batches of 8..64 tokens read the f16 copies of AMV_ACT_Q8_K_MMA; AMEVA_MMQ_FORM=scaled selects the scaled layouts (f16 q * d) above 64 tokens
+        // batches of 8..32 tokens read the f16 copies of AMV_ACT_Q8_K_MMA; AMEVA_MMQ_FORM=scaled selects the scaled layouts (f16 q * d) above 64 tokens
         const bool mmq = M >= 8 && (w->type == GGML_TYPE_Q4_0 || w->type == GGML_TYPE_Q8_0 || w->type == GGML_TYPE_Q4_K ||
                                     w->type == GGML_TYPE_Q6_K);
         const bool kq = w->type == GGML_TYPE_Q4_K || w->type == GGML_TYPE_Q6_K;
         const bool deq = mmq && M > 64 && mmq_scaled() && w->type != GGML_TYPE_Q6_K;  // Q6_K: exact form only
         const int atype = deq ? (kq ? AMV_ACT_Q8_K_DEQ : AMV_ACT_Q8_0_DEQ)
-                        : (mmq && w->type == GGML_TYPE_Q4_K && M <= 64) ? AMV_ACT_Q8_K_MMA
+                        : (mmq && w->type == GGML_TYPE_Q4_K && M <= 32) ? AMV_ACT_Q8_K_MMA
                         : (mmq && w->type == GGML_TYPE_Q4_0 && M > 64) ? AMV_ACT_Q8_0_F6
                         : kq ? (int)GGML_TYPE_Q8_K : (int)GGML_TYPE_Q8_0;
         if (!mmq && !ep && raw_readable(w)) return mul_mat_raw(n, atype);

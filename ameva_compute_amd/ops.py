@@ -71,7 +71,10 @@ def act_type(wtype: int, m: int = 1, exact: bool | None = None) -> int:
 
 def gemm_act_type(wtype: int, m: int) -> int:
     """The activation layout the fastest MUL_MAT of m tokens in MMQ_FORM's arithmetic takes: act_type's, with the digits'
-    scratch for Q4_0 above MMQ16_MIN_M tokens in the exact form (the same results from the 6-bit matrix instruction)."""
+    scratch for Q4_0 above MMQ16_MIN_M tokens in the exact form (the 6-bit matrix instruction), and without the f16
+    copies for Q4_K above QGEMM_MIN_M tokens (the tiled kernel reads the plain prefix)."""
+    if wtype == Q4_K and QGEMM_MIN_M < m <= MMQ16_MIN_M:
+        return Q8_K
     if wtype == Q4_0 and m > MMQ16_MIN_M and MMQ_FORM == "exact":
         return Q8_0_F6
     return act_type(wtype, m)
@@ -153,7 +156,8 @@ def quantize_q4_0(x: torch.Tensor) -> torch.Tensor:
 
 # batch size from which MUL_MAT runs the int8-MFMA kernel (AMEVA_QGEMM_MIN_M of the reference, ggml-ameva.cpp:2486)
 MMQ_MIN_M = 8
-MMQ16_MIN_M = 64  # above this many tokens the tiled kernels run (amv_mmq.hip MMQ16_MIN_M)
+QGEMM_MIN_M = 32  # above this many tokens the exact tiled kernels run (amv_mmq.hip QGEMM_MIN_M)
+MMQ16_MIN_M = 64  # above this many tokens the scaled form and act_type's plain Q4_K layout (amv_mmq.hip MMQ16_MIN_M)
 MMQ_TYPES = (Q4_0, Q8_0, Q4_K, Q6_K)  # Q4_K of MMQ_MIN_M..MMQ16_MIN_M tokens: the activations must be Q8_K_MMA
 
 

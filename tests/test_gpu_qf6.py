@@ -1,6 +1,6 @@
 """The batched Q4_0 MUL_MAT on the 6-bit matrix instruction (amv_qf6.hip, activation layout AMV_ACT_Q8_0_F6): block integers
-against the oracle bit for bit, outputs against the int8 kernel (the plain layout), at the edges of its tiles (128 and 64
-tokens, 128 rows, two-block steps, the two groups that share k, splits of k)."""
+against the oracle bit for bit, outputs against the int8 kernel (the plain layout), at the edges of its tiles (128 tokens,
+128 rows, two-block steps, splits of k)."""
 import numpy as np
 import pytest
 import torch
@@ -20,12 +20,12 @@ def _case(n, k, m, seed):
     return ops.QWeight.from_ggml(ops.Q4_0, wg, n, k), wg, torch.from_numpy(x).cuda()
 
 
-# (rows, k, tokens, exact): exact where one group sums all of k, as the int8 kernel does; elsewhere two f32 sums of
-# k / 32 products differ by at most 2 k / 32 roundings of 2^-24 of the sum of magnitudes
+# (rows, k, tokens, exact): exact where all of k is summed in one order, as the int8 kernel does (which also takes the small
+# launches); with k split at other places two f32 sums of k / 32 products differ by at most 2 k / 32 roundings of 2^-24 of
+# the sum of magnitudes
 @pytest.mark.parametrize("n,k,m,exact", [
-    (128, 32, 65, False), (127, 96, 66, False), (2, 64, 127, False), (257, 160, 128, False), (300, 1056, 129, False),
-    (1025, 512, 257, False), (12416, 256, 512, True), (12415, 224, 500, True), (8320, 96, 300, True),
-    (520, 6144, 65, False), (1030, 7200, 130, False)])
+    (128, 32, 65, True), (1025, 512, 257, True), (12416, 256, 512, True), (12415, 224, 500, True), (12290, 32, 511, True),
+    (49100, 96, 65, True), (3072, 7200, 500, False)])
 def test_f6_against_int8(n, k, m, exact):
     w, _, x = _case(n, k, m, n + k + m)
     print(n, k, m, flush=True)
@@ -43,7 +43,7 @@ def test_f6_against_int8(n, k, m, exact):
         assert bool(((y0 - y1).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("n,k,m", [(131, 96, 70), (256, 2048, 129), (12300, 64, 490)])
+@pytest.mark.parametrize("n,k,m", [(131, 96, 70), (12300, 96, 490)])
 def test_f6_block_sums(n, k, m):
     w, wg, x = _case(n, k, m, n * 3 + m)
     x[0, :32] = 127.0  # the largest digits
