@@ -245,6 +245,274 @@ __global__ __launch_bounds__(256) void k_fa_prefill(const float* __restrict__ q,
     }
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// The same attention with the K / V blocks shared by the waves of a workgroup, for launches that fill the GPU without
+// splitting a tile's keys further. 8 waves: 4 consecutive (query tile, head of the group) pairs of one KV head, head fastest,
+// so with 4 query heads per KV head a block of 32 keys is read from L2 once for 128 query rows (k_fa_prefill reads it once
+// per 32: 1 GB through L2 for 2048 causal tokens of 32 heads); each pair has two waves, which take the even and the odd
+// blocks and merge at the end (one wave per pair: 84 us against 75 before the next point, the longest tiles then run alone).
+// A block's exponentials run between the dependent products of the next block's scores. What bounds it: latency, at two
+// waves per SIMD (matrix cores 23 %, VALU 30 % busy).
+// K and V rows go from memory to LDS without registers (global_load_lds), one step ahead, double-buffered. The loads write
+// the rows as they come, so pieces of a row are exchanged by an XOR with the key index on the memory side: K 16-byte pieces
+// by key % 16 (the fragment reads of 16 keys hit all banks once), V 32-byte pieces by key % 8 (so do the transposing reads
+// of 8 keys). KV heads go to XCDs in turn, so an XCD's L2 serves one head's rows.
+// ---------------------------------------------------------------------------------------------------------------
+typedef __attribute__((address_space(3))) void fq_lds;
+typedef __attribute__((address_space(1))) const void fq_glb;
+// Every wave's LDS accesses done and at most n of its vector memory loads out, then the workgroup's barrier. (The fence of
+// __syncthreads would wait for all loads into LDS, the next step's too.)
+#define FQ_BARRIER(n)                              \
+    do {                                           \
+        asm volatile("" ::: "memory");             \
+        __builtin_amdgcn_s_waitcnt(0x0070 | (n));  \
+        __builtin_amdgcn_s_barrier();              \
+        asm volatile("" ::: "memory");             \
+    } while (0)
+
+template <bool MASK>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k_fa_prefill_sh(
+    const float* __restrict__ q, int64_t q_ts, int64_t q_hs, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+    const uint16_t* __restrict__ mask, int64_t mask_stride, float* __restrict__ out, int n_tok, int n_head, int n_head_kv,
+    int G, int n_kv, int64_t k_row, int64_t k_head, int64_t v_row, int64_t v_head, float scale, int64_t pos0) {
+    // two buffers as variables of their own: reads of one do not wait for the loads into the other
+    __shared__ __align__(16) uint16_t sKa[2 * FQ_KB * FQ_D], sKb[2 * FQ_KB * FQ_D], sVa[2 * FQ_KB * FQ_D], sVb[2 * FQ_KB * FQ_D];
+    const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, h = lane >> 5;
+    const int w8 = __builtin_amdgcn_readfirstlane(tid >> 6), w = w8 & 3, kg = w8 >> 2;
+    const int n_tiles = (n_tok + 31) / 32, n_units = n_tiles * G;
+    const int hk = (int)blockIdx.x % n_head_kv;
+    const int bx = (int)gridDim.x / n_head_kv - 1 - (int)blockIdx.x / n_head_kv;  // the most keys first
+    const int u = min(4 * bx + w, n_units - 1);  // (a wave past the last unit repeats it and stores nothing)
+    const bool idle = 4 * bx + w >= n_units;
+    const int q0 = 32 * (u / G), hq = hk * G + u % G;
+    const int qi = q0 + c, qc = min(qi, n_tok - 1);
+    // keys of a tile: up to the last key its last query may see
+    const auto keys = [&](int unit) {
+        const int t0 = 32 * (unit / G);
+        return pos0 >= 0 ? (int)min((int64_t)n_kv, pos0 + min(t0 + 31, n_tok - 1) + 1) : n_kv;
+    };
+    const int nblk = (keys(u) + FQ_KB - 1) / FQ_KB;
+    // steps of two blocks, one for each group of waves; the workgroup's last unit sees the most keys
+    const int nall = (keys(min(4 * bx + 3, n_units - 1)) + 2 * FQ_KB - 1) / (2 * FQ_KB);
+    const int qlim = (int)min(pos0 >= 0 ? pos0 + qi : (int64_t)n_kv, (int64_t)n_kv - 1);
+    const int klim0 = (int)min(pos0 >= 0 ? pos0 + q0 + 1 : (int64_t)n_kv, (int64_t)n_kv);
+    const float sl2 = scale * FQ_LOG2E;
+
+    // staging: piece x = tid + 512 i (i = 0, 1) of a step's 1024: key x / 16, place x % 16 of its row
+    const int srow = tid >> 4, kp = ((tid & 15) ^ (srow & 15)) * 8, vp = ((tid & 15) ^ (2 * (srow & 7))) * 8;  // (key + 32: same)
+    const uint16_t* kh = k + (int64_t)hk * k_head + kp;
+    const uint16_t* vh = v + (int64_t)hk * v_head + vp;
+    const auto load = [&](const uint16_t* src, int64_t row, uint16_t* to, int s) {  // the rows of step s
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int64_t key = min(2 * FQ_KB * s + srow + 32 * i, n_kv - 1);
+            __builtin_amdgcn_global_load_lds((fq_glb*)(src + key * row), (fq_lds*)(to + 4096 * i + 512 * w8), 16, 0, 0);
+        }
+    };
+    // ggml's mask: the query's 4 runs of 4 keys of a block, loaded with the block's rows
+    const uint16_t* mrow = MASK ? mask + (int64_t)qc * mask_stride : nullptr;
+    const bool mvec = MASK && ((uintptr_t)mask & 7) == 0 && mask_stride % 4 == 0;
+    uint2 mk[4];
+    const auto load_mask = [&](int b) {
+        if (!MASK) return;
+        const int k0 = FQ_KB * min(b, (n_kv - 1) / FQ_KB) + 4 * h;
+        if (mvec && k0 - 4 * h + FQ_KB <= n_kv) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) mk[g] = *reinterpret_cast<const uint2*>(mrow + k0 + 8 * g);
+        } else {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                uint32_t e[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) e[r] = mrow[min(k0 + 8 * g + r, n_kv - 1)];
+                mk[g] = make_uint2(e[0] | e[1] << 16, e[2] | e[3] << 16);
+            }
+        }
+    };
+    load_mask(kg);
+    load(kh, k_row, sKa, 0);
+    load(vh, v_row, sVa, 0);
+    load(kh, k_row, sKb, 1);
+
+    fq_h8 qb[8];  // Q^T operand: qb[s] = q[qi][16 s + 8 h .. + 7] as f16
+    {
+        const float* qr = q + (int64_t)qc * q_ts + (int64_t)hq * q_hs + 8 * h;
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const fq_f4 a = *reinterpret_cast<const fq_f4*>(qr + 16 * s), b = *reinterpret_cast<const fq_f4*>(qr + 16 * s + 4);
+            qb[s] = fq_h8{(_Float16)a.x, (_Float16)a.y, (_Float16)a.z, (_Float16)a.w,
+                          (_Float16)b.x, (_Float16)b.y, (_Float16)b.z, (_Float16)b.w};
+        }
+    }
+    float m = -INFINITY, l = 0.0f;
+    fq_f16v o[4];
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[dt][r] = 0.0f;
+    const int j16 = lane & 15, g16 = lane >> 4;
+    // S^T of a block: 8 dependent products; kx: the lane's row and XOR
+    const int kx = c * FQ_D;
+    const auto frag = [&](const uint16_t* sK, int st) {
+        return *reinterpret_cast<const fq_h8*>(&sK[kx + 8 * ((2 * st + h) ^ (c & 15))]);
+    };
+    const bool pos = sl2 >= 0.0f;
+    fq_f16v s = {};
+    // block b of this wave (scores s, rows of V in sV), and the scores of its next block from sK: the exponentials run
+    // between the dependent products
+    const auto step = [&](const uint16_t* sK, const uint16_t* sV, int b) {
+        const int kb0 = FQ_KB * b;
+        const bool full = kb0 + FQ_KB <= klim0;
+        if (MASK) {
+            bool any = false;
+            float x[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const uint32_t e = ((r & 2) ? mk[r >> 2].y : mk[r >> 2].x) >> (16 * (r & 1)) & 0xFFFFu;
+                any |= e != 0xFC00u;
+                x[r] = (s[r] * scale + amv_h2f(e)) * FQ_LOG2E;
+            }
+            load_mask(b + 2);
+            // a block that the mask hides from all 32 queries adds nothing (ggml skips such keys too)
+            if (!__builtin_amdgcn_ballot_w64(any)) {
+                fq_f16v z = {};
+#pragma unroll
+                for (int st = 0; st < 8; ++st) z = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag(sK, st), qb[st], z, 0, 0, 0);
+                s = z;
+                return;
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = x[r];
+        }
+        if (!full) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int key = kb0 + 8 * (r >> 2) + 4 * h + (r & 3);
+                if (key > qlim) s[r] = MASK || pos ? -INFINITY : INFINITY;  // (times sl2 below)
+            }
+        }
+        float mx = -INFINITY;
+        if (MASK || pos) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
+        } else {
+            mx = INFINITY;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mx = fminf(mx, s[r]);
+        }
+        const float f = MASK ? 1.0f : sl2;
+        mx = amv_max_x32(mx * f);
+        // The running maximum always moves (k_fa_prefill lets it lag by 8): the largest weight so far is then exactly 1, which
+        // outweighs the shorter key splits of that kernel (error against 64 bits at 2048 causal tokens 1.44e-4, there
+        // 1.55e-4; lagging by 8 it would be 1.59e-4 and 67 instead of 71 us)
+        const bool grow = mx > m;
+        if (__builtin_amdgcn_ballot_w64(grow)) {
+            const float alpha = grow ? (m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mx)) : 1.0f;
+            if (grow) m = mx;
+            l *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
+        }
+        const float mref = m == -INFINITY ? 0.0f : m;
+        // the weights' sum is taken over what enters the product, the f16 values (v_dot2_f32_f16: exact products, f32 sum):
+        // a query with one dominant key then keeps that key's row without the rounding of its weight
+        float rs = 0.0f;
+        fq_h8 p0, p1;
+        fq_f16v z = {};
+#pragma unroll
+        for (int st = 0; st < 8; ++st) z = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag(sK, st), qb[st], z, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) {
+            const amv_h2 e = {(_Float16)__builtin_amdgcn_exp2f(fmaf(s[r], f, -mref)),
+                              (_Float16)__builtin_amdgcn_exp2f(fmaf(s[r + 1], f, -mref))};
+            rs = __builtin_amdgcn_fdot2(e, amv_h2{(_Float16)1.0f, (_Float16)1.0f}, rs, false);
+            (r < 8 ? p0 : p1)[r & 7] = e.x;
+            (r < 8 ? p0 : p1)[(r + 1) & 7] = e.y;
+        }
+        __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);  // operand reads, then a product and its share of the VALU
+#pragma unroll
+        for (int st = 0; st < 8; ++st) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x402, 7, 0);
+        }
+        l += amv_sum_x32(rs);
+        s = z;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) {
+                // keys k0 + j16 / 4 (and + 8), dims 32 dt + 16 (g16 & 1) + 4 (j16 % 4) ..
+                const int key = 16 * ks + 4 * (g16 >> 1) + (j16 >> 2), unit = 2 * dt + (g16 & 1);
+                const uint16_t* p = &sV[key * FQ_D + 16 * (unit ^ (key & 7)) + 4 * (j16 & 3)];
+                const fq_s4 a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((fq_lds_s4*)(__attribute__((address_space(3))) uint16_t*)p);
+                const fq_s4 a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (fq_lds_s4*)(__attribute__((address_space(3))) uint16_t*)(p + 8 * FQ_D));
+                typedef short fq_s8 __attribute__((ext_vector_type(8)));
+                const fq_s8 ab = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
+                o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(fq_h8, ab), ks ? p1 : p0, o[dt], 0, 0, 0);
+            }
+    };
+    const int kv = kg * FQ_KB * FQ_D;  // the group's block of a step
+    FQ_BARRIER(0);
+    if (kg < nblk)
+#pragma unroll
+        for (int st = 0; st < 8; ++st) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag(sKa + kv, st), qb[st], s, 0, 0, 0);
+    FQ_BARRIER(0);
+    // step i: K rows of step i + 2 into the buffer that step i's came from, V rows of step i + 1 (past the last block: the
+    // last key again), then the wave's block
+    for (int i = 0;; i += 2) {
+        load(kh, k_row, sKa, i + 2);
+        load(vh, v_row, sVb, i + 1);
+        if (2 * i + kg < nblk) step(sKb + kv, sVa + kv, 2 * i + kg);
+        FQ_BARRIER(0);
+        if (i + 1 >= nall) break;
+        load(kh, k_row, sKb, i + 3);
+        load(vh, v_row, sVa, i + 2);
+        if (2 * (i + 1) + kg < nblk) step(sKa + kv, sVb + kv, 2 * (i + 1) + kg);
+        FQ_BARRIER(0);
+        if (i + 2 >= nall) break;
+    }
+    // the second group's (m, l, O^T) joins the first's: a quarter of O^T in each buffer, then m and l
+    float* const ex[4] = {reinterpret_cast<float*>(sKa), reinterpret_cast<float*>(sKb), reinterpret_cast<float*>(sVa),
+                          reinterpret_cast<float*>(sVb)};
+    const int t4 = tid & 255;
+    if (kg) {
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) ex[dt][r * 256 + t4] = o[dt][r];
+    }
+    float mo = m, lo = l;
+    __syncthreads();
+    fq_f16v o1[4];
+    if (!kg)
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o1[dt][r] = ex[dt][r * 256 + t4];
+    __syncthreads();
+    if (kg) {
+        ex[0][t4] = mo;
+        ex[1][t4] = lo;
+    }
+    __syncthreads();
+    if (kg || idle || qi >= n_tok) return;
+    const float m1 = ex[0][t4], l1 = ex[1][t4], M = fmaxf(m, m1);
+    const float f0 = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - M), f1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - M);
+    const float L = l * f0 + l1 * f1;
+    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+    float* orow = out + ((int64_t)qi * n_head + hq) * FQ_D + 4 * h;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+            fq_f4 v;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = (o[dt][4 * q4 + r] * f0 + o1[dt][4 * q4 + r] * f1) * inv;
+            *reinterpret_cast<fq_f4*>(orow + 32 * dt + 8 * q4) = v;
+        }
+}
+
 extern "C" int amv_flash_attn_prefill(const float* q, int64_t q_tok_stride, int64_t q_head_stride, const void* k,
                                       const void* v, const void* mask, int64_t mask_stride, float* out, int64_t n_tok,
                                       int64_t n_head, int64_t n_head_kv, int64_t n_kv, int64_t D, int64_t k_row,
@@ -264,6 +532,18 @@ extern "C" int amv_flash_attn_prefill(const float* q, int64_t q_tok_stride, int6
     AMV_REQUIRE(((uintptr_t)out & 15) == 0, "amv_flash_attn_prefill: out must be 16-byte aligned");
     AMV_REQUIRE(mask == nullptr || mask_stride >= n_kv, "amv_flash_attn_prefill: mask stride %lld < n_kv",
                 (long long)mask_stride);
+    const int64_t G = n_head / n_head_kv, wgs = ((n_tok + 31) / 32 * G + 3) / 4 * n_head_kv;
+    // Shared blocks once its workgroups (8 waves each) fill most CUs, with a mask from half of them (us, k_fa_prefill in
+    // brackets, 32 heads / 8 KV heads): 2048 causal tokens 71 (127), masked 136 (323); 1024 32 (46), 45 (94); 1024 after
+    // 1024 53 (80); 512 19 (18), 25 (29); 200 13 (9), 19 (12). Fewer tokens keep the kernel that splits a tile's keys over
+    // its four waves.
+    if (wgs >= (mask ? 128 : 192)) {
+        hipLaunchKernelGGL(mask ? k_fa_prefill_sh<true> : k_fa_prefill_sh<false>, dim3((unsigned)wgs), dim3(512), 0,
+                           amv_stream(stream), q, q_tok_stride, q_head_stride, (const uint16_t*)k, (const uint16_t*)v,
+                           (const uint16_t*)mask, mask_stride, out, (int)n_tok, (int)n_head, (int)n_head_kv, (int)G,
+                           (int)n_kv, k_row, k_head, v_row, v_head, scale, causal_pos0);
+        return amv_check_launch("amv_flash_attn_prefill");
+    }
     const dim3 grid((unsigned)((n_tok + 31) / 32), (unsigned)n_head);
     hipLaunchKernelGGL(mask ? k_fa_prefill<true> : k_fa_prefill<false>, grid, dim3(256), 0, amv_stream(stream), q, q_tok_stride, q_head_stride,
                        (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)mask, mask_stride, out, (int)n_tok,
