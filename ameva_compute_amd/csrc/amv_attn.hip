@@ -8,9 +8,9 @@
 // score = sum_b float(isum_b) * (d_k * d_q) (vec_dot_q8_0_q8_0 / vec_dot_q4_0_q8_0). A quantized V row is dequantized
 // exactly (q * d). Scores, probabilities and accumulators are f32.
 //
-// Pass 1 (k_fa_split): one workgroup of 4 waves per (key split, KV head); each wave owns KPW consecutive keys and
-// works alone (16 lanes per 256-byte K/V row, G partial dots reduced over the 16 lanes, wave maximum, probabilities
-// and P V in registers); the 4 wave partials meet once in LDS and the workgroup's (m, l, acc[D]) per head goes to
+// Pass 1 (k_fa_split_mf for an f16 cache, k_fa_split_mq for Q8_0 / Q4_0, k_fa_split for f32): one workgroup of 4 waves
+// per (key split, KV head); each wave owns KPW consecutive keys and works alone (wave maximum, probabilities and P V in
+// registers); the 4 wave partials meet once in LDS and the workgroup's (m, l, acc[D]) per head goes to
 // the workspace. Pass 2 (fa_merge): per head M = max m_z, w_z = e^(m_z - M), L = sum l_z w_z,
 // out = sum w_z acc_z / L, with the quantization of the output for the next MUL_MAT fused. The merge runs either
 // as its own launch (k_fa_combine, one workgroup per head) or in the last workgroup of each KV head to finish its
@@ -159,89 +159,34 @@ __device__ __forceinline__ void fa_merge(const float* part, int n_split, int ns,
     }
 }
 
-// One workgroup per (split of 4 * KPW keys, KV head); each of its 4 waves owns KPW consecutive keys and works alone:
-// a 16-lane group owns keys 4 u + grp (u < KPW / 4) and reads 16 B of every K and V row of them (all K and V loads of
-// the wave are issued before the first is used); the G scores of a key are reduced over its 16 lanes; the wave's
-// maximum, probabilities, l and P V stay in registers. The 4 wave partials are merged once through LDS.
-// The key count is read from n_kv_dev when given (capped at the launch's n_kv); splits past it do nothing. FUSED: the
-// last workgroup of each KV head to arrive merges the head's splits (fa_merge).
-// cache element types of the split kernel
+// cache element types of the split kernels
 #define FA_F16 0
 #define FA_Q8_0 1
 #define FA_Q4_0 2
 #define FA_F32 3  // the BitNet engine's cache (llama_bitnet_core.cpp:1022-1082): f32 q . k, no rounding of q
 
-// A lane's slice of a K / V row: .a (and .b for an f32 row, whose 8 elements are 32 bytes).
+// Pass 1 for an f32 cache. One workgroup per (split of 4 * KPW keys, KV head); each of its 4 waves owns KPW consecutive
+// keys and works alone: a 16-lane group owns keys 4 u + grp (u < KPW / 4) and reads 32 B of every K and V row of them
+// (all K and V loads of the wave are issued before the first is used); the G scores of a key are reduced over its 16
+// lanes; the wave's maximum, probabilities, l and P V stay in registers. The 4 wave partials are merged once through LDS.
+// The key count is read from n_kv_dev when given (capped at the launch's n_kv); splits past it do nothing. FUSED: the
+// last workgroup of each KV head to arrive merges the head's splits (fa_merge).
+
+// A lane's slice of an f32 K / V row: elements 8 l16 .. 8 l16 + 7 (lane l16 = 0..15 of its 16-lane group).
 struct FaRow {
     uint4 a, b;
 };
-
-// The slice of one K / V row a lane works on: lane l16 (0..15 of its 16-lane group) owns elements 8 l16 .. 8 l16 + 7.
-// f32: those 32 bytes (.a, .b). f16: those 16 bytes. Q8_0 / Q4_0 (ggml blocks of 34 / 18 bytes): element offset o = 8 (l16 & 3) in block l16 / 4;
-// .x, .y = the 8 int8 (Q8_0) or the 8 qs bytes whose low (o < 16) or high (o >= 16) nibbles are the elements (Q4_0),
-// .z = the block's fp16 d. Quantized rows need only 2-byte alignment (halfword loads).
-template <int KT>
 __device__ __forceinline__ FaRow fa_row(const uint8_t* __restrict__ row, int l16) {
-    if constexpr (KT == FA_F32) {
-        const uint4* p = reinterpret_cast<const uint4*>(row + 32 * l16);
-        return FaRow{amv_ld_stream(p), amv_ld_stream(p + 1)};
-    } else if constexpr (KT == FA_F16) {
-        return FaRow{amv_ld_stream(reinterpret_cast<const uint4*>(row + 16 * l16)), make_uint4(0u, 0u, 0u, 0u)};
-    } else {
-        constexpr int BB = KT == FA_Q8_0 ? 34 : 18;
-        const int o = 8 * (l16 & 3);
-        const uint16_t* bp = reinterpret_cast<const uint16_t*>(row + BB * (l16 >> 2));
-        const int h = KT == FA_Q8_0 ? 1 + (o >> 1) : 1 + ((o & 15) >> 1);
-        // halfword pieces of lines the 16 lanes share: ordinary (cached) loads
-        const uint32_t b0 = bp[h], b1 = bp[h + 1], b2 = bp[h + 2], b3 = bp[h + 3];
-        return FaRow{make_uint4(b0 | (b1 << 16), b2 | (b3 << 16), bp[0], 0u), make_uint4(0u, 0u, 0u, 0u)};
-    }
+    const uint4* p = reinterpret_cast<const uint4*>(row + 32 * l16);
+    return FaRow{amv_ld_stream(p), amv_ld_stream(p + 1)};
 }
 
-// The 8 elements of a quantized slice as signed bytes (Q4_0: the nibbles, not yet offset by -8).
-template <int KT>
-__device__ __forceinline__ uint2 fa_bytes(const uint4& r, int lane) {
-    if constexpr (KT == FA_Q4_0) {
-        const int sh = (lane & 3) >= 2 ? 4 : 0;
-        return make_uint2((r.x >> sh) & 0x0F0F0F0Fu, (r.y >> sh) & 0x0F0F0F0Fu);
-    } else {
-        return make_uint2(r.x, r.y);
-    }
-}
-
-// Q8_0 of q for a quantized K: the 32-block of a lane's 8 elements spans the 4 lanes l16 = 4 b .. 4 b + 3; rules of
-// amv_quantize_act (ggml quantize_row_q8_0). qq: the lane's 8 int8, dq: the block's fp16-rounded d, qs: the sum of
-// the lane's 8 q.
-__device__ __forceinline__ void fa_quant_q(const float (&x)[8], int rule, uint32_t (&qq)[2], float& dq, int& qs) {
-    float amax = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(x[e]));
-    amax = fmaxf(amax, __shfl_xor(amax, 1, AMV_WAVE));
-    amax = fmaxf(amax, __shfl_xor(amax, 2, AMV_WAVE));
-    const float d = amax / 127.0f;
-    float id;
-    if (rule == AMV_Q8_X86) id = amax != 0.0f ? 127.0f / amax : 0.0f;
-    else id = d != 0.0f ? 1.0f / d : 0.0f;
-    qq[0] = qq[1] = 0u;
-    qs = 0;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const float t = x[e] * id;
-        float qf = rule == AMV_Q8_REF ? roundf(t) : rintf(t);
-        qf = fminf(127.0f, fmaxf(-127.0f, qf));
-        const int qi = (int)qf;
-        qs += qi;
-        qq[e >> 2] |= (uint32_t)(qi & 0xFF) << (8 * (e & 3));
-    }
-    dq = amv_h2f(amv_f2h(d));
-}
-
-template <int G, int KPW, bool FUSED, int KT>
+template <int G, int KPW, bool FUSED>
 __global__ __launch_bounds__(256) void k_fa_split(const float* __restrict__ q, const uint8_t* __restrict__ k,
                                                  const uint8_t* __restrict__ v, const uint16_t* __restrict__ mask,
                                                  float* part, int n_kv_max, const int* __restrict__ n_kv_dev,
                                                  int64_t k_row, int64_t k_head, int64_t v_row, int64_t v_head,
-                                                 int n_split, float scale, int qrule, unsigned int* counters,
+                                                 int n_split, float scale, unsigned int* counters,
                                                  float* __restrict__ out, const AmvActOut act) {
     constexpr int U = KPW / 4;
     constexpr int SBUF = 4 * 4 * G * FA_D > G * (8 * FA_D + FA_MAX_NSPLIT + 1) ? 4 * 4 * G * FA_D
@@ -263,12 +208,12 @@ __global__ __launch_bounds__(256) void k_fa_split(const float* __restrict__ q, c
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int i = min(kw0 + 4 * u + grp, n_kv - 1);
-            kr[u] = fa_row<KT>(kh + (size_t)i * k_row, lane & 15);
+            kr[u] = fa_row(kh + (size_t)i * k_row, lane & 15);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int i = min(kw0 + 4 * u + grp, n_kv - 1);
-            vr[u] = fa_row<KT>(vh + (size_t)i * v_row, lane & 15);
+            vr[u] = fa_row(vh + (size_t)i * v_row, lane & 15);
         }
         // the mask values of the lane's keys, loaded with the rest and converted where they are used (a load behind
         // a branch, or converted here, makes the compiler wait for every load issued so far); without a mask the
@@ -279,70 +224,32 @@ __global__ __launch_bounds__(256) void k_fa_split(const float* __restrict__ q, c
 #pragma unroll
             for (int u = 0; u < U; ++u) mraw[u] = mp[mask ? min(kw0 + 4 * u + grp, n_kv - 1) : 0];
         }
-        // q of the G heads, 8 dims per lane: rounded to f16 for an f16 cache, else quantized to Q8_0 blocks
-        float qv[G][8];
-        uint32_t qq[G][2];
-        float qd[G];
-        int qsum[G];
-        amv_h2 qh[G][4];  // f16 cache: q as f16 pairs
+        float qv[G][8];  // q of the G heads, 8 dims per lane
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             const float4* qp = reinterpret_cast<const float4*>(q + (size_t)(hk * G + g) * FA_D + d8);
             const float4 a = qp[0], b = qp[1];
             const float t[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
-            for (int e = 0; e < 8; ++e) qv[g][e] = KT == FA_F16 ? amv_round_f16(t[e]) : t[e];
-            if constexpr (KT == FA_Q8_0 || KT == FA_Q4_0) fa_quant_q(qv[g], qrule, qq[g], qd[g], qsum[g]);
-            if constexpr (KT == FA_F16)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) qh[g][e] = amv_h2{(_Float16)qv[g][2 * e], (_Float16)qv[g][2 * e + 1]};
+            for (int e = 0; e < 8; ++e) qv[g][e] = t[e];
         }
         float s[U][G];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int i = kw0 + 4 * u + grp;
             const float mk = (i < n_kv) ? (mask ? amv_h2f(mraw[u]) : 0.0f) : -INFINITY;
-            if constexpr (KT == FA_F16) {
-                // q (rounded to f16) . k as 4 v_dot2_f32_f16 per head: the f16 products are exact in f32
-                const uint32_t kw[4] = {kr[u].a.x, kr[u].a.y, kr[u].a.z, kr[u].a.w};
+            const uint4 x0 = kr[u].a, x1 = kr[u].b;
+            const uint32_t kw[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+            float kf[8];
 #pragma unroll
-                for (int g = 0; g < G; ++g) {
-                    float d = 0.0f;
+            for (int e = 0; e < 8; ++e) kf[e] = __uint_as_float(kw[e]);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) d = __builtin_amdgcn_fdot2(__builtin_bit_cast(amv_h2, kw[e]), qh[g][e], d, false);
-                    d = amv_row16_sum(d);
-                    s[u][g] = (mk == -INFINITY) ? -INFINITY : (d * scale + mk) * AMV_LOG2E;
-                }
-            } else if constexpr (KT == FA_F32) {
-                float kf[8];
-                const uint4 x0 = kr[u].a, x1 = kr[u].b;
-                const uint32_t kw[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+            for (int g = 0; g < G; ++g) {
+                float d = 0.0f;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) kf[e] = __uint_as_float(kw[e]);
-#pragma unroll
-                for (int g = 0; g < G; ++g) {
-                    float d = 0.0f;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) d = fmaf(qv[g][e], kf[e], d);
-                    d = amv_row16_sum(d);
-                    s[u][g] = (mk == -INFINITY) ? -INFINITY : (d * scale + mk) * AMV_LOG2E;
-                }
-            } else {
-                const uint2 kb = fa_bytes<KT>(kr[u].a, lane);
-                const float dk = amv_h2f((uint16_t)kr[u].a.z);
-#pragma unroll
-                for (int g = 0; g < G; ++g) {
-                    int is = amv_dot4((int)kb.x, (int)qq[g][0], amv_dot4((int)kb.y, (int)qq[g][1], 0));
-                    if constexpr (KT == FA_Q4_0) is -= 8 * qsum[g];
-                    is += __shfl_xor(is, 1, AMV_WAVE);  // the block's exact integer sum in its 4 lanes
-                    is += __shfl_xor(is, 2, AMV_WAVE);
-                    // vec_dot_q8_0_q8_0: isum * (d_k * d_q); vec_dot_q4_0_q8_0: (isum * d_k) * d_q
-                    const float t = (lane & 3) != 0         ? 0.0f
-                                    : KT == FA_Q8_0 ? (float)is * (dk * qd[g])
-                                                    : ((float)is * dk) * qd[g];
-                    const float d = amv_row16_sum(t);
-                    s[u][g] = (mk == -INFINITY) ? -INFINITY : (d * scale + mk) * AMV_LOG2E;
-                }
+                for (int e = 0; e < 8; ++e) d = fmaf(qv[g][e], kf[e], d);
+                d = amv_row16_sum(d);
+                s[u][g] = (mk == -INFINITY) ? -INFINITY : (d * scale + mk) * AMV_LOG2E;
             }
         }
         float m[G], l[G];
@@ -371,29 +278,10 @@ __global__ __launch_bounds__(256) void k_fa_split(const float* __restrict__ q, c
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             float vf[8];
-            if constexpr (KT == FA_F32) {
-                const uint4 x0 = vr[u].a, x1 = vr[u].b;
-                const uint32_t vw[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+            const uint4 x0 = vr[u].a, x1 = vr[u].b;
+            const uint32_t vw[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
 #pragma unroll
-                for (int e = 0; e < 8; ++e) vf[e] = __uint_as_float(vw[e]);
-            } else if constexpr (KT == FA_F16) {
-                const uint32_t vw[4] = {vr[u].a.x, vr[u].a.y, vr[u].a.z, vr[u].a.w};
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    vf[2 * e] = amv_h2f(vw[e] & 0xFFFFu);
-                    vf[2 * e + 1] = amv_h2f(vw[e] >> 16);
-                }
-            } else {  // ggml dequantize_row_q8_0 / q4_0: q * d, (nibble - 8) * d
-                const uint2 vb = fa_bytes<KT>(vr[u].a, lane);
-                const float dv = amv_h2f((uint16_t)vr[u].a.z);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int lo = KT == FA_Q8_0 ? (int)(int8_t)(vb.x >> (8 * e)) : (int)((vb.x >> (8 * e)) & 0xFF) - 8;
-                    const int hi = KT == FA_Q8_0 ? (int)(int8_t)(vb.y >> (8 * e)) : (int)((vb.y >> (8 * e)) & 0xFF) - 8;
-                    vf[e] = (float)lo * dv;
-                    vf[4 + e] = (float)hi * dv;
-                }
-            }
+            for (int e = 0; e < 8; ++e) vf[e] = __uint_as_float(vw[e]);
 #pragma unroll
             for (int g = 0; g < G; ++g)
 #pragma unroll
@@ -450,8 +338,8 @@ __global__ __launch_bounds__(256) void k_fa_split(const float* __restrict__ q, c
     }
 }
 
-// Pass 1 for an f16 cache with q . k on the matrix cores (KPW = 16 or 32 keys per wave, as k_fa_split<G, KPW, FUSED,
-// FA_F16>, same splits and partials; 32 at long contexts: 16384 / 32768 keys 18.7 / 30.5 us against 20.0 / 32.4 us
+// Pass 1 for an f16 cache with q . k on the matrix cores (KPW = 16 or 32 keys per wave, as k_fa_split,
+// same splits and partials; 32 at long contexts: 16384 / 32768 keys 18.7 / 30.5 us against 20.0 / 32.4 us
 // for the VALU form): per 16-key chunk, S = K q^T of its 16 keys and the G heads is four v_mfma_f32_16x16x32_f16
 // over the 128 dims (A: key l % 16, dims 32 kk + 8 (l / 16) .. + 7 of its row, loaded as 16 bytes; B: q of head
 // l % 16 rounded to f16, zero columns from G on), so the f16 products are exact and summed in f32 as the dot2 form
@@ -649,6 +537,260 @@ __global__ __launch_bounds__(256) void k_fa_split_mf(const float* __restrict__ q
     }
 }
 
+// Pass 1 for a Q8_0 or Q4_0 cache with the integer block dots on the matrix cores (same splits and partials): per
+// 16-key chunk and 32-block one v_mfma_i32_16x16x32_i8 gives the exact block integers of 16 keys and the G heads (A: key
+// l % 16, 8 bytes at dims 8 (l / 16); B: the quantized q of head l % 16, zero columns from G on; Q4_0: C = -8 sum(q)).
+// Lane l then holds keys 4 (l / 16) + e of head l % 16 and applies the blocks' scales as ggml does:
+// vec_dot_q8_0_q8_0 isum * (d_k * d_q), vec_dot_q4_0_q8_0 (isum * d_k) * d_q. Each of the 4 waves quantizes one of q's
+// 4 blocks for all. What bounded this before (8 dot4 per lane, then per key and head two LDS round trips to add a block's
+// lanes, a 16-lane sum, and q quantized by every lane group) was that work and not the cache's bytes: Q8_0, 8192 keys, 8
+// KV heads of 4 heads with the merge: 19.5 us, now 14.4 ( the rows are 17.8 MB, 3.5 us at the rate of a
+// copy). Rows are only 2-byte aligned: 8-byte loads at that alignment, where halfwords were read one by one. V: 16 lanes
+// per row, 8 dims per lane.
+typedef uint2 __attribute__((aligned(2))) fa_u2a;
+typedef int fa_i4 __attribute__((ext_vector_type(4)));
+
+struct FaQ {
+    uint2 b;
+    uint32_t d;
+};
+// the bytes that hold elements 8 j .. 8 j + 7 (j = 0..3) of block b of a quantized row (Q4_0: j >= 2 the high nibbles)
+// and the block's f16 scale
+template <int KT>
+__device__ __forceinline__ FaQ fa_q8(const uint8_t* __restrict__ row, int b, int j) {
+    constexpr int BB = KT == FA_Q8_0 ? 34 : 18;
+    const uint8_t* p = row + BB * b;
+    return FaQ{*reinterpret_cast<const fa_u2a*>(p + 2 + 8 * (KT == FA_Q8_0 ? j : j & 1)),
+               *reinterpret_cast<const uint16_t*>(p)};
+}
+
+template <int G, bool FUSED, int KPW, int KT>
+__global__ __launch_bounds__(256) void k_fa_split_mq(const float* __restrict__ q, const uint8_t* __restrict__ k,
+                                                    const uint8_t* __restrict__ v, const uint16_t* __restrict__ mask,
+                                                    float* part, int n_kv_max, const int* __restrict__ n_kv_dev,
+                                                    int64_t k_row, int64_t k_head, int64_t v_row, int64_t v_head,
+                                                    int n_split, float scale, int qrule, unsigned int* counters,
+                                                    float* __restrict__ out, const AmvActOut act) {
+    constexpr int NC = KPW / 16, U = 4;  // 16-key chunks per wave
+    constexpr int BB = KT == FA_Q8_0 ? 34 : 18;
+    static_assert(KPW == 16 || KPW == 32, "16 or 32 keys per wave");
+    constexpr int SBUF = 4 * 4 * G * FA_D > G * (8 * FA_D + FA_MAX_NSPLIT + 1) ? 4 * 4 * G * FA_D
+                                                                              : G * (8 * FA_D + FA_MAX_NSPLIT + 1);
+    __shared__ __align__(16) float sbuf[SBUF];  // [wave][lane group][head][dim] partial P V; then the merge
+    __shared__ float sM[4][G], sL[4][G];
+    __shared__ float sP[4][KPW][G];                      // per wave: probability of key, head
+    __shared__ __align__(16) float sDk[4][NC][4][16];    // per wave: K scale of chunk, block, key
+    __shared__ __align__(8) uint2 sQ[4][64];             // q's block, operand of lane
+    __shared__ float sDq[4][16];                         // its scale by head
+    __shared__ int sSq[4][16];                           // and its sum
+    const int split = blockIdx.y, hk = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int grp = lane >> 4, c16 = lane & 15, d8 = 8 * c16;
+    int n_kv = n_kv_max;
+    if (n_kv_dev) n_kv = max(0, min(*n_kv_dev, n_kv_max));
+    const int ns = (n_kv + 4 * KPW - 1) / (4 * KPW);  // splits holding keys
+    if (split < ns) {                                 // uniform per workgroup
+        const int kw0 = split * 4 * KPW + wv * KPW;   // first key of this wave; keys past the last read its row
+        const int klast = n_kv - 1;
+        const uint8_t* kh = k + (size_t)hk * k_head;
+        const uint8_t* vh = v + (size_t)hk * v_head;
+        // K: lane (grp, c16) takes key kw0 + 16 c + c16, elements 8 grp .. of each block, and the scale of block grp
+        uint2 kr[NC][4];
+        uint16_t kd[NC];
+        FaQ vr[NC][U];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const uint8_t* row = kh + (size_t)min(kw0 + 16 * c + c16, klast) * k_row;
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk)
+                kr[c][kk] = *reinterpret_cast<const fa_u2a*>(row + BB * kk + 2 + 8 * (KT == FA_Q8_0 ? grp : grp & 1));
+            kd[c] = *reinterpret_cast<const uint16_t*>(row + BB * grp);
+        }
+        // V: lane (grp, c16) takes key kw0 + 16 c + 4 u + grp, dims 8 c16 .. + 7
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                vr[c][u] = fa_q8<KT>(vh + (size_t)min(kw0 + 16 * c + 4 * u + grp, klast) * v_row, c16 >> 2, c16 & 3);
+        uint16_t mraw[NC][4];  // (converted where used; without a mask element 0 of q, ignored)
+        {
+            const uint16_t* mp = mask ? mask : reinterpret_cast<const uint16_t*>(q);
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) mraw[c][e] = mp[mask ? min(kw0 + 16 * c + 4 * grp + e, klast) : 0];
+        }
+        // q's block wv: head c16, dims 32 wv + 8 grp .. + 7
+        float qx[8];
+        {
+            const float* qp = q + (size_t)(hk * G + min(c16, G - 1)) * FA_D + 32 * wv + 8 * grp;
+            const float4 a = *reinterpret_cast<const float4*>(qp), b = *reinterpret_cast<const float4*>(qp + 4);
+            const float t[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) qx[e] = t[e];
+        }
+        {  // Q8_0 of the block with the rules of amv_quantize_act (ggml quantize_row_q8_0): 4 lanes of 8 elements
+            float amax = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(qx[e]));
+            amax = amv_max_x32(amv_max_x16(amax));
+            const float d = amax / 127.0f;
+            float id;
+            if (qrule == AMV_Q8_X86) id = amax != 0.0f ? 127.0f / amax : 0.0f;
+            else id = d != 0.0f ? 1.0f / d : 0.0f;
+            uint32_t qq[2] = {0u, 0u};
+            int qs = 0;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float t = qx[e] * id;
+                float qf = qrule == AMV_Q8_REF ? roundf(t) : rintf(t);
+                qf = fminf(127.0f, fmaxf(-127.0f, qf));
+                const int qi = (int)qf;
+                qs += qi;
+                qq[e >> 2] |= (uint32_t)(qi & 0xFF) << (8 * (e & 3));
+            }
+            sQ[wv][lane] = c16 < G ? make_uint2(qq[0], qq[1]) : make_uint2(0u, 0u);
+            const auto r16 = __builtin_amdgcn_permlane16_swap(qs, qs, false, false);
+            qs = (int)r16[0] + (int)r16[1];
+            const auto r32 = __builtin_amdgcn_permlane32_swap(qs, qs, false, false);
+            qs = (int)r32[0] + (int)r32[1];
+            if (grp == 0) {
+                sDq[wv][c16] = amv_h2f(amv_f2h(d));
+                sSq[wv][c16] = qs;
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < NC; ++c) sDk[wv][c][grp][c16] = amv_h2f(kd[c]);
+        __syncthreads();
+        // lane (grp, c16): keys kw0 + 16 c + 4 grp + e of head c16, in log2 units
+        float sc[NC][4];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            float t[4][4];
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) {
+                uint2 kb = kr[c][kk];
+                const uint2 qb = sQ[kk][lane];
+                fa_i4 C = {0, 0, 0, 0};
+                if constexpr (KT == FA_Q4_0) {
+                    const int sh = grp >= 2 ? 4 : 0, z = -8 * sSq[kk][c16];
+                    kb = make_uint2((kb.x >> sh) & 0x0F0F0F0Fu, (kb.y >> sh) & 0x0F0F0F0Fu);
+                    C = fa_i4{z, z, z, z};
+                }
+                C = __builtin_amdgcn_mfma_i32_16x16x32_i8((long)((uint64_t)kb.y << 32 | kb.x),
+                                                          (long)((uint64_t)qb.y << 32 | qb.x), C, 0, 0, 0);
+                const float dq = sDq[kk][c16];
+                const float4 dk4 = *reinterpret_cast<const float4*>(&sDk[wv][c][kk][4 * grp]);
+                const float dk[4] = {dk4.x, dk4.y, dk4.z, dk4.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    t[kk][e] = KT == FA_Q8_0 ? (float)C[e] * (dk[e] * dq) : ((float)C[e] * dk[e]) * dq;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float S = (t[0][e] + t[1][e]) + (t[2][e] + t[3][e]);
+                const int i = kw0 + 16 * c + 4 * grp + e;
+                const float mk = (i < n_kv) ? (mask ? amv_h2f(mraw[c][e]) : 0.0f) : -INFINITY;
+                sc[c][e] = (mk == -INFINITY) ? -INFINITY : (S * scale + mk) * AMV_LOG2E;
+            }
+        }
+        float mm = -INFINITY;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) mm = fmaxf(mm, fmaxf(fmaxf(sc[c][0], sc[c][1]), fmaxf(sc[c][2], sc[c][3])));
+        mm = amv_max_x32(amv_max_x16(mm));
+        float ll = 0.0f;
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                sc[c][e] = __builtin_amdgcn_exp2f(sc[c][e] - (mm == -INFINITY ? 0.0f : mm));
+                ll += sc[c][e];
+            }
+        ll = amv_sum_x32(amv_sum_x16(ll));
+        if (c16 < G) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sP[wv][16 * c + 4 * grp + e][c16] = sc[c][e];
+            if (grp == 0) {
+                sM[wv][c16] = mm;
+                sL[wv][c16] = ll;
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        float acc[G][8];
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[g][e] = 0.0f;
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                float vf[8];
+                // ggml dequantize_row_q8_0 / q4_0: q * d, (nibble - 8) * d
+                const float dv = amv_h2f((uint16_t)vr[c][u].d);
+                const uint32_t w[2] = {vr[c][u].b.x, vr[c][u].b.y};
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    if constexpr (KT == FA_Q8_0)
+                        vf[e] = (float)(int8_t)(w[e >> 2] >> (8 * (e & 3))) * dv;
+                    else
+                        vf[e] = ((float)((w[e >> 2] >> (8 * (e & 3) + ((c16 & 2) ? 4 : 0))) & 0xFu) - 8.0f) * dv;
+                }
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    const float p = sP[wv][16 * c + 4 * u + grp][g];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) acc[g][e] = fmaf(p, vf[e], acc[g][e]);
+                }
+            }
+        // the 4 lane groups of a wave share the wave's maximum, so their accumulators add; the sum is taken below
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            float4* dst = reinterpret_cast<float4*>(sbuf + ((wv * 4 + grp) * G + g) * FA_D + d8);
+            dst[0] = make_float4(acc[g][0], acc[g][1], acc[g][2], acc[g][3]);
+            dst[1] = make_float4(acc[g][4], acc[g][5], acc[g][6], acc[g][7]);
+        }
+        __syncthreads();
+        // merge the 4 wave partials of this workgroup
+        for (int e = tid; e < G * FA_D; e += 256) {
+            const int g = e / FA_D, d = e % FA_D;
+            const float M = fmaxf(fmaxf(sM[0][g], sM[1][g]), fmaxf(sM[2][g], sM[3][g]));
+            float a = 0.0f, L = 0.0f;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const float f = (sM[w][g] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(sM[w][g] - M);
+                const float* sa = sbuf + ((w * 4) * G + g) * FA_D + d;
+                const float aw = (sa[0] + sa[G * FA_D]) + (sa[2 * G * FA_D] + sa[3 * G * FA_D]);
+                a = fmaf(aw, f, a);
+                L = fmaf(sL[w][g], f, L);
+            }
+            float* pp = part + ((size_t)(hk * G + g) * n_split + split) * FA_PS;
+            if constexpr (FUSED) {  // handed over to the merging workgroup within the launch
+                amv_store_coh(pp + 4 + d, a);
+                if (d == 0) {
+                    amv_store_coh(pp, M);
+                    amv_store_coh(pp + 1, L);
+                }
+            } else {
+                pp[4 + d] = a;
+                if (d == 0) {
+                    pp[0] = M;
+                    pp[1] = L;
+                }
+            }
+        }
+    }
+    if constexpr (FUSED) {
+        if (!amv_arrive_last(counters + AMV_CNT_STRIDE * hk, gridDim.y)) return;
+        amv_acquire();
+        fa_merge<G>(part, n_split, ns, hk, out, act, sbuf);
+    }
+}
+
 // The merge as its own launch: one workgroup per GH heads (GH = 1, or 2 for Q8_K output blocks of 256), the key
 // count from n_kv_dev when given, as in k_fa_split.
 template <int GH>
@@ -717,24 +859,34 @@ static void fa_launch_split(int G, int kpw, dim3 grid, hipStream_t st, const flo
                             int64_t k_row, int64_t k_head, int64_t v_row, int64_t v_head, int n_split, float scale,
                             int rule, unsigned int* counters, float* out, const AmvActOut& act) {
 #define FA_LAUNCH(GG, KK)                                                                                              \
-    hipLaunchKernelGGL((k_fa_split<GG, KK, FUSED, KT>), grid, dim3(256), 0, st, q, kk, vv, mm, part, n_kv, n_kv_dev, \
-                       k_row, k_head, v_row, v_head, n_split, scale, rule, counters, out, act)
+    hipLaunchKernelGGL((k_fa_split<GG, KK, FUSED>), grid, dim3(256), 0, st, q, kk, vv, mm, part, n_kv, n_kv_dev, \
+                       k_row, k_head, v_row, v_head, n_split, scale, counters, out, act)
 #define FA_MF(GG, KK)                                                                                            \
     hipLaunchKernelGGL((k_fa_split_mf<GG, FUSED, KK>), dim3(grid.y, grid.x), dim3(256), 0, st, q, kk, vv, mm, part, \
                        n_kv, n_kv_dev, k_row, k_head, v_row, v_head, n_split, scale, counters, out, act)
-#define FA_G(GG)                                  \
-    if (KT == FA_F16 && kpw == 16) FA_MF(GG, 16);  \
-    else if (KT == FA_F16) FA_MF(GG, 32);          \
-    else if (kpw == 16) FA_LAUNCH(GG, 16);         \
-    else FA_LAUNCH(GG, 32)
+#define FA_MQ(GG, KK)                                                                                                  \
+    hipLaunchKernelGGL((k_fa_split_mq<GG, FUSED, KK, KT>), dim3(grid.y, grid.x), dim3(256), 0, st, q, kk, vv, mm, part, \
+                       n_kv, n_kv_dev, k_row, k_head, v_row, v_head, n_split, scale, rule, counters, out, act)
+#define FA_G(GG)                                                              \
+    if constexpr (KT == FA_F16) {                                             \
+        if (kpw == 16) FA_MF(GG, 16);                                         \
+        else FA_MF(GG, 32);                                                   \
+    } else if constexpr (KT == FA_F32) {                                      \
+        if (kpw == 16) FA_LAUNCH(GG, 16);                                     \
+        else FA_LAUNCH(GG, 32);                                               \
+    } else {                                                                  \
+        if (kpw == 16) FA_MQ(GG, 16);                                         \
+        else FA_MQ(GG, 32);                                                   \
+    }
     switch (G) {
-    case 1: FA_G(1); break;
-    case 2: FA_G(2); break;
-    case 4: FA_G(4); break;
-    default: FA_G(8); break;
+    case 1: FA_G(1) break;
+    case 2: FA_G(2) break;
+    case 4: FA_G(4) break;
+    default: FA_G(8) break;
     }
 #undef FA_G
 #undef FA_MF
+#undef FA_MQ
 #undef FA_LAUNCH
 }
 
