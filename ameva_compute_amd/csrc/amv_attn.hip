@@ -544,7 +544,7 @@ __global__ __launch_bounds__(256) void k_fa_split_mf(const float* __restrict__ q
 // vec_dot_q8_0_q8_0 isum * (d_k * d_q), vec_dot_q4_0_q8_0 (isum * d_k) * d_q. Each of the 4 waves quantizes one of q's
 // 4 blocks for all. What bounded this before (8 dot4 per lane, then per key and head two LDS round trips to add a block's
 // lanes, a 16-lane sum, and q quantized by every lane group) was that work and not the cache's bytes: Q8_0, 8192 keys, 8
-// KV heads of 4 heads with the merge: 19.5 us, now 14.4 ( the rows are 17.8 MB, 3.5 us at the rate of a
+// KV heads of 4 heads with the merge: 19.5 us, now 14.4 (the rows are 17.8 MB, 3.5 us at the rate of a
 // copy). Rows are only 2-byte aligned: 8-byte loads at that alignment, where halfwords were read one by one. V: 16 lanes
 // per row, 8 dims per lane.
 typedef uint2 __attribute__((aligned(2))) fa_u2a;

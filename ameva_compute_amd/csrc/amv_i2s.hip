@@ -284,7 +284,7 @@ __global__ __launch_bounds__(256) void k_i2s_mmq_p(const uint8_t* __restrict__ w
     }
 }
 
-float* amv_splitk_workspace(size_t bytes, hipStream_t st, bool optional = false);
+float* amv_splitk_workspace(size_t bytes, hipStream_t st);
 
 extern "C" int64_t amv_i2s_act_bytes(int64_t m, int64_t k) { return (m < 0 || k < 0) ? -1 : m * k + m * 8; }
 

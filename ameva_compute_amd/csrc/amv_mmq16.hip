@@ -258,8 +258,7 @@ std::map<int, float*> g_splitk_ws;  // device -> the workspace (AMV_SPLITK_WS_BY
 // 2048 x (128 x 128) x 4 = 128 MiB. The workspace never grows, so a captured graph's pointer stays valid. Under
 // stream capture no allocation is possible: a call that splits k before any uncaptured call did fails (it never
 // falls back to an unsplit launch, whose f32 summation order would differ from the same call outside capture).
-// optional: a caller that can do without gets nullptr and no error message.
-float* amv_splitk_workspace(size_t bytes, hipStream_t st, bool optional = false) {
+float* amv_splitk_workspace(size_t bytes, hipStream_t st) {
     if (bytes > AMV_SPLITK_WS_BYTES) {
         amv_set_error("split-k workspace: %zu bytes asked, %zu available", bytes, (size_t)AMV_SPLITK_WS_BYTES);
         return nullptr;
@@ -275,7 +274,6 @@ float* amv_splitk_workspace(size_t bytes, hipStream_t st, bool optional = false)
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
         (void)hipGetLastError();
-        if (optional) return nullptr;
         amv_set_error("split-k workspace: first needed under stream capture; run a batched MUL_MAT that splits k "
                       "(k >= 6144 with fewer than 1024 tiles) once before capturing");
         return nullptr;

@@ -282,7 +282,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // ---------------------------------------------------------------------------------------------------------------
 // host
 // ---------------------------------------------------------------------------------------------------------------
-float* amv_splitk_workspace(size_t bytes, hipStream_t st, bool optional = false);
+float* amv_splitk_workspace(size_t bytes, hipStream_t st);
 int amv_splitk_count(int64_t tiles, int steps);
 void amv_splitk_reduce(const float* part, int S, int64_t zstride, int64_t m, int64_t n, float* dst, int64_t ldd,
                        hipStream_t st, const float* add = nullptr);

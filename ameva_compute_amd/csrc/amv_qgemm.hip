@@ -665,7 +665,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // host
 // ---------------------------------------------------------------------------------------------------------------
 // split of k shared with the f16 kernels (amv_mmq16.hip): workspace per device and the in-order partial sum
-float* amv_splitk_workspace(size_t bytes, hipStream_t st, bool optional = false);
+float* amv_splitk_workspace(size_t bytes, hipStream_t st);
 int amv_splitk_count(int64_t tiles, int steps);
 void amv_splitk_reduce(const float* part, int S, int64_t zstride, int64_t m, int64_t n, float* dst, int64_t ldd,
                        hipStream_t st, const float* add = nullptr);
@@ -691,18 +691,10 @@ static int qg_plan(QgPlan& p, int bm, int bn, int64_t n_rows, int64_t m, int64_t
         p.S = (n_blk + p.per - 1) / p.per;
     }
     if (p.S > 1) {
-        // Never unsplit above 64 tokens: the summation order would change. Up to 64 tokens a capture that runs before any
-        // such call has no workspace and must not fail: it keeps k whole.
-        float* ws = amv_splitk_workspace((size_t)p.S * m * n_rows * 4, st, m <= 64);
-        if (!ws && m > 64) return AMV_ERR_HIP;
-        if (ws) {
-            p.out = ws;
-            p.ldo = n_rows;
-            p.zstride = m * n_rows;
-        } else {
-            p.S = 1;
-            p.per = n_blk;
-        }
+        p.out = amv_splitk_workspace((size_t)p.S * m * n_rows * 4, st);
+        if (!p.out) return AMV_ERR_HIP;  // never unsplit: the summation order would change
+        p.ldo = n_rows;
+        p.zstride = m * n_rows;
     }
     return AMV_OK;
 }
@@ -787,7 +779,9 @@ static int qg_q6k(const QgCall& c) {  // ql [n][nsb][128] | qh [n][nsb][64] | sc
 
 int amv_qgemm(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int64_t m, float* dst, int64_t ldd,
               int32_t* sums, hipStream_t st, const float* add) {
-    const QgCall c{w, n_rows, k, act, m, dst, ldd, sums, st, add, !sums};
+    // Up to 64 tokens of Q4_0 / Q8_0 / Q4_K k stays whole: calls this small are made on several streams, which the split's
+    // workspace does not allow at the same time.
+    const QgCall c{w, n_rows, k, act, m, dst, ldd, sums, st, add, !sums && (m > 64 || wtype == AMV_T_Q6_K)};
     const auto tiles = [&](int bm, int bn) { return ((m + bm - 1) / bm) * ((n_rows + bn - 1) / bn); };
     const auto wgs = [&](int bm, int bn) {  // workgroups with the split of k
         return tiles(bm, bn) * (c.split ? amv_splitk_count(tiles(bm, bn), (int)(k / 64)) : 1);
@@ -798,7 +792,7 @@ int amv_qgemm(int wtype, const void* w, int64_t n_rows, int64_t k, const void* a
     // m <= 64 on 16 x 16 tiles):
     //   rows x k, tokens     Q4_K           Q8_0           Q4_0
     //   14336 x 4096,  48    18 (48)        22 (111)       22 (116)
-    //   4096 x 14336,  48    22 (173)       24 (373)       24 (395)
+    //   4096 x 14336,  48    48 (173)       61 (373)       63 (395)     (split over workgroups 22, 24, 24)
     //   4096 x 4096,   96    16 (38)        19 (39)        21 (42)
     //   14336 x 4096, 128    27 (46)        35 (51)        33 (52)
     //   4096 x 4096,  512    29 (47)        39 (56)        39 (56)
