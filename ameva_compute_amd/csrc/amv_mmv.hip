@@ -1447,12 +1447,24 @@ extern "C" int amv_mul_mat_vec_ep(int wtype, const void* w, int64_t n_rows, int6
     return amv_check_launch("amv_mul_mat_vec_ep");
 }
 
+// Columns 3..7 of Q4_0, Q8_0 and Q6_K: the streamed small-batch kernels read the weights once for all columns (the same
+// block integers; Q4_K's read activations of another layout). Measured (us, 28672 x 4096 / 4096 x 14336, a launch per
+// column against one): Q4_0 2 columns 20 / 14 against 21 / 12, 3 30 / 20 against 21 / 12, 7 67 / 45 against 23 / 14; Q8_0
+// 3 56 / 33 against 35 / 18, 7 131 / 76 against 37 / 20; Q6_K 3 50 / 30 against 30 / 16, 7 114 / 67 against 31 / 17. Rows
+// that the streamed kernel does not take (k % 128 != 0, Q4_0 with an odd row count) from 5 columns: Q4_0 1025 x 4096
+// 4 9.2 against 10.9, 5 11.4 against 11.1, 7 16.0 against 11.7.
+static bool mmv_columns_batched(int wtype, int64_t n_rows, int64_t k, int64_t m) {
+    if (m < 3 || m > 7 || wtype == AMV_T_Q4_K) return false;
+    return m >= 5 || wtype == AMV_T_Q6_K || (k % 128 == 0 && (wtype == AMV_T_Q8_0 || n_rows % 2 == 0));
+}
+
 extern "C" int amv_mul_mat_vec(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int64_t m,
                                float* dst, int64_t ldd, void* stream) {
     int rc = check_common("amv_mul_mat_vec", wtype, w, n_rows, k, act, m);
     if (rc) return rc;
     AMV_REQUIRE(dst, "amv_mul_mat_vec: null dst");
     AMV_REQUIRE(ldd >= n_rows, "amv_mul_mat_vec: ldd %lld < n_rows %lld", (long long)ldd, (long long)n_rows);
+    if (mmv_columns_batched(wtype, n_rows, k, m)) return amv_mul_mat_q(wtype, w, n_rows, k, act, m, dst, ldd, stream);
     hipStream_t st = amv_stream(stream);
     for (int64_t c = 0; c < m; ++c) {
         MmvArgs a{wtype, (const uint8_t*)w, (int)n_rows, (int)k, nullptr, nullptr, nullptr, dst + c * ldd, nullptr,

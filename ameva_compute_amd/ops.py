@@ -71,10 +71,12 @@ def act_type(wtype: int, m: int = 1, exact: bool | None = None) -> int:
 
 def gemm_act_type(wtype: int, m: int) -> int:
     """The activation layout the fastest MUL_MAT of m tokens in MMQ_FORM's arithmetic takes: act_type's, with the digits'
-    scratch for Q4_0 above MMQ16_MIN_M tokens in the exact form (the 6-bit matrix instruction), and without the f16
-    copies for Q4_K above QGEMM_MIN_M tokens (the tiled kernel reads the plain prefix)."""
+    scratch for Q4_0 above MMQ16_MIN_M tokens in the exact form (the 6-bit matrix instruction), and for Q4_K without the
+    f16 copies above QGEMM_MIN_M tokens (the tiled kernel reads the plain prefix) and with them from Q4_K_SB_MIN_M."""
     if wtype == Q4_K and QGEMM_MIN_M < m <= MMQ16_MIN_M:
         return Q8_K
+    if wtype == Q4_K and Q4_K_SB_MIN_M <= m < MMQ_MIN_M:
+        return Q8_K_MMA
     if wtype == Q4_0 and m > MMQ16_MIN_M and MMQ_FORM == "exact":
         return Q8_0_F6
     return act_type(wtype, m)
@@ -156,6 +158,10 @@ def quantize_q4_0(x: torch.Tensor) -> torch.Tensor:
 
 # batch size from which MUL_MAT runs the int8-MFMA kernel (AMEVA_QGEMM_MIN_M of the reference, ggml-ameva.cpp:2486)
 MMQ_MIN_M = 8
+# Q4_K of fewer than MMQ_MIN_M tokens with Q8_K_MMA activations: from here one batched launch beats a GEMV per token (us,
+# 28672 x 4096 / 4096 x 14336: 2 tokens 24 / 15 against 26 / 16, 3 36 / 22 against 26 / 16, 7 78 / 50 against 28 / 18); the
+# types whose batched kernels read the plain layout switch in amv_mul_mat_vec
+Q4_K_SB_MIN_M = 3
 QGEMM_MIN_M = 32  # above this many tokens the exact tiled kernels run (amv_mmq.hip QGEMM_MIN_M)
 MMQ16_MIN_M = 64  # above this many tokens the scaled form and act_type's plain Q4_K layout (amv_mmq.hip MMQ16_MIN_M)
 MMQ_TYPES = (Q4_0, Q8_0, Q4_K, Q6_K)  # Q4_K of MMQ_MIN_M..MMQ16_MIN_M tokens: the activations must be Q8_K_MMA
@@ -178,13 +184,15 @@ def mul_mat_q_add(w: QWeight, act: torch.Tensor, m: int, add: torch.Tensor, act_
 def mul_mat_q(w: QWeight, act: torch.Tensor, m: int, out: torch.Tensor | None = None,
               kernel: str = "auto", act_t: int | None = None) -> torch.Tensor:
     """dst [m, n_rows] f32 from already quantized activations (amv_quantize_act layout of m rows).
-    kernel: "auto" (the reference's routing: MFMA GEMM for m >= MMQ_MIN_M where the type has one), "mmv", "mmq".
+    kernel: "auto" (the reference's routing: MFMA GEMM for m >= MMQ_MIN_M where the type has one; Q4_K with act_t
+    Q8_K_MMA from Q4_K_SB_MIN_M), "mmv", "mmq".
     Q4_K on "mmq" needs Q8_K_MMA activations up to MMQ16_MIN_M tokens. act_t: the activation layout (the DEQ
     layouts have the MMA sizes, so they must be named; None: told apart by size, i.e. plain or MMA)."""
     _need_gpu(act, "mul_mat_q")
     if out is None:
         out = torch.empty((m, w.n_rows), dtype=torch.float32, device=act.device)
-    use_mmq = kernel == "mmq" or (kernel == "auto" and m >= MMQ_MIN_M and w.type in MMQ_TYPES)
+    use_mmq = kernel == "mmq" or (kernel == "auto" and w.type in MMQ_TYPES and
+                                  (m >= MMQ_MIN_M or (m >= Q4_K_SB_MIN_M and w.type == Q4_K and act_t == Q8_K_MMA)))
     if use_mmq:
         at = act_layout(w.type, act, m, w.k) if act_t is None else act_t
         check(lib().amv_mul_mat_q_act(w.type, w.data.data_ptr(), w.n_rows, w.k, act.data_ptr(), at, m,
