@@ -16,26 +16,54 @@
 // q = clamp(roundf(x * scale), -127, 127) (round half away from zero), dequant = 1 / scale, plus sum(q).
 // Output layout: q int8 [m][k] | {f32 dequant, i32 sum q} [m].
 // ---------------------------------------------------------------------------------------------------------------
+// Bound by its chain of loads, not by bytes: a row's first 1024 U elements go out as U 16-byte loads at once and stay in
+// registers for the second pass (before: one 4-byte load per step, twice; rows of 6912: 8.1 us, of 2560: 4.3). VEC: rows
+// 16-byte aligned.
+template <int U, bool VEC>
 __global__ __launch_bounds__(256) void k_i2s_quant(const float* __restrict__ x, int k, int8_t* __restrict__ q,
                                                   int2* __restrict__ meta) {
     __shared__ float smax[4];
     __shared__ int ssum[4];
     const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const float* xr = x + (size_t)row * k;
+    const int n4 = k >> 2;  // k % 128 == 0
     float amax = 1e-7f;
-    for (int i = tid; i < k; i += 256) amax = fmaxf(amax, fabsf(xr[i]));
+    float4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {  // (a select of the value, not a branch around the load: the loads go out together)
+        const int i = tid + 256 * u;
+        v[u] = VEC ? *reinterpret_cast<const float4*>(xr + 4 * min(i, n4 - 1))
+                   : make_float4(xr[4 * min(i, n4 - 1)], xr[4 * min(i, n4 - 1) + 1], xr[4 * min(i, n4 - 1) + 2],
+                                 xr[4 * min(i, n4 - 1) + 3]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)  // (a lane past the row holds its last elements again)
+        amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v[u].x), fabsf(v[u].y)), fmaxf(fabsf(v[u].z), fabsf(v[u].w))));
+    for (int i = tid + 256 * U; i < n4; i += 256)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) amax = fmaxf(amax, fabsf(xr[4 * i + e]));
     amax = amv_wave_max_u(amax);
     if (lane == 0) smax[w] = amax;
     __syncthreads();
     amax = fmaxf(fmaxf(smax[0], smax[1]), fmaxf(smax[2], smax[3]));
     const float scale = 127.0f / amax;
     int s = 0;
-    for (int i = tid; i < k; i += 256) {
-        float v = roundf(xr[i] * scale);
-        v = fminf(127.0f, fmaxf(-127.0f, v));
-        q[(size_t)row * k + i] = (int8_t)(int)v;
-        s += (int)v;
-    }
+    int* qr = reinterpret_cast<int*>(q + (size_t)row * k);
+    const auto quant = [&](int i, const float4& f) {
+        const float t[4] = {f.x, f.y, f.z, f.w};
+        int b[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            b[e] = (int)fminf(127.0f, fmaxf(-127.0f, roundf(t[e] * scale)));
+            s += b[e];
+        }
+        qr[i] = amv_pack4(b);
+    };
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (tid + 256 * u < n4) quant(tid + 256 * u, v[u]);
+    for (int i = tid + 256 * U; i < n4; i += 256)
+        quant(i, make_float4(xr[4 * i], xr[4 * i + 1], xr[4 * i + 2], xr[4 * i + 3]));
     s = amv_wave_sum_i_u(s);
     if (lane == 0) ssum[w] = s;
     __syncthreads();
@@ -119,7 +147,7 @@ __global__ __launch_bounds__(256) void k_i2s_gemv(const uint4* __restrict__ w, i
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// Batched (m >= 8 tokens) I2_S MUL_MAT on int8 MFMA. The activation scale is per token over the whole row, so the
+// Batched (m >= I2S_MMQ_MIN_M tokens) I2_S MUL_MAT on int8 MFMA. The activation scale is per token over the whole row, so the
 // ternary dot stays integer across all of k: v_mfma_i32_32x32x32_i8 (the full-rate int8 shape of gfx950) accumulates
 // sum_k code * q in its int32 accumulator from the first block to the last (codes 0..3 are valid signed bytes), and
 // sum q is subtracted once.
@@ -295,12 +323,19 @@ extern "C" int amv_i2s_quantize_act(const float* x, int64_t m, int64_t k, void* 
     AMV_REQUIRE(k % 128 == 0, "amv_i2s_quantize_act: k %% 128 != 0");
     int8_t* q = (int8_t*)act;
     int2* meta = (int2*)((uint8_t*)act + m * k);
-    hipLaunchKernelGGL(k_i2s_quant, dim3((unsigned)m), dim3(256), 0, amv_stream(stream), x, (int)k, q, meta);
+    const bool vec = ((uintptr_t)x & 15) == 0;
+#define I2S_Q(U, V) hipLaunchKernelGGL((k_i2s_quant<U, V>), dim3((unsigned)m), dim3(256), 0, amv_stream(stream), x, (int)k, q, meta)
+    if (!vec) I2S_Q(2, false);
+    else if (k <= 3072) I2S_Q(3, true);
+    else I2S_Q(8, true);
+#undef I2S_Q
     return amv_check_launch("amv_i2s_quantize_act");
 }
 
-// batch from which the MFMA kernel runs (as the Q4_0 / Q8_0 MUL_MAT, AMEVA_QGEMM_MIN_M = 8)
-#define I2S_MMQ_MIN_M 8
+// Tokens from which the MFMA kernel runs; below, a GEMV per token. 4 to 7 tokens keep k whole (no workspace: such calls
+// could always run on several streams at a time). Measured (us, GEMVs against one launch): 2560 x 6912 3 tokens 9.7 / 11,
+// 4 12.7 / 11.3, 7 21.5 / 11.9; 6912 x 2560 4 12.1 / 6.7, 7 19.8 / 7.3; 640 x 2560 3 6.2 / 6.6, 4 8 / 6.6, 7 13.5 / 7.1.
+#define I2S_MMQ_MIN_M 4
 // The batched launch (k_i2s_mmq_p): 64 x 64 tiles, k split over S workgroups when the tiles alone leave CUs idle (about
 // one workgroup per CU: the four-block prefetch keeps a wave's 250 VGPRs, one wave per SIMD), the partials added by
 // k_i2s_split_sum. The integers do not depend on S (exact in any order): without the workspace (first needed under
@@ -318,6 +353,10 @@ static void i2s_mmq_p(const void* w, int64_t n_rows, int kb, const void* act, in
     int kb_per = (kb + S - 1) / S;
     S = (kb + kb_per - 1) / kb_per;
     int32_t* part = nullptr;
+    if (m < 8) {  // no workspace
+        S = 1;
+        kb_per = kb;
+    }
     if (S > 1) {
         const size_t bytes = (size_t)S * m * n_rows * 4;
         part = bytes <= AMV_SPLITK_WS_BYTES ? reinterpret_cast<int32_t*>(amv_splitk_workspace(bytes, st)) : nullptr;
