@@ -1123,6 +1123,18 @@ extern "C" int amv_mul_mat_q_act(int wtype, const void* w, int64_t n_rows, int64
     return mmq_act_impl("amv_mul_mat_q_act", wtype, w, n_rows, k, act, act_type, m, dst, ldd, nullptr, stream);
 }
 
+// the two calls of a MUL_MAT on f32 activations in one, for callers that pay for each call into the library
+extern "C" int amv_mul_mat_f32(int wtype, const void* w, int64_t n_rows, int64_t k, const float* x, int64_t m,
+                               int act_type, int rule, int batched, void* act, float* dst, int64_t ldd, void* stream) {
+    AMV_REQUIRE(act, "amv_mul_mat_f32: null act");
+    AMV_REQUIRE(batched || act_type == AMV_T_Q8_0 || act_type == AMV_T_Q8_K,
+                "amv_mul_mat_f32: activation type %d needs the batched kernels", act_type);
+    const int rc = amv_quantize_act(act_type, x, m, k, rule, nullptr, act, stream);
+    if (rc) return rc;
+    return batched ? amv_mul_mat_q_act(wtype, w, n_rows, k, act, act_type, m, dst, ldd, stream)
+                   : amv_mul_mat_vec(wtype, w, n_rows, k, act, m, dst, ldd, stream);
+}
+
 extern "C" int amv_mul_mat_q_act_add(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act,
                                      int act_type, int64_t m, float* dst, int64_t ldd, const float* add, void* stream) {
     AMV_REQUIRE(dst && add, "amv_mul_mat_q_act_add: null dst or add");

@@ -8,6 +8,7 @@ there is no CPU path.
 """
 from __future__ import annotations
 
+import functools
 import os
 
 import torch
@@ -22,8 +23,17 @@ Q8_X86, Q8_ARM, Q8_REF = 0, 1, 2
 BLOCK = {Q4_0: (32, 18), Q8_0: (32, 34), Q4_K: (256, 144), Q6_K: (256, 210), Q8_K: (256, 292)}
 
 
+# the current stream's handle without building a torch.cuda.Stream object
+_raw_stream, _device = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
+
+
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_device())
+
+
+@functools.lru_cache(maxsize=4096)
+def _act_bytes(atype: int, m: int, k: int) -> int:
+    return lib().amv_act_bytes(atype, m, k)
 
 
 def _ptr(t: torch.Tensor | None):
@@ -135,7 +145,7 @@ def quantize_act(x: torch.Tensor, atype: int = Q8_0, rule: int = Q8_X86, ggml: b
         raise ValueError("quantize_act: f32 input expected")
     x2 = x.reshape(-1, x.shape[-1])
     m, k = x2.shape
-    n = lib().amv_act_bytes(atype, m, k)
+    n = _act_bytes(atype, m, k)
     if n < 0:
         raise ValueError(f"quantize_act: type {atype} cannot hold rows of {k}")
     act = torch.empty(n, dtype=torch.uint8, device=x.device)
@@ -181,6 +191,10 @@ def mul_mat_q_add(w: QWeight, act: torch.Tensor, m: int, add: torch.Tensor, act_
     return out
 
 
+def _batched(wtype: int, m: int, act_t: int | None) -> bool:
+    return wtype in MMQ_TYPES and (m >= MMQ_MIN_M or (m >= Q4_K_SB_MIN_M and wtype == Q4_K and act_t == Q8_K_MMA))
+
+
 def mul_mat_q(w: QWeight, act: torch.Tensor, m: int, out: torch.Tensor | None = None,
               kernel: str = "auto", act_t: int | None = None) -> torch.Tensor:
     """dst [m, n_rows] f32 from already quantized activations (amv_quantize_act layout of m rows).
@@ -191,9 +205,7 @@ def mul_mat_q(w: QWeight, act: torch.Tensor, m: int, out: torch.Tensor | None = 
     _need_gpu(act, "mul_mat_q")
     if out is None:
         out = torch.empty((m, w.n_rows), dtype=torch.float32, device=act.device)
-    use_mmq = kernel == "mmq" or (kernel == "auto" and w.type in MMQ_TYPES and
-                                  (m >= MMQ_MIN_M or (m >= Q4_K_SB_MIN_M and w.type == Q4_K and act_t == Q8_K_MMA)))
-    if use_mmq:
+    if kernel == "mmq" or (kernel == "auto" and _batched(w.type, m, act_t)):
         at = act_layout(w.type, act, m, w.k) if act_t is None else act_t
         check(lib().amv_mul_mat_q_act(w.type, w.data.data_ptr(), w.n_rows, w.k, act.data_ptr(), at, m,
                                       out.data_ptr(), w.n_rows, _stream()), "amv_mul_mat_q_act")
@@ -290,11 +302,23 @@ def gemv_rope_kv(w: QWeight, act: torch.Tensor, n_head: int, n_head_kv: int, pos
 def mul_mat(w: QWeight, x: torch.Tensor, rule: int = Q8_X86) -> torch.Tensor:
     """ggml_mul_mat(src0 = w, src1 = x): x f32 [m, k] -> [m, n_rows]; activations quantized to vec_dot_type."""
     x2 = x.reshape(-1, x.shape[-1])
-    if x2.shape[1] != w.k:
-        raise ValueError(f"mul_mat: k mismatch {x2.shape[1]} != {w.k}")
-    at = gemm_act_type(w.type, x2.shape[0])
-    act, _ = quantize_act(x2, at, rule)
-    return mul_mat_q(w, act, x2.shape[0], act_t=at)
+    m, k = x2.shape
+    if k != w.k:
+        raise ValueError(f"mul_mat: k mismatch {k} != {w.k}")
+    _need_gpu(x2, "quantize_act")
+    if x2.dtype != torch.float32:
+        raise ValueError("quantize_act: f32 input expected")
+    at = gemm_act_type(w.type, m)
+    n = _act_bytes(at, m, k)
+    if n < 0:
+        raise ValueError(f"quantize_act: type {at} cannot hold rows of {k}")
+    act = torch.empty(n, dtype=torch.uint8, device=x2.device)
+    out = torch.empty((m, w.n_rows), dtype=torch.float32, device=x2.device)
+    # one call for both launches: a token's MUL_MAT is bound by the host's path to them (4096 x 4096 Q4_0: 20.3 us with two
+    # calls, two size queries and two stream objects, 12.3 with this one; the kernels take 5)
+    check(lib().amv_mul_mat_f32(w.type, w.data.data_ptr(), w.n_rows, k, x2.data_ptr(), m, at, rule,
+                                _batched(w.type, m, at), act.data_ptr(), out.data_ptr(), w.n_rows, _stream()), "amv_mul_mat")
+    return out
 
 
 def block_sums(w: QWeight, act: torch.Tensor, m: int, kernel: str = "mmv") -> torch.Tensor:
@@ -323,12 +347,17 @@ def quantize_k(x: torch.Tensor, wtype: int) -> torch.Tensor:
 
 
 # ------------------------------------------------------------------------------------------------ BitNet I2_S
+@functools.lru_cache(maxsize=4096)
+def _i2s_act_bytes(m: int, k: int) -> int:
+    return lib().amv_i2s_act_bytes(m, k)
+
+
 def i2s_quantize_act(x: torch.Tensor) -> torch.Tensor:
     """quantize_activation_int8 per row of x f32 [m, k] -> activation buffer (int8 q | {dequant, sum q} per row)."""
     _need_gpu(x, "i2s_quantize_act")
     x2 = x.reshape(-1, x.shape[-1])
     m, k = x2.shape
-    act = torch.empty(lib().amv_i2s_act_bytes(m, k), dtype=torch.uint8, device=x.device)
+    act = torch.empty(_i2s_act_bytes(m, k), dtype=torch.uint8, device=x.device)
     check(lib().amv_i2s_quantize_act(x2.data_ptr(), m, k, act.data_ptr(), _stream()), "amv_i2s_quantize_act")
     return act
 

@@ -235,6 +235,11 @@ int amv_mul_mat_q_block_sums(int wtype, const void* w, int64_t n_rows, int64_t k
  * activations' f16 q_a d_a and the matrix cores accumulate across all of k (no per-block epilogue; within ~3e-4
  * relative L2 of the exact form). 8..64 tokens run the small-batch kernels (Q4_K on the MMA layout's f16 copies).
  * Block sums need a plain or MMA layout. */
+/* MUL_MAT of f32 activations x [m][k] in one call: amv_quantize_act(act_type, x, m, k, rule, NULL, act) and the product,
+ * amv_mul_mat_q_act with batched != 0, else amv_mul_mat_vec (act_type then Q8_0 or Q8_K, plain). act: amv_act_bytes(act_type,
+ * m, k) bytes, which hold the quantized activations afterwards. */
+int amv_mul_mat_f32(int wtype, const void* w, int64_t n_rows, int64_t k, const float* x, int64_t m, int act_type, int rule,
+                    int batched, void* act, float* dst, int64_t ldd, void* stream);
 int amv_mul_mat_q_act(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int act_type, int64_t m,
                       float* dst, int64_t ldd, void* stream);
 int amv_mul_mat_q_act_block_sums(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int act_type,
