@@ -181,16 +181,20 @@ class LlamaLayer:
         check(L.amv_binary(0, P(self.down), P(self.x1), P(out), 1, H, 1, st), "residual 2")
 
     def _prefill_buffers(self, n_tok: int) -> dict:
-        """Per-token-count buffers of prefill (allocated on first use; a captured graph must see them allocated)."""
-        bufs = getattr(self, "_pf", None)
-        if bufs is not None and bufs["n"] >= n_tok and bufs["at"] == ops.gemm_act_type(self.wqkv.type, n_tok):
-            return bufs
+        """Per-token-count buffers of prefill (allocated on first use; a captured graph must see them allocated). A set
+        per activation layout is held, so that a captured graph keeps its own through prompts of another layout."""
+        bufs, at = getattr(self, "_pf", None), ops.gemm_act_type(self.wqkv.type, n_tok)
+        sets = self.__dict__.setdefault("_pf_sets", {})
+        if bufs is not None:
+            sets[bufs["at"]] = bufs
+        if at in sets and sets[at]["n"] >= n_tok:
+            self._pf = sets[at]
+            return self._pf
         dev = self.attn_norm.device
         f32 = dict(dtype=torch.float32, device=dev)
         u8 = dict(dtype=torch.uint8, device=dev)
         L = lib()
         H, FF = self.H, self.FF
-        at = ops.gemm_act_type(self.wqkv.type, n_tok)
         bufs = {"n": n_tok, "at": at,
                 "t_o": torch.empty((n_tok, H), **f32), "qkv": torch.empty((n_tok, self.wqkv.n_rows), **f32),
                 "att": torch.empty((n_tok, H), **f32),
@@ -203,7 +207,7 @@ class LlamaLayer:
                 "h": torch.empty((n_tok, FF), **f32) if at not in (ops.Q8_0, ops.Q8_0_F6, ops.Q8_K) else None,
                 "pos": torch.zeros(n_tok, dtype=torch.int32, device=dev),
                 "idx": torch.zeros(n_tok, dtype=torch.int64, device=dev)}
-        self._pf = bufs
+        self._pf = sets[at] = bufs
         return bufs
 
     def set_prefill_position(self, pos0: int, n_tok: int) -> None:
@@ -217,7 +221,7 @@ class LlamaLayer:
     def prefill(self, x: torch.Tensor, out: torch.Tensor) -> None:
         """A prompt chunk through the layer: x f32 [n_tok, H] at positions set_prefill_position(pos0, n_tok) ->
         out f32 [n_tok, H]; writes the chunk's K/V rows into the cache and attends causally over keys
-        0 .. pos0 + t. The MUL_MATs run on the int8 MFMA kernel (n_tok >= 8, the reference's crossover) and the
+        0 .. pos0 + t. The MUL_MATs run on the matrix cores (n_tok >= 8, the reference's crossover, or where a few tokens gain) and the
         attention on the f16 MFMA prefill kernel; the residual ADDs in the epilogues of the o and down GEMMs:
         10 launches (13 where the activation layout is an extended one, whose quantization is a launch of its own)."""
         L, st = lib(), torch.cuda.current_stream().cuda_stream
@@ -226,7 +230,7 @@ class LlamaLayer:
         H, kv, D, FF = self.H, self.kv, self.D, self.FF
         P = lambda t: t.data_ptr()  # noqa: E731
         at = b["at"]
-        if n >= ops.MMQ_MIN_M and self.wqkv.type in ops.MMQ_TYPES:
+        if ops._batched(self.wqkv.type, n, at):
             def mm(wt, w, nr, k, act, m, dst, ldd, s):
                 return L.amv_mul_mat_q_act(wt, w, nr, k, act, at, m, dst, ldd, s)
 

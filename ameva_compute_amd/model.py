@@ -86,11 +86,9 @@ class LlamaModel:
         if self._pf is None or self._pf[0].shape[0] < n:
             f32 = dict(dtype=torch.float32, device=tokens.device)
             self._pf = (torch.empty((n, self.H), **f32), torch.empty((n, self.H), **f32))
-            shared = None
-            for lay in self.layers:  # one set of prompt buffers for all layers
-                if shared is None:
-                    shared = lay._prefill_buffers(n)
-                lay._pf = shared
+        shared = self.layers[0]._prefill_buffers(n)  # one set of prompt buffers (positions included) for all layers
+        for lay in self.layers:
+            lay._pf = shared
         a, b = self._pf[0][:n], self._pf[1][:n]
         self._embed(tokens, a, n, st)
         self.layers[0].set_prefill_position(0, n)  # shared position buffers
