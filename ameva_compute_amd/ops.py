@@ -67,8 +67,8 @@ if MMQ_FORM not in ("exact", "scaled"):
 
 def act_type(wtype: int, m: int = 1, exact: bool | None = None) -> int:
     """The activation layout a MUL_MAT of m tokens reads: ggml's vec_dot_type (Q8_0 for Q4_0/Q8_0, Q8_K for the
-    K-quants) in the plain layout, except for batched Q4_K of MMQ_MIN_M..MMQ16_MIN_M tokens (the small-batch kernel
-    reads the f16 copies of Q8_K_MMA) and for the scaled form above MMQ16_MIN_M tokens when exact is False (DEQ;
+    K-quants) in the plain layout, except for batched Q4_K of MMQ_MIN_M..MMQ16_MIN_M tokens (Q8_K_MMA, whose f16 copies
+    the small-batch kernel reads up to QGEMM_MIN_M) and for the scaled form above MMQ16_MIN_M tokens when exact is False (DEQ;
     None: MMQ_FORM decides). The exact tiled kernel above MMQ16_MIN_M tokens reads the plain layout."""
     if exact is None:
         exact = MMQ_FORM == "exact"
@@ -174,7 +174,7 @@ MMQ_MIN_M = 8
 Q4_K_SB_MIN_M = 3
 QGEMM_MIN_M = 32  # above this many tokens the exact tiled kernels run (amv_mmq.hip QGEMM_MIN_M)
 MMQ16_MIN_M = 64  # above this many tokens the scaled form and act_type's plain Q4_K layout (amv_mmq.hip MMQ16_MIN_M)
-MMQ_TYPES = (Q4_0, Q8_0, Q4_K, Q6_K)  # Q4_K of MMQ_MIN_M..MMQ16_MIN_M tokens: the activations must be Q8_K_MMA
+MMQ_TYPES = (Q4_0, Q8_0, Q4_K, Q6_K)  # Q4_K of up to QGEMM_MIN_M tokens: Q8_K_MMA activations (plain Q8_K: tiled kernel)
 
 
 def mul_mat_q_add(w: QWeight, act: torch.Tensor, m: int, add: torch.Tensor, act_t: int | None = None,

@@ -67,7 +67,7 @@ int amv_unrepack(int type, const void* src, void* dst_ggml, int64_t n_rows, int6
  *           Q8_K: qs int8[m][k] | f32 d[m][k/256] | i32 sum(qs)[m][k/16]
  *           AMV_ACT_Q8_K_MMA: the Q8_K layout, then (16-byte aligned) the same values as f16 [m][k] (exact), the
  *           sums per 16 as f16 [m][k/16] and (16-byte aligned) the super-block scales transposed, f32 [k/256][m]:
- *           the batched Q4_K MUL_MAT of 8..64 tokens reads the f16 copies; its Q8_K prefix is a plain Q8_K
+ *           the batched Q4_K MUL_MAT of up to 32 tokens reads the f16 copies; its Q8_K prefix is a plain Q8_K
  *           activation of the m rows (amv_mul_mat_vec and the larger batches read it as such).
  *           AMV_ACT_Q8_0_MMA: the Q8_0 layout, then (16-byte aligned) the same values as f16 [m][k] and the block
  *           scales transposed, f32 [k/32][m]; its prefix is a plain Q8_0 activation of the m rows, which is what
@@ -95,6 +95,7 @@ int amv_quantize_q4_0(const float* x, int64_t n_rows, int64_t k, void* y_ggml, v
  *   w:   repacked weight (amv_repack layout) of n_rows x k
  *   act: amv_quantize_act y_act of m rows x k (Q8_0 for Q4_0/Q8_0 weights, Q8_K for Q4_K/Q6_K)
  *   dst: f32, element (row n, column c) at dst[c * ldd + n]; ldd >= n_rows
+ * 3..7 columns of Q4_0 / Q8_0 / Q6_K run amv_mul_mat_q's kernels where those are faster (the same block integers).
  * ---------------------------------------------------------------------------------------------------------- */
 int amv_mul_mat_vec(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int64_t m, float* dst,
                     int64_t ldd, void* stream);
@@ -226,20 +227,22 @@ int amv_mul_mat_q(int wtype, const void* w, int64_t n_rows, int64_t k, const voi
                   int64_t ldd, void* stream);
 int amv_mul_mat_q_block_sums(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int64_t m,
                              int32_t* sums, void* stream);
-/* amv_mul_mat_q with the activation layout named: act_type AMV_T_Q8_0, AMV_ACT_Q8_0_MMA, AMV_ACT_Q8_0_F6 (m > 64, Q4_0:
- * the 6-bit matrix instruction, bit for bit the plain layout's result) or AMV_ACT_Q8_0_DEQ for
- * Q4_0 / Q8_0 weights, AMV_T_Q8_K, AMV_ACT_Q8_K_MMA or AMV_ACT_Q8_K_DEQ for Q4_K (Q6_K: AMV_T_Q8_K or
- * AMV_ACT_Q8_K_MMA). With the plain or MMA layouts and m > 64 the product is the exact form on the int8 matrix cores
- * (one v_mfma_i32_32x32x32_i8 per 32-block: each block's ggml integer comes out exact, then ggml's f32 epilogue);
- * with the DEQ layouts and m > 64 the weights are staged as f16 (q - 8) d_w (Q4_K: (d sc) q - dmin m) against the
- * activations' f16 q_a d_a and the matrix cores accumulate across all of k (no per-block epilogue; within ~3e-4
- * relative L2 of the exact form). 8..64 tokens run the small-batch kernels (Q4_K on the MMA layout's f16 copies).
- * Block sums need a plain or MMA layout. */
 /* MUL_MAT of f32 activations x [m][k] in one call: amv_quantize_act(act_type, x, m, k, rule, NULL, act) and the product,
  * amv_mul_mat_q_act with batched != 0, else amv_mul_mat_vec (act_type then Q8_0 or Q8_K, plain). act: amv_act_bytes(act_type,
  * m, k) bytes, which hold the quantized activations afterwards. */
 int amv_mul_mat_f32(int wtype, const void* w, int64_t n_rows, int64_t k, const float* x, int64_t m, int act_type, int rule,
                     int batched, void* act, float* dst, int64_t ldd, void* stream);
+/* amv_mul_mat_q with the activation layout named: act_type AMV_T_Q8_0, AMV_ACT_Q8_0_MMA, AMV_ACT_Q8_0_F6 (m > 64, Q4_0:
+ * the 6-bit matrix instruction: the plain layout's block integers and f32 epilogue, k split where its own tiles leave CUs
+ * idle; small launches run the plain layout's kernels) or AMV_ACT_Q8_0_DEQ for
+ * Q4_0 / Q8_0 weights, AMV_T_Q8_K, AMV_ACT_Q8_K_MMA or AMV_ACT_Q8_K_DEQ for Q4_K (Q6_K: AMV_T_Q8_K or
+ * AMV_ACT_Q8_K_MMA). With the plain or MMA layouts and m > 32 the product is the exact form on the int8 matrix cores
+ * (one v_mfma_i32_32x32x32_i8 per 32-block: each block's ggml integer comes out exact, then ggml's f32 epilogue);
+ * with the DEQ layouts and m > 64 the weights are staged as f16 (q - 8) d_w (Q4_K: (d sc) q - dmin m) against the
+ * activations' f16 q_a d_a and the matrix cores accumulate across all of k (no per-block epilogue; within ~3e-4
+ * relative L2 of the exact form). Up to 32 tokens run the small-batch kernels (Q4_K on the MMA layout's f16 copies; a plain
+ * Q8_K activation of Q4_K runs the tiled one).
+ * Block sums need a plain or MMA layout. */
 int amv_mul_mat_q_act(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int act_type, int64_t m,
                       float* dst, int64_t ldd, void* stream);
 int amv_mul_mat_q_act_block_sums(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int act_type,
