@@ -284,6 +284,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // ---------------------------------------------------------------------------------------------------------------
 float* amv_splitk_workspace(size_t bytes, hipStream_t st);
 int amv_splitk_count(int64_t tiles, int steps);
+bool amv_qgemm_may_split(int64_t n_rows, int64_t m);
 void amv_splitk_reduce(const float* part, int S, int64_t zstride, int64_t m, int64_t n, float* dst, int64_t ldd,
                        hipStream_t st, const float* add = nullptr);
 
@@ -292,7 +293,7 @@ static int f6_launch(const void* w, int64_t n_rows, int64_t k, uint8_t* act, int
     const int nb = (int)(k / 32);
     const int n_tw = (int)((n_rows + BN - 1) / BN), n_tt = (int)((m + BM - 1) / BM);
     const int64_t tiles = (int64_t)n_tw * n_tt;
-    int S = sums ? 1 : amv_splitk_count(tiles, (nb + 1) / 2), per = nb;
+    int S = sums || !amv_qgemm_may_split(n_rows, m) ? 1 : amv_splitk_count(tiles, (nb + 1) / 2), per = nb;
     float* out = dst;
     int64_t ldo = ldd, zstride = 0;
     if (S > 1) {
@@ -339,7 +340,7 @@ int amv_qgemm_f6(const void* w, int64_t n_rows, int64_t k, void* act, int64_t m,
     // fewer than 1.5 workgroups per CU: the int8 kernel, whose smaller tiles share k between groups of waves (6144 x 4096 x
     // 512 57 us against 73, 4096 x 4096 x 96 21 against 69). Measured here against it (us): 28672 x 4096 x 512 184 (195),
     // 14336 x 4096 x 512 97 (98), 4096 x 14336 x 512 106 (114).
-    if (tiles * (sums ? 1 : amv_splitk_count(tiles, (nb + 1) / 2)) < 384)
+    if (tiles * (sums || !amv_qgemm_may_split(n_rows, m) ? 1 : amv_splitk_count(tiles, (nb + 1) / 2)) < 384)
         return amv_qgemm(AMV_T_Q4_0, w, n_rows, k, act, m, dst, ldd, sums, st, add);
     uint8_t* a = (uint8_t*)act;
     const AmvQ80F6 L = amv_q8_0_f6_layout(m, k);

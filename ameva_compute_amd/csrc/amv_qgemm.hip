@@ -777,11 +777,21 @@ static int qg_q6k(const QgCall& c) {  // ql [n][nsb][128] | qh [n][nsb][64] | sc
 }
 #undef QG_GO
 
+// Whether k may be split over workgroups: not where 64 x 64 tiles alone give four workgroups per CU and the 128 x 128 ones
+// are too few to be taken. Such a product fills the GPU with its wider tiles too (us, unsplit against 64 x 64 tiles staged
+// through registers: 11000 x 6144 x 331 Q4_K 83 / 129, Q8_0 122 / 166, Q4_0 122 / 160; 16400 x 6144 x 200 83 / 125, 120 /
+// 157, 116 / 155), and without the workspace it can overlap others on several streams and be a program's first product
+// under capture.
+bool amv_qgemm_may_split(int64_t n_rows, int64_t m) {
+    return ((m + 127) / 128) * ((n_rows + 127) / 128) >= 384 || ((m + 63) / 64) * ((n_rows + 63) / 64) < 1024;
+}
+
 int amv_qgemm(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int64_t m, float* dst, int64_t ldd,
               int32_t* sums, hipStream_t st, const float* add) {
     // Up to 64 tokens of Q4_0 / Q8_0 / Q4_K k stays whole: calls this small are made on several streams, which the split's
     // workspace does not allow at the same time.
-    const QgCall c{w, n_rows, k, act, m, dst, ldd, sums, st, add, !sums && (m > 64 || wtype == AMV_T_Q6_K)};
+    const QgCall c{w, n_rows, k, act, m, dst, ldd, sums, st, add,
+                   !sums && (wtype == AMV_T_Q6_K || (m > 64 && amv_qgemm_may_split(n_rows, m)))};
     const auto tiles = [&](int bm, int bn) { return ((m + bm - 1) / bm) * ((n_rows + bn - 1) / bn); };
     const auto wgs = [&](int bm, int bn) {  // workgroups with the split of k
         return tiles(bm, bn) * (c.split ? amv_splitk_count(tiles(bm, bn), (int)(k / 64)) : 1);
@@ -813,7 +823,7 @@ int amv_qgemm(int wtype, const void* w, int64_t n_rows, int64_t k, const void* a
     else if (wtype == AMV_T_Q4_0)
         rc = t64                ? qg_block<AMV_T_Q4_0, 1, 2, 4>(c)
              : t128             ? qg_block<AMV_T_Q4_0, 1, 4, 4>(c)
-             : big || k >= 6144 ? qg_block<AMV_T_Q4_0, 2, 4, 1>(c)
+             : big || (c.split && k >= 6144) ? qg_block<AMV_T_Q4_0, 2, 4, 1>(c)
                                 : qg_block<AMV_T_Q4_0, 1, 4, 2>(c);
     else if (wtype == AMV_T_Q8_0)
         rc = t64 ? qg_block<AMV_T_Q8_0, 1, 2, 4>(c) : t128 ? qg_block<AMV_T_Q8_0, 1, 4, 2>(c) : qg_block<AMV_T_Q8_0, 2, 4, 1>(c);
