@@ -137,19 +137,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 
     // Weights run four steps ahead in registers (a row's 32 bytes of a step are a quarter of a line, so this is the line
     // being fetched once, early); digits go to LDS without registers, one step ahead. Buffer loads: the per-thread
-    // offsets are fixed, the step is a scalar, and rows past N read as zero.
+    // offsets are fixed, the step is a scalar, and rows past N read as zero. A buffer's range check leaves out the scalar
+    // offset: each step's weights have a buffer that begins at its first block (an odd last step reads the next row's
+    // first block as its second, zero behind the last row), and the digits' block index stays below b_end. That second
+    // block is not computed.
     F6W sw0, sw1, sw2, sw3;
     const int blk = t & 1, wrow = t >> 1;
-    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(wq + (size_t)n0 * nb * 16), 0, (uint32_t)(min(BN, N - n0) * nb) * 16u, 0x00027000);
+    const uint8_t* const pw = wq + ((size_t)n0 * nb + b0) * 16;
+    const uint32_t wbytes = ((uint32_t)min(BN, N - n0) * nb - b0) * 16u;
     const __amdgpu_buffer_rsrc_t rd =
         __builtin_amdgcn_make_buffer_rsrc((void*)wd, 0, (uint32_t)N * (uint32_t)nb * 2u, 0x00027000);
-    const uint32_t ow = ((uint32_t)wrow * nb + b0 + blk) * 16u;
+    const uint32_t ow = ((uint32_t)wrow * nb + blk) * 16u;
     const int srow = min(n0 + wrow, N - 1);  // scales of a row pair side by side, an odd last row by itself
     const uint32_t od = (uint32_t)amv_q4_0_didx(srow, b0 + blk, nb, N) * 2u, sd = srow < (N & ~1) ? 8u : 4u;
     const auto load_w = [&](F6W& g, int step) {
         const int s = min(step, nsteps - 1);
-        g.w = __builtin_amdgcn_raw_buffer_load_b128(rw, ow, s * 32, 0);
+        const __amdgpu_buffer_rsrc_t rw =
+            __builtin_amdgcn_make_buffer_rsrc((void*)(pw + s * 32), 0, wbytes - s * 32, 0x00027000);
+        g.w = __builtin_amdgcn_raw_buffer_load_b128(rw, ow, 0, 0);
         g.dw = __builtin_amdgcn_raw_buffer_load_b16(rd, od + (uint32_t)s * sd, 0, 0);
         __builtin_amdgcn_sched_barrier(0);  // not after the step's arithmetic, where the compiler would put them
     };
@@ -160,34 +165,36 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     const __amdgpu_buffer_rsrc_t r8 = __builtin_amdgcn_make_buffer_rsrc((void*)d8, 0, (uint32_t)(region * 16), 0x00027000);
     const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc((void*)meta, 0, (uint32_t)(region * 8), 0x00027000);
     const auto load_d = [&](uint4* a16, uint2* a8, float2* mt, int step) {
-        const int s = min(step, nsteps - 1);
-        const uint32_t at = (uint32_t)(b0 + 2 * s) * (uint32_t)mp + (uint32_t)m0;  // (block, token) index
+        const int s = min(step, nsteps - 1), b = b0 + 2 * s, b1 = min(b + 1, b_end - 1);
+        const uint32_t at[2] = {(uint32_t)b * (uint32_t)mp + (uint32_t)m0,  // (block, token) index
+                                (uint32_t)b1 * (uint32_t)mp + (uint32_t)m0};
 #pragma unroll
         for (int bl = 0; bl < 2; ++bl) {
-            const uint32_t ab = at + bl * (uint32_t)mp;
+            const uint32_t ab = at[bl];
             // BM * 32 bytes of a block, 1 KB per wave; BM * 8, 256 per wave
             __builtin_amdgcn_raw_ptr_buffer_load_lds(r16, (f6_lds*)(a16 + bl * 2 * BM + 64 * wv), 16, 16 * t, ab * 32u, 0, 0);
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rm, (f6_lds*)(mt + bl * BM + 32 * wv), 4, 4 * t, ab * 8u, 0, 0);
         }
         // BM * 16 bytes per block: the two blocks' 1 KB pieces dealt to the waves
         __builtin_amdgcn_raw_ptr_buffer_load_lds(r8, (f6_lds*)(a8 + 128 * wv), 16, 16 * lane + 1024 * (wv & 1),
-                                                 (at + (wv >> 1) * (uint32_t)mp) * 16u, 0, 0);
+                                                 (wv >> 1 ? at[1] : at[0]) * 16u, 0, 0);
         __builtin_amdgcn_sched_barrier(0);  // these before the step's weight loads: the wait below counts on it
     };
-    const auto store = [&](const F6W& g, int step, uint4* w16, uint2* w8, float* dw) {
+    const auto store = [&](const F6W& g, uint4* w16, uint2* w8, float* dw) {
         int d[6];
         f6_spread(g.w.x, g.w.y, d[0], d[1], d[2]);
         f6_spread(g.w.z, g.w.w, d[3], d[4], d[5]);
         w16[blk * BN + wrow] = make_uint4(d[0], d[1], d[2], d[3]);
         w8[blk * BN + wrow] = make_uint2(d[4], d[5]);
-        // a block past the split's end: weight scale 0
-        dw[blk * BN + wrow] = b0 + 2 * step + blk >= b_end ? 0.0f : amv_h2f((uint16_t)g.dw);
+        dw[blk * BN + wrow] = amv_h2f((uint16_t)g.dw);
     };
     const int ea = F6_EXP_LO, eb = h ? F6_EXP_LO : F6_EXP_HI;  // half 0: the high digits
     const auto compute = [&](int step, const uint4* a16, const uint2* a8, const float2* mt,
                              const uint4* w16, const uint2* w8, const float* dw) {
+        const bool one = b0 + 2 * step + 1 == b_end;
 #pragma unroll 1
         for (int bl = 0; bl < 2; ++bl) {
+            if (bl && one) break;  // (a variable count of blocks compiles to a slower loop)
             const int tok = 32 * wm + c;
             const uint4 b4 = a16[(bl * BM + tok) * 2 + h];
             const uint2 b2 = a8[(bl * BM + tok) * 2 + h];
@@ -216,7 +223,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
                         for (int r = 0; r < 16; ++r) {
                             const int n = n0 + 32 * j + 8 * (r >> 2) + 4 * h + (r & 3);
-                            if (b < b_end && m < M && n < N) sums[((size_t)m * N + n) * nb + b] = (int32_t)P[r];
+                            if (m < M && n < N) sums[((size_t)m * N + n) * nb + b] = (int32_t)P[r];
                         }
                     } else {
 #pragma unroll
@@ -231,7 +238,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     load_w(sw1, 1);
     load_w(sw2, 2);
     load_w(sw3, 3);
-    store(sw0, 0, sW16a, sW8a, sDwa);
+    store(sw0, sW16a, sW8a, sDwa);
     F6_WAIT(6);  // the digits; the three later weight blocks (two loads each) may be out
     __syncthreads();
     // step u of four: digits of step + 1 to the other buffer, weights of step + 4 to the registers just free; then
@@ -241,7 +248,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     load_w(W, s0 + u + 4);                                                             \
     compute(s0 + u, sA16##X, sA8##X, sMt##X, sW16##X, sW8##X, sDw##X); \
     if (s0 + u + 1 >= nsteps) break;                                                   \
-    store(WN1, s0 + u + 1, sW16##Y, sW8##Y, sDw##Y);                       \
+    store(WN1, sW16##Y, sW8##Y, sDw##Y);                                               \
     F6_WAIT(2);                                                                        \
     __syncthreads();
     for (int s0 = 0;; s0 += 4) {
