@@ -121,22 +121,28 @@ __global__ __launch_bounds__(64 * WM * WN * KG) __attribute__((amdgpu_waves_per_
     const int b0 = z0 + 4 * nsteps * kg, b_end = min(z_end, b0 + 4 * nsteps);
     dst += (size_t)z * zstride;
 
-    const int mr = min(BM, M - m0), nr = min(BN, N - n0);  // rows past N and tokens past M read as zero
-    const __amdgpu_buffer_rsrc_t ra = QG_RSRC(aq + (size_t)m0 * K, mr * K);
-    const __amdgpu_buffer_rsrc_t rw = QG_RSRC(wq + (size_t)n0 * nb * WB, (uint32_t)(nr * nb) * WB);
+    // Rows past N, tokens past M and, behind the last of them, blocks past the end (a partial last step, the prefetch after
+    // it, groups without blocks) read as zero. A buffer's range check leaves out the scalar offset, so each step has a
+    // buffer that begins at its first block. Behind any other row blocks past the end are the next row's, and unused.
+    const int mr = min(BM, M - m0), nr = min(BN, N - n0);
+    const int8_t* const pa = aq + (size_t)m0 * K;
+    const uint8_t* const pw = wq + (size_t)n0 * nb * WB;
     const __amdgpu_buffer_rsrc_t rm = QG_RSRC(am + (size_t)m0 * nb, (uint32_t)(mr * nb) * 8u);
     const uint32_t oa = (uint32_t)(t >> 3) * K + 16 * ((t & 7) ^ ((t >> 4) & 7));
     const uint32_t ow = Q4 ? (uint32_t)(t >> 2) * (nb * 16) + 16 * ((t & 3) ^ ((t >> 4) & 3))
                            : (uint32_t)(t >> 3) * (nb * 32) + 16 * ((t & 7) ^ ((t >> 4) & 7));
     const auto load = [&](uint4* sA, uint4* sW, int b) {
+        const int bc = min(b, nb);
+        const __amdgpu_buffer_rsrc_t ra = QG_RSRC(pa + 32 * bc, (uint32_t)mr * K - 32u * bc);
+        const __amdgpu_buffer_rsrc_t rw = QG_RSRC(pw + WB * bc, (uint32_t)nr * (nb * WB) - (uint32_t)WB * bc);
 #pragma unroll
         for (int i = 0; i < RA; ++i)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (qg_lds*)(sA + NT * i + 64 * wv), 16,
-                                                     oa + (uint32_t)(NT / 8 * i) * K, 32 * b, 0, 0);
+                                                     oa + (uint32_t)(NT / 8 * i) * K, 0, 0, 0);
 #pragma unroll
         for (int i = 0; i < RW; ++i)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (qg_lds*)(sW + NT * i + 64 * wv), 16,
-                                                     ow + (uint32_t)(NT / WP * i) * (nb * WB), WB * b, 0, 0);
+                                                     ow + (uint32_t)(NT / WP * i) * (nb * WB), 0, 0, 0);
     };
     // scales, through registers: token x / 4 (row x / 4) of the block x % 4 of the step; 0 past the group's blocks
     float da[RDA];

@@ -1,6 +1,6 @@
 """Batched products whose operands are followed by 0xFF bytes (NaN scales, digits of -1): what lies behind an activation or a
 weight never reaches a product, where the last step has fewer blocks than a step holds (an odd number of 32-blocks for the
-6-bit kernel)."""
+6-bit kernel, a number that 4 does not divide for the int8 one) and where wave groups sharing k have no blocks at all."""
 import pytest
 
 torch = pytest.importorskip("torch")
@@ -38,3 +38,17 @@ def test_f6(n, k, m):
         check(lib().amv_mul_mat_q_act_block_sums(ops.Q4_0, w.data.data_ptr(), n, k, act.data_ptr(), at, m, s.data_ptr(),
                                                  torch.cuda.current_stream().cuda_stream), "block sums")
     assert torch.equal(*sums)
+
+
+@pytest.mark.parametrize("wtype", ["Q4_0", "Q8_0"])
+@pytest.mark.parametrize("n,k,m", [(1, 32, 33), (1, 96, 65), (3, 160, 40), (65, 416, 129), (8200, 32, 100)])
+def test_int8(wtype, n, k, m):
+    from ameva_compute_amd import ops
+    print(wtype, n, k, m, flush=True)
+    torch.manual_seed(n + k + m)
+    w = _weight(ops, getattr(ops, wtype), n, k)
+    act = ops.quantize_act(torch.randn((m, k), device="cuda"), ops.Q8_0)[0]
+    want = ops.mul_mat_q(w, act, m, act_t=ops.Q8_0)
+    assert bool(want.isfinite().all())
+    w.data = _framed(w.data)
+    assert torch.equal(ops.mul_mat_q(w, _framed(act), m, act_t=ops.Q8_0), want)
