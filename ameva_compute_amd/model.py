@@ -78,6 +78,17 @@ class LlamaModel:
         self.history.zero_()
 
     # ---------------------------------------------------------------------------------------------- prompt
+    def _prompt_buffers(self, n: int) -> None:
+        """The layers' prompt buffers for positions 0 .. n - 1: one set (positions included) for all layers whose weights
+        take the same activation layout at n tokens, each with its positions written."""
+        shared = {}
+        for lay in self.layers:
+            at = ops.gemm_act_type(lay.wqkv.type, n)
+            if at not in shared:
+                lay.set_prefill_position(0, n)
+                shared[at] = lay._pf
+            lay._pf, lay.pf_pos0, lay.pf_n = shared[at], 0, n
+
     def prefill(self, tokens: torch.Tensor) -> None:
         """The prompt (int32 [n] on the device, n <= ctx) through all layers at positions 0 .. n - 1; samples the
         first new token (token, history[step]) and sets the decode position to n."""
@@ -86,14 +97,10 @@ class LlamaModel:
         if self._pf is None or self._pf[0].shape[0] < n:
             f32 = dict(dtype=torch.float32, device=tokens.device)
             self._pf = (torch.empty((n, self.H), **f32), torch.empty((n, self.H), **f32))
-        shared = self.layers[0]._prefill_buffers(n)  # one set of prompt buffers (positions included) for all layers
-        for lay in self.layers:
-            lay._pf = shared
+        self._prompt_buffers(n)
         a, b = self._pf[0][:n], self._pf[1][:n]
         self._embed(tokens, a, n, st)
-        self.layers[0].set_prefill_position(0, n)  # shared position buffers
         for lay in self.layers:
-            lay.pf_pos0, lay.pf_n = 0, n
             lay.prefill(a, b)
             a, b = b, a
         self._head(a[n - 1], st)
