@@ -356,7 +356,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
     const auto frag = [&](const uint16_t* sK, int st) {
         return *reinterpret_cast<const fq_h8*>(&sK[kx + 8 * ((2 * st + h) ^ (c & 15))]);
     };
-    const bool pos = sl2 >= 0.0f;
+    const bool zero = sl2 == 0.0f, pos = sl2 >= 0.0f;
     fq_f16v s = {};
     // block b of this wave (scores s, rows of V in sV), and the scores of its next block from sK: the exponentials run
     // between the dependent products
@@ -384,11 +384,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
             for (int r = 0; r < 16; ++r) s[r] = x[r];
         }
+        float f = MASK ? 1.0f : sl2;  // what is left to multiply the scores with
+        if (!MASK && zero) {          // (before keys are hidden: infinity times 0 is no number)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] *= f;
+            f = 1.0f;
+        }
         if (!full) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int key = kb0 + 8 * (r >> 2) + 4 * h + (r & 3);
-                if (key > qlim) s[r] = MASK || pos ? -INFINITY : INFINITY;  // (times sl2 below)
+                if (key > qlim) s[r] = MASK || pos ? -INFINITY : INFINITY;  // (times f below)
             }
         }
         float mx = -INFINITY;
@@ -400,7 +406,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
             for (int r = 0; r < 16; ++r) mx = fminf(mx, s[r]);
         }
-        const float f = MASK ? 1.0f : sl2;
         mx = amv_max_x32(mx * f);
         // The running maximum always moves (k_fa_prefill lets it lag by 8): the largest weight so far is then exactly 1, which
         // outweighs the shorter key splits of that kernel (error against 64 bits at 2048 causal tokens 1.44e-4, there
