@@ -407,20 +407,23 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
             for (int r = 0; r < 16; ++r) mx = fminf(mx, s[r]);
         }
         mx = amv_max_x32(mx * f);
-        // The running maximum always moves (k_fa_prefill lets it lag by 8): the largest weight so far is then exactly 1, which
-        // outweighs the shorter key splits of that kernel (error against 64 bits at 2048 causal tokens 1.44e-4, there
-        // 1.55e-4; lagging by 8 it would be 1.59e-4 and 67 instead of 71 us)
-        const bool grow = mx > m;
+        // The weights' reference m: 14 below the running maximum, so that they reach 2^14 and f16 holds them in full down to
+        // 2^-28 of the largest (from the maximum itself f16 loses bits 2^-14 below it: a key that outweighs all others, such
+        // as a prompt's first one, then cost the others theirs: one at 11 above the rest with V = 0, error against 64 bits
+        // 2.0e-4, from the maximum 7.7e-3, k_fa_prefill 5.4e-3).
+        float mb = mx - 14.0f;
+        if (fabsf(mx) > 0x1p20f) mb = mx;  // where no difference of 14 is exact
+        const bool grow = mb > m;
         if (__builtin_amdgcn_ballot_w64(grow)) {
-            const float alpha = grow ? (m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mx)) : 1.0f;
-            if (grow) m = mx;
+            const float alpha = grow ? (m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mb)) : 1.0f;
+            if (grow) m = mb;
             l *= alpha;
 #pragma unroll
             for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
         }
         const float mref = m == -INFINITY ? 0.0f : m;
         // the weights' sum is taken over what enters the product, the f16 values (v_dot2_f32_f16: exact products, f32 sum):
-        // a query with one dominant key then keeps that key's row without the rounding of its weight
+        // a rounding is then in both (error against 64 bits at 2048 causal tokens 1.44e-4, with the sum before it 1.47e-4)
         float rs = 0.0f;
         fq_h8 p0, p1;
         fq_f16v z = {};

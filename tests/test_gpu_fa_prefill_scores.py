@@ -1,5 +1,6 @@
 """Prompt attention over shared K / V blocks at scores that are not the usual ones: a scale of 0 (every visible key weighs the
-same) or next to it, a negative one."""
+same) or next to it, a negative one; one key that outweighs all others; scores so far apart that f32 rounds them to whole
+numbers."""
 import math
 
 import pytest
@@ -37,3 +38,23 @@ def test_scale_zero_and_below(scale, n, keys, kind):
     mask = torch.zeros(n, keys, dtype=torch.float16, device="cuda").masked_fill_(~see, -math.inf) if kind == "mask" else None
     y = ops.flash_attn_prefill(q, k, v, scale, n_kv=keys, mask=mask, causal_pos0=0 if kind == "causal" else -1)
     assert _rel(y, _ref(q, k, v, see, scale)) < 2.0 ** -11  # weights rounded to f16
+
+
+@pytest.mark.parametrize("above,sinks", [(8, 1), (11, 16), (14, 1)])
+@pytest.mark.parametrize("kind", ["causal", "mask"])
+def test_dominating_first_keys(above, sinks, kind):
+    """Keys that draw most of every query's weight and hold no value: what is left of the others' weights is the result."""
+    from ameva_compute_amd import ops
+    n = 1024
+    torch.manual_seed(above)
+    q, k = torch.randn(n, 32, 128, device="cuda"), torch.randn(8, n, 128, device="cuda")
+    v = torch.randn(8, n, 128, device="cuda").half()
+    q[..., 0], k[..., 0], k[:, :sinks], v[:, :sinks] = 4.0, 0.0, 0.0, 0.0
+    k[:, :sinks, 0] = above * 128 ** 0.5 / 4
+    k = k.half()
+    see = torch.tril(torch.ones(n, n, dtype=torch.bool, device="cuda"))
+    mask = torch.zeros(n, n, dtype=torch.float16, device="cuda").masked_fill_(~see, -math.inf) if kind == "mask" else None
+    y = ops.flash_attn_prefill(q, k, v, 128 ** -0.5, n_kv=n, mask=mask, causal_pos0=0 if kind == "causal" else -1)
+    r = _ref(q, k, v, see, 128 ** -0.5)
+    # the others' weights, 2^(-1.44 (above + 4)) and more of the largest, rounded to f16 in full: 2^-11 at most each
+    assert _rel(y[sinks:], r[sinks:]) < 2.0 ** -11
