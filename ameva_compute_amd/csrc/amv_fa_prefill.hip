@@ -412,7 +412,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
         // as a prompt's first one, then cost the others theirs: one at 11 above the rest with V = 0, error against 64 bits
         // 2.0e-4, from the maximum 7.7e-3, k_fa_prefill 5.4e-3).
         float mb = mx - 14.0f;
-        if (fabsf(mx) > 0x1p20f) mb = mx;  // where no difference of 14 is exact
+        if (__builtin_amdgcn_ballot_w64(fabsf(mx) > 0x1p20f)) {  // where no difference of 14 is exact
+            // nor one of a score scaled in the fma below, unrounded, and the rounded maximum: it reached f16's infinity
+            if (!MASK) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[r] *= f;
+                f = 1.0f;
+            }
+            if (fabsf(mx) > 0x1p20f) mb = mx;
+        }
         const bool grow = mb > m;
         if (__builtin_amdgcn_ballot_w64(grow)) {
             const float alpha = grow ? (m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mb)) : 1.0f;

@@ -58,3 +58,23 @@ def test_dominating_first_keys(above, sinks, kind):
     r = _ref(q, k, v, see, 128 ** -0.5)
     # the others' weights, 2^(-1.44 (above + 4)) and more of the largest, rounded to f16 in full: 2^-11 at most each
     assert _rel(y[sinks:], r[sinks:]) < 2.0 ** -11
+
+
+@pytest.mark.parametrize("size", [3000.0, 20000.0])
+@pytest.mark.parametrize("kind", ["causal", "mask"])
+def test_huge_scores(size, kind):
+    """q and k near the end of f16's range: scores of 2^24 to 2^30, where the nearest f32 numbers are up to 64 apart and all
+    of a query's weight is on one key."""
+    from ameva_compute_amd import ops
+    n = 900
+    torch.manual_seed(int(size))
+    q, k = ((torch.randn(s, device="cuda") * size).clamp(-65000, 65000) for s in ((n, 32, 128), (8, n, 128)))
+    k, v = k.half(), torch.randn(8, n, 128, device="cuda").half()
+    see = torch.tril(torch.ones(n, n, dtype=torch.bool, device="cuda"))
+    mask = torch.zeros(n, n, dtype=torch.float16, device="cuda").masked_fill_(~see, -math.inf) if kind == "mask" else None
+    y = ops.flash_attn_prefill(q, k, v, 128 ** -0.5, n_kv=n, mask=mask, causal_pos0=0 if kind == "causal" else -1)
+    r = _ref(q, k, v, see, 128 ** -0.5)
+    assert bool(y.isfinite().all())
+    # two keys whose scores f32 cannot tell apart (about one query in a thousand at the larger size) share the weight
+    near = ((y - r).norm(dim=-1) < 2.0 ** -10 * r.norm(dim=-1)).float().mean().item()
+    assert near > 0.99
