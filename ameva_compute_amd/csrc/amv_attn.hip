@@ -8,7 +8,8 @@
 // score = sum_b float(isum_b) * (d_k * d_q) (vec_dot_q8_0_q8_0 / vec_dot_q4_0_q8_0). A quantized V row is dequantized
 // exactly (q * d). Scores, probabilities and accumulators are f32.
 //
-// Pass 1 (k_fa_split_mf for an f16 cache, k_fa_split_mq for Q8_0 / Q4_0, k_fa_split for f32): one workgroup of 4 waves
+// Pass 1 (k_fa_split_mf for an f16 cache, k_fa_split_mq for Q8_0 / Q4_0 and two or more heads per KV head, k_fa_split for
+// one, and for f32): one workgroup of 4 waves
 // per (key split, KV head); each wave owns KPW consecutive keys and works alone (wave maximum, probabilities and P V in
 // registers); the 4 wave partials meet once in LDS and the workgroup's (m, l, acc[D]) per head goes to
 // the workspace. Pass 2 (fa_merge): per head M = max m_z, w_z = e^(m_z - M), L = sum l_z w_z,
@@ -165,28 +166,95 @@ __device__ __forceinline__ void fa_merge(const float* part, int n_split, int ns,
 #define FA_Q4_0 2
 #define FA_F32 3  // the BitNet engine's cache (llama_bitnet_core.cpp:1022-1082): f32 q . k, no rounding of q
 
-// Pass 1 for an f32 cache. One workgroup per (split of 4 * KPW keys, KV head); each of its 4 waves owns KPW consecutive
-// keys and works alone: a 16-lane group owns keys 4 u + grp (u < KPW / 4) and reads 32 B of every K and V row of them
-// (all K and V loads of the wave are issued before the first is used); the G scores of a key are reduced over its 16
-// lanes; the wave's maximum, probabilities, l and P V stay in registers. The 4 wave partials are merged once through LDS.
-// The key count is read from n_kv_dev when given (capped at the launch's n_kv); splits past it do nothing. FUSED: the
-// last workgroup of each KV head to arrive merges the head's splits (fa_merge).
+typedef uint2 __attribute__((aligned(2))) fa_u2a;
 
-// A lane's slice of an f32 K / V row: elements 8 l16 .. 8 l16 + 7 (lane l16 = 0..15 of its 16-lane group).
+struct FaQ {
+    uint2 b;
+    uint32_t d;
+};
+// the bytes that hold elements 8 j .. 8 j + 7 (j = 0..3) of block b of a quantized row (Q4_0: j >= 2 the high nibbles)
+// and the block's f16 scale
+template <int KT>
+__device__ __forceinline__ FaQ fa_q8(const uint8_t* __restrict__ row, int b, int j) {
+    constexpr int BB = KT == FA_Q8_0 ? 34 : 18;
+    const uint8_t* p = row + BB * b;
+    return FaQ{*reinterpret_cast<const fa_u2a*>(p + 2 + 8 * (KT == FA_Q8_0 ? j : j & 1)),
+               *reinterpret_cast<const uint16_t*>(p)};
+}
+
+// the 8 values of such bytes: ggml dequantize_row_q8_0 / q4_0, q * d and (nibble - 8) * d
+template <int KT>
+__device__ __forceinline__ void fa_dequant(uint2 b, uint32_t d16, int j, float (&f)[8]) {
+    const float d = amv_h2f((uint16_t)d16);
+    const uint32_t w[2] = {b.x, b.y};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        if constexpr (KT == FA_Q8_0) f[e] = (float)(int8_t)(w[e >> 2] >> (8 * (e & 3))) * d;
+        else f[e] = ((float)((w[e >> 2] >> (8 * (e & 3) + ((j & 2) ? 4 : 0))) & 0xFu) - 8.0f) * d;
+    }
+}
+
+// A lane's slice of a K / V row: elements 8 l16 .. 8 l16 + 7 (lane l16 = 0..15 of its 16-lane group): 32 bytes of an f32 row;
+// fa_q8's bytes and scale (a.x, a.y, a.z) of a quantized one.
 struct FaRow {
     uint4 a, b;
 };
+template <int KT>
 __device__ __forceinline__ FaRow fa_row(const uint8_t* __restrict__ row, int l16) {
-    const uint4* p = reinterpret_cast<const uint4*>(row + 32 * l16);
-    return FaRow{amv_ld_stream(p), amv_ld_stream(p + 1)};
+    if constexpr (KT == FA_F32) {
+        const uint4* p = reinterpret_cast<const uint4*>(row + 32 * l16);
+        return FaRow{amv_ld_stream(p), amv_ld_stream(p + 1)};
+    } else {
+        const FaQ r = fa_q8<KT>(row, l16 >> 2, l16 & 3);
+        return FaRow{make_uint4(r.b.x, r.b.y, r.d, 0u), make_uint4(0u, 0u, 0u, 0u)};
+    }
+}
+template <int KT>
+__device__ __forceinline__ void fa_values(const FaRow& r, int l16, float (&f)[8]) {
+    if constexpr (KT == FA_F32) {
+        const uint32_t w[8] = {r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y, r.b.z, r.b.w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = __uint_as_float(w[e]);
+    } else {
+        fa_dequant<KT>(make_uint2(r.a.x, r.a.y), r.a.z, l16, f);
+    }
 }
 
-template <int G, int KPW, bool FUSED>
+// Q8_0 of 8 elements of q whose 32-block is spread over 4 lanes (amax the block's largest magnitude), with the rules of
+// amv_quantize_act (ggml quantize_row_q8_0): the int8, their sum, and the block's f16-rounded scale.
+__device__ __forceinline__ uint2 fa_quant8(const float (&x)[8], float amax, int rule, float& dq, int& sum) {
+    const float d = amax / 127.0f;
+    float id;
+    if (rule == AMV_Q8_X86) id = amax != 0.0f ? 127.0f / amax : 0.0f;
+    else id = d != 0.0f ? 1.0f / d : 0.0f;
+    uint32_t qq[2] = {0u, 0u};
+    sum = 0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float t = x[e] * id;
+        float qf = rule == AMV_Q8_REF ? roundf(t) : rintf(t);
+        qf = fminf(127.0f, fmaxf(-127.0f, qf));
+        const int qi = (int)qf;
+        sum += qi;
+        qq[e >> 2] |= (uint32_t)(qi & 0xFF) << (8 * (e & 3));
+    }
+    dq = amv_h2f(amv_f2h(d));
+    return make_uint2(qq[0], qq[1]);
+}
+
+// Pass 1 for an f32 cache, and for a Q8_0 / Q4_0 cache with one head per KV head. One workgroup per (split of 4 * KPW keys,
+// KV head); each of its 4 waves owns KPW consecutive keys and works alone: a 16-lane group owns keys 4 u + grp (u < KPW /
+// 4), each lane 8 dims of every K and V row of them (all K and V loads of the wave are issued before the first is used);
+// the G scores of a key are reduced over its 16 lanes; the wave's maximum, probabilities, l and P V stay in registers. The
+// 4 wave partials are merged once through LDS.
+// The key count is read from n_kv_dev when given (capped at the launch's n_kv); splits past it do nothing. FUSED: the
+// last workgroup of each KV head to arrive merges the head's splits (fa_merge).
+template <int G, int KPW, bool FUSED, int KT>
 __global__ __launch_bounds__(256) void k_fa_split(const float* __restrict__ q, const uint8_t* __restrict__ k,
                                                  const uint8_t* __restrict__ v, const uint16_t* __restrict__ mask,
                                                  float* part, int n_kv_max, const int* __restrict__ n_kv_dev,
                                                  int64_t k_row, int64_t k_head, int64_t v_row, int64_t v_head,
-                                                 int n_split, float scale, unsigned int* counters,
+                                                 int n_split, float scale, int qrule, unsigned int* counters,
                                                  float* __restrict__ out, const AmvActOut act) {
     constexpr int U = KPW / 4;
     constexpr int SBUF = 4 * 4 * G * FA_D > G * (8 * FA_D + FA_MAX_NSPLIT + 1) ? 4 * 4 * G * FA_D
@@ -208,12 +276,12 @@ __global__ __launch_bounds__(256) void k_fa_split(const float* __restrict__ q, c
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int i = min(kw0 + 4 * u + grp, n_kv - 1);
-            kr[u] = fa_row(kh + (size_t)i * k_row, lane & 15);
+            kr[u] = fa_row<KT>(kh + (size_t)i * k_row, lane & 15);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int i = min(kw0 + 4 * u + grp, n_kv - 1);
-            vr[u] = fa_row(vh + (size_t)i * v_row, lane & 15);
+            vr[u] = fa_row<KT>(vh + (size_t)i * v_row, lane & 15);
         }
         // the mask values of the lane's keys, loaded with the rest and converted where they are used (a load behind
         // a branch, or converted here, makes the compiler wait for every load issued so far); without a mask the
@@ -224,30 +292,56 @@ __global__ __launch_bounds__(256) void k_fa_split(const float* __restrict__ q, c
 #pragma unroll
             for (int u = 0; u < U; ++u) mraw[u] = mp[mask ? min(kw0 + 4 * u + grp, n_kv - 1) : 0];
         }
-        float qv[G][8];  // q of the G heads, 8 dims per lane
+        float qv[G][8];  // q of the G heads, 8 dims per lane; for a quantized cache its Q8_0 blocks, 4 lanes each
+        uint2 qq[G];
+        float qd[G];
+        int qsum[G];
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             const float4* qp = reinterpret_cast<const float4*>(q + (size_t)(hk * G + g) * FA_D + d8);
             const float4 a = qp[0], b = qp[1];
             const float t[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+            float amax = 0.0f;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) qv[g][e] = t[e];
+            for (int e = 0; e < 8; ++e) {
+                qv[g][e] = t[e];
+                amax = fmaxf(amax, fabsf(t[e]));
+            }
+            if constexpr (KT != FA_F32) {
+                amax = fmaxf(amax, __shfl_xor(amax, 1, AMV_WAVE));
+                amax = fmaxf(amax, __shfl_xor(amax, 2, AMV_WAVE));
+                qq[g] = fa_quant8(qv[g], amax, qrule, qd[g], qsum[g]);
+            }
         }
         float s[U][G];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int i = kw0 + 4 * u + grp;
             const float mk = (i < n_kv) ? (mask ? amv_h2f(mraw[u]) : 0.0f) : -INFINITY;
-            const uint4 x0 = kr[u].a, x1 = kr[u].b;
-            const uint32_t kw[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
             float kf[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) kf[e] = __uint_as_float(kw[e]);
+            uint2 kb = make_uint2(kr[u].a.x, kr[u].a.y);
+            const float dk = amv_h2f((uint16_t)kr[u].a.z);
+            if constexpr (KT == FA_F32) fa_values<KT>(kr[u], lane & 15, kf);
+            if constexpr (KT == FA_Q4_0) {
+                const int sh = (lane & 2) ? 4 : 0;
+                kb = make_uint2((kb.x >> sh) & 0x0F0F0F0Fu, (kb.y >> sh) & 0x0F0F0F0Fu);
+            }
 #pragma unroll
             for (int g = 0; g < G; ++g) {
                 float d = 0.0f;
+                if constexpr (KT == FA_F32) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) d = fmaf(qv[g][e], kf[e], d);
+                    for (int e = 0; e < 8; ++e) d = fmaf(qv[g][e], kf[e], d);
+                } else {
+                    int is = amv_dot4((int)kb.x, (int)qq[g].x, amv_dot4((int)kb.y, (int)qq[g].y, 0));
+                    if constexpr (KT == FA_Q4_0) is -= 8 * qsum[g];
+                    is += __shfl_xor(is, 1, AMV_WAVE);  // the block's exact integer sum in its 4 lanes
+                    is += __shfl_xor(is, 2, AMV_WAVE);
+                    // vec_dot_q8_0_q8_0: isum * (d_k * d_q); vec_dot_q4_0_q8_0: (isum * d_k) * d_q
+                    d = (lane & 3) != 0     ? 0.0f
+                        : KT == FA_Q8_0 ? (float)is * (dk * qd[g])
+                                        : ((float)is * dk) * qd[g];
+                }
                 d = amv_row16_sum(d);
                 s[u][g] = (mk == -INFINITY) ? -INFINITY : (d * scale + mk) * AMV_LOG2E;
             }
@@ -278,10 +372,7 @@ __global__ __launch_bounds__(256) void k_fa_split(const float* __restrict__ q, c
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             float vf[8];
-            const uint4 x0 = vr[u].a, x1 = vr[u].b;
-            const uint32_t vw[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-#pragma unroll
-            for (int e = 0; e < 8; ++e) vf[e] = __uint_as_float(vw[e]);
+            fa_values<KT>(vr[u], lane & 15, vf);
 #pragma unroll
             for (int g = 0; g < G; ++g)
 #pragma unroll
@@ -537,7 +628,8 @@ __global__ __launch_bounds__(256) void k_fa_split_mf(const float* __restrict__ q
     }
 }
 
-// Pass 1 for a Q8_0 or Q4_0 cache with the integer block dots on the matrix cores (same splits and partials): per
+// Pass 1 for a Q8_0 or Q4_0 cache and at least two heads per KV head, with the integer block dots on the matrix cores (same
+// splits and partials; one head leaves 15 of the 16 columns empty: 8192 keys of 32 heads Q8_0 28 us, k_fa_split 19): per
 // 16-key chunk and 32-block one v_mfma_i32_16x16x32_i8 gives the exact block integers of 16 keys and the G heads (A: key
 // l % 16, 8 bytes at dims 8 (l / 16); B: the quantized q of head l % 16, zero columns from G on; Q4_0: C = -8 sum(q)).
 // Lane l then holds keys 4 (l / 16) + e of head l % 16 and applies the blocks' scales as ggml does:
@@ -547,22 +639,7 @@ __global__ __launch_bounds__(256) void k_fa_split_mf(const float* __restrict__ q
 // KV heads of 4 heads with the merge: 19.5 us, now 14.4 (the rows are 17.8 MB, 3.5 us at the rate of a
 // copy). Rows are only 2-byte aligned: 8-byte loads at that alignment, where halfwords were read one by one. V: 16 lanes
 // per row, 8 dims per lane.
-typedef uint2 __attribute__((aligned(2))) fa_u2a;
 typedef int fa_i4 __attribute__((ext_vector_type(4)));
-
-struct FaQ {
-    uint2 b;
-    uint32_t d;
-};
-// the bytes that hold elements 8 j .. 8 j + 7 (j = 0..3) of block b of a quantized row (Q4_0: j >= 2 the high nibbles)
-// and the block's f16 scale
-template <int KT>
-__device__ __forceinline__ FaQ fa_q8(const uint8_t* __restrict__ row, int b, int j) {
-    constexpr int BB = KT == FA_Q8_0 ? 34 : 18;
-    const uint8_t* p = row + BB * b;
-    return FaQ{*reinterpret_cast<const fa_u2a*>(p + 2 + 8 * (KT == FA_Q8_0 ? j : j & 1)),
-               *reinterpret_cast<const uint16_t*>(p)};
-}
 
 template <int G, bool FUSED, int KPW, int KT>
 __global__ __launch_bounds__(256) void k_fa_split_mq(const float* __restrict__ q, const uint8_t* __restrict__ k,
@@ -629,33 +706,21 @@ __global__ __launch_bounds__(256) void k_fa_split_mq(const float* __restrict__ q
 #pragma unroll
             for (int e = 0; e < 8; ++e) qx[e] = t[e];
         }
-        {  // Q8_0 of the block with the rules of amv_quantize_act (ggml quantize_row_q8_0): 4 lanes of 8 elements
+        {  // Q8_0 of the block: 4 lanes of 8 elements
             float amax = 0.0f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(qx[e]));
             amax = amv_max_x32(amv_max_x16(amax));
-            const float d = amax / 127.0f;
-            float id;
-            if (qrule == AMV_Q8_X86) id = amax != 0.0f ? 127.0f / amax : 0.0f;
-            else id = d != 0.0f ? 1.0f / d : 0.0f;
-            uint32_t qq[2] = {0u, 0u};
-            int qs = 0;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float t = qx[e] * id;
-                float qf = qrule == AMV_Q8_REF ? roundf(t) : rintf(t);
-                qf = fminf(127.0f, fmaxf(-127.0f, qf));
-                const int qi = (int)qf;
-                qs += qi;
-                qq[e >> 2] |= (uint32_t)(qi & 0xFF) << (8 * (e & 3));
-            }
-            sQ[wv][lane] = c16 < G ? make_uint2(qq[0], qq[1]) : make_uint2(0u, 0u);
+            float dq;
+            int qs;
+            const uint2 qq = fa_quant8(qx, amax, qrule, dq, qs);
+            sQ[wv][lane] = c16 < G ? qq : make_uint2(0u, 0u);
             const auto r16 = __builtin_amdgcn_permlane16_swap(qs, qs, false, false);
             qs = (int)r16[0] + (int)r16[1];
             const auto r32 = __builtin_amdgcn_permlane32_swap(qs, qs, false, false);
             qs = (int)r32[0] + (int)r32[1];
             if (grp == 0) {
-                sDq[wv][c16] = amv_h2f(amv_f2h(d));
+                sDq[wv][c16] = dq;
                 sSq[wv][c16] = qs;
             }
         }
@@ -730,16 +795,7 @@ __global__ __launch_bounds__(256) void k_fa_split_mq(const float* __restrict__ q
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 float vf[8];
-                // ggml dequantize_row_q8_0 / q4_0: q * d, (nibble - 8) * d
-                const float dv = amv_h2f((uint16_t)vr[c][u].d);
-                const uint32_t w[2] = {vr[c][u].b.x, vr[c][u].b.y};
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    if constexpr (KT == FA_Q8_0)
-                        vf[e] = (float)(int8_t)(w[e >> 2] >> (8 * (e & 3))) * dv;
-                    else
-                        vf[e] = ((float)((w[e >> 2] >> (8 * (e & 3) + ((c16 & 2) ? 4 : 0))) & 0xFu) - 8.0f) * dv;
-                }
+                fa_dequant<KT>(vr[c][u].b, vr[c][u].d, c16, vf);
 #pragma unroll
                 for (int g = 0; g < G; ++g) {
                     const float p = sP[wv][16 * c + 4 * u + grp][g];
@@ -859,8 +915,8 @@ static void fa_launch_split(int G, int kpw, dim3 grid, hipStream_t st, const flo
                             int64_t k_row, int64_t k_head, int64_t v_row, int64_t v_head, int n_split, float scale,
                             int rule, unsigned int* counters, float* out, const AmvActOut& act) {
 #define FA_LAUNCH(GG, KK)                                                                                              \
-    hipLaunchKernelGGL((k_fa_split<GG, KK, FUSED>), grid, dim3(256), 0, st, q, kk, vv, mm, part, n_kv, n_kv_dev, \
-                       k_row, k_head, v_row, v_head, n_split, scale, counters, out, act)
+    hipLaunchKernelGGL((k_fa_split<GG, KK, FUSED, KT>), grid, dim3(256), 0, st, q, kk, vv, mm, part, n_kv, n_kv_dev, \
+                       k_row, k_head, v_row, v_head, n_split, scale, rule, counters, out, act)
 #define FA_MF(GG, KK)                                                                                            \
     hipLaunchKernelGGL((k_fa_split_mf<GG, FUSED, KK>), dim3(grid.y, grid.x), dim3(256), 0, st, q, kk, vv, mm, part, \
                        n_kv, n_kv_dev, k_row, k_head, v_row, v_head, n_split, scale, counters, out, act)
@@ -871,7 +927,7 @@ static void fa_launch_split(int G, int kpw, dim3 grid, hipStream_t st, const flo
     if constexpr (KT == FA_F16) {                                             \
         if (kpw == 16) FA_MF(GG, 16);                                         \
         else FA_MF(GG, 32);                                                   \
-    } else if constexpr (KT == FA_F32) {                                      \
+    } else if constexpr (KT == FA_F32 || GG == 1) {                           \
         if (kpw == 16) FA_LAUNCH(GG, 16);                                     \
         else FA_LAUNCH(GG, 32);                                               \
     } else {                                                                  \
