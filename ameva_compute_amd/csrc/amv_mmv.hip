@@ -1447,15 +1447,26 @@ extern "C" int amv_mul_mat_vec_ep(int wtype, const void* w, int64_t n_rows, int6
     return amv_check_launch("amv_mul_mat_vec_ep");
 }
 
-// Columns 3..7 of Q4_0, Q8_0 and Q6_K: the streamed small-batch kernels read the weights once for all columns (the same
-// block integers; Q4_K's read activations of another layout). Measured (us, 28672 x 4096 / 4096 x 14336, a launch per
-// column against one): Q4_0 2 columns 20 / 14 against 21 / 12, 3 30 / 20 against 21 / 12, 7 67 / 45 against 23 / 14; Q8_0
-// 3 56 / 33 against 35 / 18, 7 131 / 76 against 37 / 20; Q6_K 3 50 / 30 against 30 / 16, 7 114 / 67 against 31 / 17. Rows
-// that the streamed kernel does not take (k % 128 != 0, Q4_0 with an odd row count) from 5 columns: Q4_0 1025 x 4096
-// 4 9.2 against 10.9, 5 11.4 against 11.1, 7 16.0 against 11.7.
+// Columns 3..7 of Q4_0, Q8_0 and Q6_K: the small-batch kernels read the weights once for all columns (the same block integers;
+// Q4_K's read activations of another layout), streamed ones from 3 columns, the general one (k % 128 != 0, Q4_0 with an odd
+// row count) from 5. A launch per column costs 2.2 us and the weight's bytes each; the one launch a chain of loads along k,
+// whatever the rows. Measured (us, a launch per column against one):
+//   rows x k        Q4_0 3 columns / 7       Q8_0                     Q6_K
+//   14336 x 4096    20 / 13    35 / 14       32 / 20    75 / 21       30 / 17    64 / 17
+//   4096 x 14336    25 / 12    45 / 14       34 / 20    78 / 21       33 / 17    69 / 18
+//   2048 x 14336    15 / 12    32 / 14       16 / 17    36 / 19       18 / 17    41 / 17
+//   512 x 14336     8.7 / 12   18 / 14       8.4 / 17   18 / 19       11 / 16    24 / 16
+//   64 x 28672      9.8 / 20   21 / 23       9.4 / 30   21 / 33       14 / 29    31 / 29
+//   1024 x 4096     7.0 / 5.8  15 / 6.0      7.2 / 6.8  15 / 7.4      8.4 / 6.7  18 / 7.2
+// general: 4097 x 14368 with 5 columns Q4_0 38 / 40, Q8_0 57 / 38; 513 x 4128 12.6 / 10.6, 12.1 / 9.1
+// (two columns of 4096 x 14336 19 / 15, of 14336 x 4096 even). The times below in ns.
 static bool mmv_columns_batched(int wtype, int64_t n_rows, int64_t k, int64_t m) {
     if (m < 3 || m > 7 || wtype == AMV_T_Q4_K) return false;
-    return m >= 5 || wtype == AMV_T_Q6_K || (k % 128 == 0 && (wtype == AMV_T_Q8_0 || n_rows % 2 == 0));
+    const bool streamed = wtype == AMV_T_Q6_K || (k % 128 == 0 && (wtype == AMV_T_Q8_0 || n_rows % 2 == 0));
+    if (!streamed && m < 5) return false;
+    const double bytes = (double)amv_weight_bytes(wtype, n_rows, k);
+    const double per_k = wtype == AMV_T_Q6_K ? 0.8 : wtype == AMV_T_Q8_0 ? (streamed ? 1.2 : 1.6) : (streamed ? 0.75 : 1.8);
+    return (double)m * (2200.0 + 0.035 * (double)k + bytes / 9000.0) > 2500.0 + per_k * (double)k;
 }
 
 extern "C" int amv_mul_mat_vec(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int64_t m,

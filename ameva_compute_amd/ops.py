@@ -79,13 +79,14 @@ def act_type(wtype: int, m: int = 1, exact: bool | None = None) -> int:
     return Q8_K if wtype in (Q4_K, Q6_K) else Q8_0
 
 
-def gemm_act_type(wtype: int, m: int) -> int:
+def gemm_act_type(wtype: int, m: int, n_rows: int | None = None, k: int | None = None) -> int:
     """The activation layout the fastest MUL_MAT of m tokens in MMQ_FORM's arithmetic takes: act_type's, with the digits'
     scratch for Q4_0 above MMQ16_MIN_M tokens in the exact form (the 6-bit matrix instruction), and for Q4_K without the
-    f16 copies above QGEMM_MIN_M tokens (the tiled kernel reads the plain prefix) and with them from Q4_K_SB_MIN_M."""
+    f16 copies above QGEMM_MIN_M tokens (the tiled kernel reads the plain prefix) and with them from Q4_K_SB_MIN_M (given
+    the weight's shape: where one launch is the faster there)."""
     if wtype == Q4_K and QGEMM_MIN_M < m <= MMQ16_MIN_M:
         return Q8_K
-    if wtype == Q4_K and Q4_K_SB_MIN_M <= m < MMQ_MIN_M:
+    if wtype == Q4_K and Q4_K_SB_MIN_M <= m < MMQ_MIN_M and (k is None or _q4_k_few_batched(n_rows, k, m)):
         return Q8_K_MMA
     if wtype == Q4_0 and m > MMQ16_MIN_M and MMQ_FORM == "exact":
         return Q8_0_F6
@@ -172,6 +173,16 @@ MMQ_MIN_M = 8
 # 28672 x 4096 / 4096 x 14336: 2 tokens 24 / 15 against 26 / 16, 3 36 / 22 against 26 / 16, 7 78 / 50 against 28 / 18); the
 # types whose batched kernels read the plain layout switch in amv_mul_mat_vec
 Q4_K_SB_MIN_M = 3
+
+
+def _q4_k_few_batched(n_rows: int, k: int, m: int) -> bool:
+    """Whether one batched launch is faster than a GEMV per token for 3 to 7 tokens of Q4_K (ns): each GEMV costs a launch and
+    the weight's bytes, the one launch a chain of loads along k whatever the rows. Measured (us, 3 tokens / 7, GEMVs against
+    one launch): 512 x 14336 9.0 / 15.5, 20 / 18; 64 x 28672 12 / 26, 26 / 29; 2048 x 14336 14 / 16, 32 / 18; 1024 x 4096
+    8.4 / 6.1, 18 / 6.8; with the quantization 512 x 14336 5 tokens 17 / 19.5. The other types' rule is amv_mul_mat_vec's."""
+    return m * (2200 + 0.035 * k + n_rows * k * 0.5625 / 9000) > 2100 + 0.957 * k
+
+
 QGEMM_MIN_M = 32  # above this many tokens the exact tiled kernels run (amv_mmq.hip QGEMM_MIN_M)
 MMQ16_MIN_M = 64  # above this many tokens the scaled form and act_type's plain Q4_K layout (amv_mmq.hip MMQ16_MIN_M)
 MMQ_TYPES = (Q4_0, Q8_0, Q4_K, Q6_K)  # Q4_K of up to QGEMM_MIN_M tokens: Q8_K_MMA activations (plain Q8_K: tiled kernel)
@@ -191,21 +202,24 @@ def mul_mat_q_add(w: QWeight, act: torch.Tensor, m: int, add: torch.Tensor, act_
     return out
 
 
-def _batched(wtype: int, m: int, act_t: int | None) -> bool:
-    return wtype in MMQ_TYPES and (m >= MMQ_MIN_M or (m >= Q4_K_SB_MIN_M and wtype == Q4_K and act_t == Q8_K_MMA))
+def _batched(wtype: int, m: int, act_t: int | None, n_rows: int | None = None, k: int | None = None) -> bool:
+    if wtype not in MMQ_TYPES or m >= MMQ_MIN_M:
+        return wtype in MMQ_TYPES
+    return (m >= Q4_K_SB_MIN_M and wtype == Q4_K and act_t == Q8_K_MMA
+            and (k is None or _q4_k_few_batched(n_rows, k, m)))
 
 
 def mul_mat_q(w: QWeight, act: torch.Tensor, m: int, out: torch.Tensor | None = None,
               kernel: str = "auto", act_t: int | None = None) -> torch.Tensor:
     """dst [m, n_rows] f32 from already quantized activations (amv_quantize_act layout of m rows).
     kernel: "auto" (the reference's routing: MFMA GEMM for m >= MMQ_MIN_M where the type has one; Q4_K with act_t
-    Q8_K_MMA from Q4_K_SB_MIN_M), "mmv", "mmq".
+    Q8_K_MMA from Q4_K_SB_MIN_M where that is faster), "mmv", "mmq".
     Q4_K on "mmq" needs Q8_K_MMA activations up to MMQ16_MIN_M tokens. act_t: the activation layout (the DEQ
     layouts have the MMA sizes, so they must be named; None: told apart by size, i.e. plain or MMA)."""
     _need_gpu(act, "mul_mat_q")
     if out is None:
         out = torch.empty((m, w.n_rows), dtype=torch.float32, device=act.device)
-    if kernel == "mmq" or (kernel == "auto" and _batched(w.type, m, act_t)):
+    if kernel == "mmq" or (kernel == "auto" and _batched(w.type, m, act_t, w.n_rows, w.k)):
         at = act_layout(w.type, act, m, w.k) if act_t is None else act_t
         check(lib().amv_mul_mat_q_act(w.type, w.data.data_ptr(), w.n_rows, w.k, act.data_ptr(), at, m,
                                       out.data_ptr(), w.n_rows, _stream()), "amv_mul_mat_q_act")
@@ -308,7 +322,7 @@ def mul_mat(w: QWeight, x: torch.Tensor, rule: int = Q8_X86) -> torch.Tensor:
     _need_gpu(x2, "quantize_act")
     if x2.dtype != torch.float32:
         raise ValueError("quantize_act: f32 input expected")
-    at = gemm_act_type(w.type, m)
+    at = gemm_act_type(w.type, m, w.n_rows, k)
     n = _act_bytes(at, m, k)
     if n < 0:
         raise ValueError(f"quantize_act: type {at} cannot hold rows of {k}")

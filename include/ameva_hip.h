@@ -95,7 +95,8 @@ int amv_quantize_q4_0(const float* x, int64_t n_rows, int64_t k, void* y_ggml, v
  *   w:   repacked weight (amv_repack layout) of n_rows x k
  *   act: amv_quantize_act y_act of m rows x k (Q8_0 for Q4_0/Q8_0 weights, Q8_K for Q4_K/Q6_K)
  *   dst: f32, element (row n, column c) at dst[c * ldd + n]; ldd >= n_rows
- * 3..7 columns of Q4_0 / Q8_0 / Q6_K run amv_mul_mat_q's kernels where those are faster (the same block integers).
+ * 3..7 columns of Q4_0 / Q8_0 / Q6_K run amv_mul_mat_q's kernels where those are faster: the same block integers, their f32
+ * sums in another order than that of a column by itself.
  * ---------------------------------------------------------------------------------------------------------- */
 int amv_mul_mat_vec(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int64_t m, float* dst,
                     int64_t ldd, void* stream);
