@@ -147,7 +147,7 @@ __global__ __launch_bounds__(256) void k_i2s_gemv(const uint4* __restrict__ w, i
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// Batched (m >= I2S_MMQ_MIN_M tokens) I2_S MUL_MAT on int8 MFMA. The activation scale is per token over the whole row, so the
+// Batched (i2s_batched) I2_S MUL_MAT on int8 MFMA. The activation scale is per token over the whole row, so the
 // ternary dot stays integer across all of k: v_mfma_i32_32x32x32_i8 (the full-rate int8 shape of gfx950) accumulates
 // sum_k code * q in its int32 accumulator from the first block to the last (codes 0..3 are valid signed bytes), and
 // sum q is subtracted once.
@@ -326,16 +326,22 @@ extern "C" int amv_i2s_quantize_act(const float* x, int64_t m, int64_t k, void* 
     const bool vec = ((uintptr_t)x & 15) == 0;
 #define I2S_Q(U, V) hipLaunchKernelGGL((k_i2s_quant<U, V>), dim3((unsigned)m), dim3(256), 0, amv_stream(stream), x, (int)k, q, meta)
     if (!vec) I2S_Q(2, false);
+    else if (k <= 1024) I2S_Q(1, true);
     else if (k <= 3072) I2S_Q(3, true);
     else I2S_Q(8, true);
 #undef I2S_Q
     return amv_check_launch("amv_i2s_quantize_act");
 }
 
-// Tokens from which the MFMA kernel runs; below, a GEMV per token. 4 to 7 tokens keep k whole (no workspace: such calls
-// could always run on several streams at a time). Measured (us, GEMVs against one launch): 2560 x 6912 3 tokens 9.7 / 11,
-// 4 12.7 / 11.3, 7 21.5 / 11.9; 6912 x 2560 4 12.1 / 6.7, 7 19.8 / 7.3; 640 x 2560 3 6.2 / 6.6, 4 8 / 6.6, 7 13.5 / 7.1.
-#define I2S_MMQ_MIN_M 4
+// Whether the MFMA kernel runs, below it a GEMV per token: from 8 tokens, and for 4 to 7 where one launch is faster. Those
+// keep k whole (no workspace: such calls could always run on several streams at a time), so the launch takes a chain of loads
+// along k whatever the rows; a GEMV costs 1.7 us and the weight's bytes. Measured (us, GEMVs against one launch): 2560 x 6912
+// 3 tokens 10 / 11, 4 13 / 12, 7 22 / 12; 6912 x 2560 4 13 / 7.3, 7 21 / 7.7; 640 x 2560 3 6.5 / 6.6, 4 8.4 / 7.0; 320 x
+// 6912 4 9.4 / 11.5, 5 11.6 / 11.6; 320 x 17024 4 13 / 23, 6 20 / 23, 7 24 / 23; 2560 x 17024 4 22 / 23, 5 27 / 23. (In ns.)
+static bool i2s_batched(int64_t n_rows, int64_t k, int64_t m) {
+    if (m < 4 || m >= 8) return m >= 8;
+    return (double)m * (1650.0 + 0.094 * (double)k + (double)n_rows * (double)k / 18000.0) > 3900.0 + 1.12 * (double)k;
+}
 // The batched launch (k_i2s_mmq_p): 64 x 64 tiles, k split over S workgroups when the tiles alone leave CUs idle (about
 // one workgroup per CU: the four-block prefetch keeps a wave's 250 VGPRs, one wave per SIMD), the partials added by
 // k_i2s_split_sum. The integers do not depend on S (exact in any order): without the workspace (first needed under
@@ -410,7 +416,7 @@ static int i2s_gemv_impl(const void* w, int64_t n_rows, int64_t k, const void* a
     AMV_REQUIRE(((uintptr_t)w & 15) == 0 && ((uintptr_t)act & 15) == 0, "amv_i2s_gemv: buffers must be 16-byte aligned");
     AMV_REQUIRE(!dst || ldd >= n_rows, "amv_i2s_gemv: ldd < n_rows");
     hipStream_t st = amv_stream(stream);
-    if (m >= I2S_MMQ_MIN_M) {
+    if (i2s_batched(n_rows, k, m)) {
         i2s_mmq_p(w, n_rows, (int)(k / 128), act, m, wscale, dst, ldd, sums, st);
         return amv_check_launch("amv_i2s_gemv");
     }
