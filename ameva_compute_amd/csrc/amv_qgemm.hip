@@ -762,6 +762,16 @@ static int qg_q4k(const QgCall& c) {
     return AMV_OK;
 }
 
+// kg groups of waves (1, 2 or 4, at most MAX) share k
+template <int WT, int WM, int WN, int MAX = 4>
+static int qg_block_groups(const QgCall& c, int kg) {
+    return kg == 1 ? qg_block<WT, WM, WN, 1>(c) : kg == 2 ? qg_block<WT, WM, WN, 2>(c) : qg_block<WT, WM, WN, MAX>(c);
+}
+template <int WM, int WN>
+static int qg_q4k_groups(const QgCall& c, int kg) {
+    return kg == 1 ? qg_q4k<WM, WN, 1>(c) : kg == 2 ? qg_q4k<WM, WN, 2>(c) : qg_q4k<WM, WN, 4>(c);
+}
+
 template <int TT, int TW>
 static int qg_q6k(const QgCall& c) {  // ql [n][nsb][128] | qh [n][nsb][64] | scales [n][nsb][16] | d [n][nsb]
     const int nsb = (int)(c.k / 256);
@@ -819,20 +829,27 @@ int amv_qgemm(int wtype, const void* w, int64_t n_rows, int64_t k, const void* a
     // The neighbours of a choice: 14336 x 128 rows of Q4_K 35 with 64 x 64 tiles (448 of them), 6144 x 128 24 with 64 x 128
     // (17 with 64 x 64), 4096 x 512 41 with one group (29 with four).
     const bool t64 = wgs(64, 64) <= 256, t128 = wgs(64, 128) <= 256, two = wgs(64, 128) <= 512, big = tiles(128, 128) >= 384;
+    // No more groups than k has steps (Q4_K: super-blocks) for: those without cost their turns and the joining of the sums
+    // (us, 4096 x 256 with 65 / 512 tokens, four groups in brackets: Q4_K 6.0 (8.2) / 7.7 (12.7), Q4_0 6.1 (6.9) / 8.2 (10.4);
+    // 4096 x 768 of Q4_K keeps four: 8.2, two 8.9).
+    const int64_t units = wtype == AMV_T_Q4_K ? k / 256 : (k + 127) / 128;
+    const int kg = units >= 3 ? 4 : (int)units, kg2 = std::min(kg, 2);
     int rc;
     if (wtype == AMV_T_Q4_K)
-        rc = t64    ? qg_q4k<1, 2, 4>(c)
-             : t128 ? qg_q4k<1, 4, 4>(c)
-             : two  ? qg_q4k<1, 4, 2>(c)
+        rc = t64    ? qg_q4k_groups<1, 2>(c, kg)
+             : t128 ? qg_q4k_groups<1, 4>(c, kg)
+             : two  ? qg_q4k_groups<1, 4>(c, kg2)
              : big  ? qg_q4k<2, 4, 1>(c)
                     : qg_q4k<1, 4, 1>(c);
     else if (wtype == AMV_T_Q4_0)
-        rc = t64                ? qg_block<AMV_T_Q4_0, 1, 2, 4>(c)
-             : t128             ? qg_block<AMV_T_Q4_0, 1, 4, 4>(c)
-             : big || (c.split && k >= 6144) ? qg_block<AMV_T_Q4_0, 2, 4, 1>(c)
-                                : qg_block<AMV_T_Q4_0, 1, 4, 2>(c);
+        rc = t64                               ? qg_block_groups<AMV_T_Q4_0, 1, 2>(c, kg)
+             : t128                            ? qg_block_groups<AMV_T_Q4_0, 1, 4>(c, kg)
+             : big || (c.split && k >= 6144)   ? qg_block<AMV_T_Q4_0, 2, 4, 1>(c)
+                                               : qg_block_groups<AMV_T_Q4_0, 1, 4>(c, kg2);
     else if (wtype == AMV_T_Q8_0)
-        rc = t64 ? qg_block<AMV_T_Q8_0, 1, 2, 4>(c) : t128 ? qg_block<AMV_T_Q8_0, 1, 4, 2>(c) : qg_block<AMV_T_Q8_0, 2, 4, 1>(c);
+        rc = t64 ? qg_block_groups<AMV_T_Q8_0, 1, 2>(c, kg)
+             : t128 ? qg_block_groups<AMV_T_Q8_0, 1, 4, 2>(c, kg2)
+                    : qg_block<AMV_T_Q8_0, 2, 4, 1>(c);
     else
         rc = big ? qg_q6k<2, 2>(c) : qg_q6k<1, 1>(c);
     if (rc) return rc;
