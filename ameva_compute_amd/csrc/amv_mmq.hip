@@ -1012,6 +1012,18 @@ int amv_qgemm_f6(const void* w, int64_t n_rows, int64_t k, void* act, int64_t m,
 #define QGEMM_MIN_M 32
 #define MMQ16_MIN_M 64
 
+// The tiled kernels address a tile's rows by 32-bit offsets: rows of 2^25 elements and more (batches of up to 64 tokens: more
+// have always been limited to m k < 2^31) run a GEMV per token.
+#define QGEMM_MAX_K (1 << 25)
+static bool mmq_long_rows(int wtype, int64_t k, int64_t m, bool q4k_plain) {
+    return k >= QGEMM_MAX_K && wtype != AMV_T_Q6_K && m <= MMQ16_MIN_M && (m > QGEMM_MIN_M || q4k_plain);
+}
+static int mmq_per_token(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int64_t m, float* dst,
+                         int64_t ldd, int32_t* sums, void* stream) {
+    return sums ? amv_mul_mat_block_sums(wtype, w, n_rows, k, act, m, sums, stream)
+                : amv_mul_mat_vec(wtype, w, n_rows, k, act, m, dst, ldd, stream);
+}
+
 // q4k_mma: act is AMV_ACT_Q8_K_MMA (the small-batch Q4_K kernels read its f16 copies); with a plain Q8_K act every
 // Q4_K batch runs the tiled int8 kernel
 static int mmq_impl(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int64_t m, float* dst,
@@ -1029,7 +1041,9 @@ static int mmq_impl(int wtype, const void* w, int64_t n_rows, int64_t k, const v
     if (m > QGEMM_MIN_M || wtype == AMV_T_Q6_K || (wtype == AMV_T_Q4_K && !q4k_mma)) {
         AMV_REQUIRE((wtype != AMV_T_Q4_K && wtype != AMV_T_Q6_K) || k % 256 == 0,
                     "amv_mul_mat_q: K-quants need k %% 256 == 0");
-        AMV_REQUIRE(m * k <= INT32_MAX && m <= 65535LL * 128, "amv_mul_mat_q: too large");
+        const bool q4k_plain = wtype == AMV_T_Q4_K && !q4k_mma, too_long = mmq_long_rows(wtype, k, m, q4k_plain);
+        AMV_REQUIRE((m * k <= INT32_MAX || (too_long && !q4k_plain)) && m <= 65535LL * 128, "amv_mul_mat_q: too large");
+        if (too_long) return mmq_per_token(wtype, w, n_rows, k, act, m, dst, ldd, sums, stream);
         return amv_qgemm(wtype, w, n_rows, k, act, m, dst, ldd, sums, amv_stream(stream));
     }
     if (wtype == AMV_T_Q4_K) return mmq_q4k(w, n_rows, k, act, m, dst, ldd, sums, amv_stream(stream));
@@ -1077,7 +1091,8 @@ static int mmq_act_impl(const char* fn, int wtype, const void* w, int64_t n_rows
     const bool q80x = act_type == AMV_ACT_Q8_0_MMA || act_type == AMV_ACT_Q8_0_DEQ;
     const bool q8kx = act_type == AMV_ACT_Q8_K_MMA || act_type == AMV_ACT_Q8_K_DEQ;
     // Q6_K batches above 32 tokens run the tiled int8 kernel (up to 32 the streamed k_mmq_q6k_sb)
-    const bool tiled = (m > (deq ? MMQ16_MIN_M : QGEMM_MIN_M) && (((q80x || act_type == AMV_T_Q8_0) && (wtype == AMV_T_Q4_0 || wtype == AMV_T_Q8_0)) ||
+    const bool too_long = !deq && mmq_long_rows(wtype, k, m, act_type == AMV_T_Q8_K && wtype == AMV_T_Q4_K);
+    const bool tiled = !too_long && (m > (deq ? MMQ16_MIN_M : QGEMM_MIN_M) && (((q80x || act_type == AMV_T_Q8_0) && (wtype == AMV_T_Q4_0 || wtype == AMV_T_Q8_0)) ||
                                             ((q8kx || act_type == AMV_T_Q8_K) && wtype == AMV_T_Q4_K))) ||
                        ((q8kx || act_type == AMV_T_Q8_K) && wtype == AMV_T_Q6_K && m > 32);
     if (add && !(tiled && !deq)) {  // only the exact tiled kernels add the residual in their epilogue
