@@ -243,6 +243,9 @@ int amv_mul_mat_f32(int wtype, const void* w, int64_t n_rows, int64_t k, const f
  * activations' f16 q_a d_a and the matrix cores accumulate across all of k (no per-block epilogue; within ~3e-4
  * relative L2 of the exact form). Up to 32 tokens run the small-batch kernels (Q4_K on the MMA layout's f16 copies; a plain
  * Q8_K activation of Q4_K runs the tiled one).
+ * act is read only, except for an AMV_ACT_Q8_0_F6 activation of Q4_0 weights and m > 64: the product writes that layout's
+ * scratch part, so such an activation feeds one product at a time (overlapping products on two streams need one each; the
+ * plain layout has no such limit).
  * Block sums need a plain or MMA layout. */
 int amv_mul_mat_q_act(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int act_type, int64_t m,
                       float* dst, int64_t ldd, void* stream);

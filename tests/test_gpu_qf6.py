@@ -20,11 +20,11 @@ def _case(n, k, m, seed):
     return ops.QWeight.from_ggml(ops.Q4_0, wg, n, k), wg, torch.from_numpy(x).cuda()
 
 
-# (rows, k, tokens, exact): exact where all of k is summed in one order, as the int8 kernel does (which also takes the small
-# launches); with k split at other places two f32 sums of k / 32 products differ by at most 2 k / 32 roundings of 2^-24 of
+# (rows, k, tokens, exact), each of at least 384 tiles of 128 x 128, below which the int8 kernel runs: exact where all of k is
+# summed in one order, as the int8 kernel does; with k split at other places two f32 sums of k / 32 products differ by at most 2 k / 32 roundings of 2^-24 of
 # the sum of magnitudes
 @pytest.mark.parametrize("n,k,m,exact", [
-    (128, 32, 65, True), (1025, 512, 257, True), (12416, 256, 512, True), (12415, 224, 500, True), (12290, 32, 511, True),
+    (24450, 32, 129, True), (16301, 512, 257, True), (12416, 256, 512, True), (12415, 224, 500, True), (12290, 32, 511, True),
     (49100, 96, 65, True), (3072, 7200, 500, False)])
 def test_f6_against_int8(n, k, m, exact):
     w, _, x = _case(n, k, m, n + k + m)
@@ -43,7 +43,7 @@ def test_f6_against_int8(n, k, m, exact):
         assert bool(((y0 - y1).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("n,k,m", [(131, 96, 70), (12300, 96, 490)])
+@pytest.mark.parametrize("n,k,m", [(49031, 96, 70), (12300, 96, 490)])
 def test_f6_block_sums(n, k, m):
     w, wg, x = _case(n, k, m, n * 3 + m)
     x[0, :32] = 127.0  # the largest digits
@@ -54,6 +54,17 @@ def test_f6_block_sums(n, k, m):
                                              out.data_ptr(), torch.cuda.current_stream().cuda_stream), "block sums")
     _, ref = oracle.mul_mat(oracle.Q4_0, wg.cpu().numpy(), n, k, ag.cpu().numpy(), m, with_blocks=True)
     assert np.array_equal(out.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("n,k,m", [(128, 32, 65), (1025, 512, 257), (131, 96, 70)])
+def test_f6_small_launches(n, k, m):
+    """Fewer than 384 tiles: the activation's plain prefix on the int8 kernel."""
+    w, _, x = _case(n, k, m, n + k + m)
+    a0, a1 = (ops.quantize_act(x, t)[0] for t in (ops.Q8_0, ops.Q8_0_F6))
+    y = ops.mul_mat_q(w, a0, m, act_t=ops.Q8_0)
+    assert torch.equal(y, ops.mul_mat_q(w, a1, m, act_t=ops.Q8_0_F6))
+    e = torch.randn(m, n, device="cuda")
+    assert torch.equal(ops.mul_mat_q_add(w, a1, m, e, act_t=ops.Q8_0_F6), y + e)
 
 
 def test_f6_is_plain_elsewhere():
