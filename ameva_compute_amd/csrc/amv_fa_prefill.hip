@@ -260,14 +260,13 @@ __global__ __launch_bounds__(256) void k_fa_prefill(const float* __restrict__ q,
 // ---------------------------------------------------------------------------------------------------------------
 typedef __attribute__((address_space(3))) void fq_lds;
 typedef __attribute__((address_space(1))) const void fq_glb;
-// Every wave's LDS accesses done and at most n of its vector memory loads out, then the workgroup's barrier. (The fence of
-// __syncthreads would wait for all loads into LDS, the next step's too.)
-#define FQ_BARRIER(n)                              \
-    do {                                           \
-        asm volatile("" ::: "memory");             \
-        __builtin_amdgcn_s_waitcnt(0x0070 | (n));  \
-        __builtin_amdgcn_s_barrier();              \
-        asm volatile("" ::: "memory");             \
+// every wave's LDS accesses and vector memory loads (those into LDS too) done, then the workgroup's barrier
+#define FQ_BARRIER()                        \
+    do {                                    \
+        asm volatile("" ::: "memory");      \
+        __builtin_amdgcn_s_waitcnt(0x0070); \
+        __builtin_amdgcn_s_barrier();       \
+        asm volatile("" ::: "memory");      \
     } while (0)
 
 template <bool MASK>
@@ -469,23 +468,23 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
             }
     };
     const int kv = kg * FQ_KB * FQ_D;  // the group's block of a step
-    FQ_BARRIER(0);
+    FQ_BARRIER();
     if (kg < nblk)
 #pragma unroll
         for (int st = 0; st < 8; ++st) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag(sKa + kv, st), qb[st], s, 0, 0, 0);
-    FQ_BARRIER(0);
+    FQ_BARRIER();
     // step i: K rows of step i + 2 into the buffer that step i's came from, V rows of step i + 1 (past the last block: the
     // last key again), then the wave's block
     for (int i = 0;; i += 2) {
         load(kh, k_row, sKa, i + 2);
         load(vh, v_row, sVb, i + 1);
         if (2 * i + kg < nblk) step(sKb + kv, sVa + kv, 2 * i + kg);
-        FQ_BARRIER(0);
+        FQ_BARRIER();
         if (i + 1 >= nall) break;
         load(kh, k_row, sKb, i + 3);
         load(vh, v_row, sVa, i + 2);
         if (2 * (i + 1) + kg < nblk) step(sKa + kv, sVb + kv, 2 * (i + 1) + kg);
-        FQ_BARRIER(0);
+        FQ_BARRIER();
         if (i + 2 >= nall) break;
     }
     // the second group's (m, l, O^T) joins the first's: a quarter of O^T in each buffer, then m and l
@@ -550,9 +549,10 @@ extern "C" int amv_flash_attn_prefill(const float* q, int64_t q_tok_stride, int6
                 (long long)mask_stride);
     const int64_t G = n_head / n_head_kv, wgs = ((n_tok + 31) / 32 * G + 3) / 4 * n_head_kv;
     // Shared blocks once its workgroups (8 waves each) fill most CUs, with a mask from half of them (us, k_fa_prefill in
-    // brackets, 32 heads / 8 KV heads): 2048 causal tokens 71 (127), masked 136 (323); 1024 32 (46), 45 (94); 1024 after
-    // 1024 53 (80); 512 19 (18), 25 (29); 200 13 (9), 19 (12). Fewer tokens keep the kernel that splits a tile's keys over
-    // its four waves.
+    // brackets, 32 heads / 8 KV heads): 2048 causal tokens 66 (117), masked 130 (321); 1024 32 (44), 43 (90); 1024 after
+    // 8000 192 (298), 279 (662); 512 masked 26 (29), after 7680 248 (307). One head per KV head, 32: 1024 causal 31 (46),
+    // masked 43 (94), 512 masked 26 (36), after 7680 253 (354). Fewer tokens keep the kernel that splits a tile's keys over
+    // its four waves (512 causal 18, shared 19; 200 9, 13).
     if (wgs >= (mask ? 128 : 192)) {
         hipLaunchKernelGGL(mask ? k_fa_prefill_sh<true> : k_fa_prefill_sh<false>, dim3((unsigned)wgs), dim3(512), 0,
                            amv_stream(stream), q, q_tok_stride, q_head_stride, (const uint16_t*)k, (const uint16_t*)v,

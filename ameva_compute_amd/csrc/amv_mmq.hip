@@ -117,19 +117,15 @@ __device__ __forceinline__ void mmq_compute(const MmqFrag<TI, TJ, U>& f, int b0,
 }
 
 // FULLK: nb % U == 0 (every step is whole: block indices need no clamp and fold into load offsets).
-// KS = 4: the 4 waves share one tile (16 TI rows x 16 TJ tokens per workgroup) and split its pipeline steps
-// (wave w takes steps w, w + 4, ...); their f32 partials are added in LDS in wave order (small batches: many
-// workgroups instead of few long ones).
-template <int WT, bool SUMS, int TI, int TJ, int U, bool FULL, bool FULLK, int WR, int KS>
+// The 4 waves share one tile (16 TI rows x 16 TJ tokens per workgroup) and split its pipeline steps (wave w takes steps w,
+// w + 4, ...); their f32 partials are added in LDS in wave order: many workgroups instead of few long ones.
+template <int WT, bool SUMS, int TI, int TJ, int U, bool FULL, bool FULLK>
 __global__ __launch_bounds__(256) void k_mmq(const uint8_t* __restrict__ wq, const uint16_t* __restrict__ wd, int N,
                                             int nb, const int8_t* __restrict__ aq, const int2* __restrict__ ameta,
                                             int M, float* __restrict__ dst, int64_t ldd, int32_t* __restrict__ sums) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int r16 = lane & 15, g = lane >> 4;
-    // WR waves along the weight rows, 4 / WR along the tokens (KS = 1); with KS = 4 one tile per workgroup
-    const int n_wave = KS == 4 ? blockIdx.x * (16 * TI) : blockIdx.x * (WR * 16 * TI) + (w % WR) * (16 * TI);
-    const int m_wave = KS == 4 ? blockIdx.y * (16 * TJ) : blockIdx.y * ((4 / WR) * 16 * TJ) + (w / WR) * (16 * TJ);
-    const int ks = KS == 4 ? w : 0;
+    const int n_wave = blockIdx.x * (16 * TI), m_wave = blockIdx.y * (16 * TJ);
     const int K = nb * 32;
     float acc[TI][TJ][4];
 #pragma unroll
@@ -149,18 +145,18 @@ __global__ __launch_bounds__(256) void k_mmq(const uint8_t* __restrict__ wq, con
     // (steps of U blocks; the last step may be partial when nb % U != 0)
     const int steps = (nb + U - 1) / U;
     MmqFrag<TI, TJ, U> f0, f1;
-    int s = ks;
+    int s = w;
     if (s < steps) mmq_load<WT, TI, TJ, U, FULL, FULLK>(f0, s * U, wq, wd, N, nb, aq, ameta, K, nrow, mrow, n_wave, g);
-    for (; s + KS < steps; s += 2 * KS) {
-        mmq_load<WT, TI, TJ, U, FULL, FULLK>(f1, (s + KS) * U, wq, wd, N, nb, aq, ameta, K, nrow, mrow, n_wave, g);
+    for (; s + 4 < steps; s += 8) {
+        mmq_load<WT, TI, TJ, U, FULL, FULLK>(f1, (s + 4) * U, wq, wd, N, nb, aq, ameta, K, nrow, mrow, n_wave, g);
         mmq_compute<WT, SUMS, TI, TJ, U, FULLK>(f0, s * U, nb, sh, acc, N, M, n_wave, m_wave, g, r16, sums);
-        if (s + 2 * KS < steps)
-            mmq_load<WT, TI, TJ, U, FULL, FULLK>(f0, (s + 2 * KS) * U, wq, wd, N, nb, aq, ameta, K, nrow, mrow, n_wave,
+        if (s + 8 < steps)
+            mmq_load<WT, TI, TJ, U, FULL, FULLK>(f0, (s + 8) * U, wq, wd, N, nb, aq, ameta, K, nrow, mrow, n_wave,
                                                  g);
-        mmq_compute<WT, SUMS, TI, TJ, U, FULLK>(f1, (s + KS) * U, nb, sh, acc, N, M, n_wave, m_wave, g, r16, sums);
+        mmq_compute<WT, SUMS, TI, TJ, U, FULLK>(f1, (s + 4) * U, nb, sh, acc, N, M, n_wave, m_wave, g, r16, sums);
     }
     if (s < steps) mmq_compute<WT, SUMS, TI, TJ, U, FULLK>(f0, s * U, nb, sh, acc, N, M, n_wave, m_wave, g, r16, sums);
-    if constexpr (KS == 4 && !SUMS) {
+    if constexpr (!SUMS) {
         __shared__ float red[3][TI * TJ * 4][64];
         if (w > 0) {
 #pragma unroll
@@ -453,23 +449,20 @@ static bool mmq_sb_launch(const uint8_t* wq, const uint16_t* wd, int N, int nb, 
     return true;
 }
 
-template <int WT, bool SUMS, int TI, int TJ, int U, int WR = 2, int KS = 1>
+template <int WT, bool SUMS, int TI, int TJ, int U>
 static void mmq_launch(const uint8_t* wq, const uint16_t* wd, int N, int nb, const int8_t* aq, const int2* ameta,
                        int M, float* dst, int64_t ldd, int32_t* sums, hipStream_t st) {
-    constexpr int RT = KS == 4 ? 16 * TI : WR * 16 * TI, MT = KS == 4 ? 16 * TJ : (4 / WR) * 16 * TJ;
-    const dim3 grid((unsigned)((N + RT - 1) / RT), (unsigned)((M + MT - 1) / MT));
-    const bool full = N % RT == 0 && (!dst || ((uintptr_t)dst & 15) == 0);
+    const dim3 grid((unsigned)((N + 16 * TI - 1) / (16 * TI)), (unsigned)((M + 16 * TJ - 1) / (16 * TJ)));
+    const bool full = N % (16 * TI) == 0 && (!dst || ((uintptr_t)dst & 15) == 0);
     if (full && nb % U == 0)
-        hipLaunchKernelGGL((k_mmq<WT, SUMS, TI, TJ, U, true, true, WR, KS>), grid, dim3(256), 0, st, wq, wd, N, nb, aq,
-                           ameta, M, dst, ldd, sums);
+        hipLaunchKernelGGL((k_mmq<WT, SUMS, TI, TJ, U, true, true>), grid, dim3(256), 0, st, wq, wd, N, nb, aq, ameta, M,
+                           dst, ldd, sums);
     else
-        hipLaunchKernelGGL((k_mmq<WT, SUMS, TI, TJ, U, false, false, WR, KS>), grid, dim3(256), 0, st, wq, wd, N, nb,
-                           aq, ameta, M, dst, ldd, sums);
+        hipLaunchKernelGGL((k_mmq<WT, SUMS, TI, TJ, U, false, false>), grid, dim3(256), 0, st, wq, wd, N, nb, aq, ameta, M,
+                           dst, ldd, sums);
 }
 
-// Token tile by batch and grid fill (MI355X sweep, 512 tokens): 128-token workgroups (TJ = 4, one block per step)
-// while that still gives >= 192 workgroups (gate/up 28672 rows: 169 TOPS, q/k/v 6144: 136), otherwise 64 tokens
-// (TJ = 2, two blocks per step; the 4096-row projections: 130-134 TOPS against 93-98 with TJ = 4).
+// Up to 32 tokens: the streamed kernel, or k_mmq where that does not take the shape.
 template <int WT, bool SUMS>
 static void mmq_dispatch(const uint8_t* wq, const uint16_t* wd, int N, int nb, const int8_t* aq, const int2* ameta,
                          int M, float* dst, int64_t ldd, int32_t* sums, hipStream_t st) {
@@ -478,13 +471,13 @@ static void mmq_dispatch(const uint8_t* wq, const uint16_t* wd, int N, int nb, c
     // workgroups (M = 16: 14336 x 4096 28 us with TI = 4, 4096 x 14336 41 us with TI = 1)
     const int ti = N / 64 >= 224 ? 4 : (N / 32 >= 224 ? 2 : 1);
     if (M <= 16) {
-        if (ti == 4) mmq_launch<WT, SUMS, 4, 1, 2, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
-        else if (ti == 2) mmq_launch<WT, SUMS, 2, 1, 4, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
-        else mmq_launch<WT, SUMS, 1, 1, 4, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
+        if (ti == 4) mmq_launch<WT, SUMS, 4, 1, 2>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
+        else if (ti == 2) mmq_launch<WT, SUMS, 2, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
+        else mmq_launch<WT, SUMS, 1, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
     } else {
-        if (ti == 4) mmq_launch<WT, SUMS, 4, 2, 2, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
-        else if (ti == 2) mmq_launch<WT, SUMS, 2, 2, 2, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
-        else mmq_launch<WT, SUMS, 1, 2, 4, 1, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
+        if (ti == 4) mmq_launch<WT, SUMS, 4, 2, 2>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
+        else if (ti == 2) mmq_launch<WT, SUMS, 2, 2, 2>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
+        else mmq_launch<WT, SUMS, 1, 2, 4>(wq, wd, N, nb, aq, ameta, M, dst, ldd, sums, st);
     }
 }
 
@@ -1114,6 +1107,7 @@ static int mmq_act_impl(const char* fn, int wtype, const void* w, int64_t n_rows
         AMV_REQUIRE(!dst || ldd >= n_rows, "%s: ldd < n_rows", fn);
         if (wtype == AMV_T_Q4_K || wtype == AMV_T_Q6_K) AMV_REQUIRE(k % 256 == 0, "%s: K-quants need k %% 256 == 0", fn);
         AMV_REQUIRE(!(deq && wtype == AMV_T_Q6_K), "%s: Q6_K has no scaled form (use Q8_K or AMV_ACT_Q8_K_MMA)", fn);
+        // (the layout's scratch part is the product's to write)
         if (f6) return amv_qgemm_f6(w, n_rows, k, const_cast<void*>(act), m, dst, ldd, sums, amv_stream(stream), add);
         if (!deq) return amv_qgemm(wtype, w, n_rows, k, act, m, dst, ldd, sums, amv_stream(stream), add);
         if (wtype == AMV_T_Q4_K) return amv_mmq16_q4k(w, n_rows, k, act, m, dst, ldd, amv_stream(stream));

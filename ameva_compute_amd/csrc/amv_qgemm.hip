@@ -31,12 +31,8 @@ typedef int qg_v16i __attribute__((ext_vector_type(16)));
 typedef _Float16 qg_h8 __attribute__((ext_vector_type(8)));
 typedef float qg_f16v __attribute__((ext_vector_type(16)));
 
-#define QG_KS 64            // k per pipeline step
-#define QG_LD (QG_KS + 16)  // LDS row stride in bytes
-
 // byte-wise n - 8 of nibbles n in 0..15 (no carry crosses a byte: n + 0x78 <= 0x87)
 __device__ __forceinline__ uint32_t qg_m8(uint32_t v) { return (v + 0x78787878u) ^ 0x80808080u; }
-
 
 // ---------------------------------------------------------------------------------------------------------------
 // Q4_0 / Q8_0 x Q8_0. Bytes go from memory to LDS without registers (buffer_load .. lds), one step of four blocks (128 k)
