@@ -47,23 +47,6 @@ static inline AmvQ80Mma amv_q8_0_mma_layout(int64_t m, int64_t k) {
     return L;
 }
 
-// Offsets (bytes) of the AMV_ACT_Q8_0_F6 activation layout: the Q8_0 layout (rounded up to 16 bytes), then scratch that
-// the batched Q4_0 MUL_MAT fills itself (k_f6_pack): 6-bit digits of the int8 values, 2 x (16 + 8) bytes per block, and
-// {d, -8 sum} per block, [k/32][mp] with mp = m rounded up to 128.
-struct AmvQ80F6 {
-    int64_t d16, d8, meta, total, mp;
-};
-static inline AmvQ80F6 amv_q8_0_f6_layout(int64_t m, int64_t k) {
-    AmvQ80F6 L;
-    const int64_t nb = k / 32;
-    L.mp = (m + 127) & ~(int64_t)127;
-    L.d16 = (m * k + m * nb * 8 + 15) & ~(int64_t)15;
-    L.d8 = L.d16 + L.mp * nb * 32;
-    L.meta = L.d8 + L.mp * nb * 16;
-    L.total = L.meta + L.mp * nb * 8;
-    return L;
-}
-
 // ---------------------------------------------------------------------------------------------------------------
 // host: error state (first message of the failing call, per thread)
 void amv_set_error(const char* fmt, ...);

@@ -994,10 +994,6 @@ static int mmq_q4k(const void* w, int64_t n_rows, int64_t k, const void* act, in
 int amv_qgemm(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int64_t m, float* dst,
               int64_t ldd, int32_t* sums, hipStream_t st, const float* add = nullptr);
 
-// amv_qf6.hip: Q4_0 on the scaled 6-bit matrix instruction (AMV_ACT_Q8_0_F6 activations)
-int amv_qgemm_f6(const void* w, int64_t n_rows, int64_t k, void* act, int64_t m, float* dst, int64_t ldd, int32_t* sums,
-                 hipStream_t st, const float* add);
-
 // Batches above QGEMM_MIN_M tokens go to the tiled int8 kernels (amv_qgemm, the plain prefix of every layout; with a DEQ
 // layout from MMQ16_MIN_M tokens to the scaled f16 kernels); smaller ones to the k_mmq kernels of this file, which read the
 // plain Q8_0 prefix (Q4_0 / Q8_0) or the f16 copies of AMV_ACT_Q8_K_MMA (Q4_K). At 32 tokens the latter take 10 (4096 x
@@ -1077,8 +1073,6 @@ __global__ __launch_bounds__(256) void k_add_rows(float* __restrict__ dst, const
 static int mmq_act_impl(const char* fn, int wtype, const void* w, int64_t n_rows, int64_t k, const void* act,
                         int act_type, int64_t m, float* dst, int64_t ldd, int32_t* sums, void* stream,
                         const float* add = nullptr) {
-    // AMV_ACT_Q8_0_F6 is a plain Q8_0 activation wherever its scratch is not used
-    const bool f6 = act_type == AMV_ACT_Q8_0_F6 && wtype == AMV_T_Q4_0 && m > MMQ16_MIN_M;
     if (act_type == AMV_ACT_Q8_0_F6) act_type = AMV_T_Q8_0;
     const bool deq = act_type == AMV_ACT_Q8_0_DEQ || act_type == AMV_ACT_Q8_K_DEQ;
     const bool q80x = act_type == AMV_ACT_Q8_0_MMA || act_type == AMV_ACT_Q8_0_DEQ;
@@ -1107,8 +1101,6 @@ static int mmq_act_impl(const char* fn, int wtype, const void* w, int64_t n_rows
         AMV_REQUIRE(!dst || ldd >= n_rows, "%s: ldd < n_rows", fn);
         if (wtype == AMV_T_Q4_K || wtype == AMV_T_Q6_K) AMV_REQUIRE(k % 256 == 0, "%s: K-quants need k %% 256 == 0", fn);
         AMV_REQUIRE(!(deq && wtype == AMV_T_Q6_K), "%s: Q6_K has no scaled form (use Q8_K or AMV_ACT_Q8_K_MMA)", fn);
-        // (the layout's scratch part is the product's to write)
-        if (f6) return amv_qgemm_f6(w, n_rows, k, const_cast<void*>(act), m, dst, ldd, sums, amv_stream(stream), add);
         if (!deq) return amv_qgemm(wtype, w, n_rows, k, act, m, dst, ldd, sums, amv_stream(stream), add);
         if (wtype == AMV_T_Q4_K) return amv_mmq16_q4k(w, n_rows, k, act, m, dst, ldd, amv_stream(stream));
         return amv_mmq16(wtype, w, n_rows, k, act, m, dst, ldd, amv_stream(stream));

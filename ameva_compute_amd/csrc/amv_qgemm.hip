@@ -794,7 +794,7 @@ static int qg_q6k(const QgCall& c) {  // ql [n][nsb][128] | qh [n][nsb][64] | sc
 // through registers: 11000 x 6144 x 331 Q4_K 83 / 129, Q8_0 122 / 166, Q4_0 122 / 160; 16400 x 6144 x 200 83 / 125, 120 /
 // 157, 116 / 155), and without the workspace it can overlap others on several streams and be a program's first product
 // under capture.
-bool amv_qgemm_may_split(int64_t n_rows, int64_t m) {
+static bool qg_may_split(int64_t n_rows, int64_t m) {
     return ((m + 127) / 128) * ((n_rows + 127) / 128) >= 384 || ((m + 63) / 64) * ((n_rows + 63) / 64) < 1024;
 }
 
@@ -803,7 +803,7 @@ int amv_qgemm(int wtype, const void* w, int64_t n_rows, int64_t k, const void* a
     // Up to 64 tokens of Q4_0 / Q8_0 / Q4_K k stays whole: calls this small are made on several streams, which the split's
     // workspace does not allow at the same time.
     const QgCall c{w, n_rows, k, act, m, dst, ldd, sums, st, add,
-                   !sums && (wtype == AMV_T_Q6_K || (m > 64 && amv_qgemm_may_split(n_rows, m)))};
+                   !sums && (wtype == AMV_T_Q6_K || (m > 64 && qg_may_split(n_rows, m)))};
     const auto tiles = [&](int bm, int bn) { return ((m + bm - 1) / bm) * ((n_rows + bn - 1) / bn); };
     const auto wgs = [&](int bm, int bn) {  // workgroups with the split of k
         return tiles(bm, bn) * (c.split ? amv_splitk_count(tiles(bm, bn), (int)(k / 64)) : 1);

@@ -420,7 +420,7 @@ extern "C" int amv_quantize_act(int type, const float* x, int64_t m, int64_t k, 
     AMV_REQUIRE(((uintptr_t)x & 15) == 0, "amv_quantize_act: input must be 16-byte aligned");
     AMV_REQUIRE(y_act == nullptr || ((uintptr_t)y_act & 15) == 0, "amv_quantize_act: y_act must be 16-byte aligned");
     hipStream_t st = amv_stream(stream);
-    if (type == AMV_ACT_Q8_0_F6) type = AMV_T_Q8_0;  // the rest of that layout is the product's own
+    if (type == AMV_ACT_Q8_0_F6) type = AMV_T_Q8_0;
     const int deq = type == AMV_ACT_Q8_0_DEQ || type == AMV_ACT_Q8_K_DEQ;
     if (type == AMV_ACT_Q8_0_DEQ) type = AMV_ACT_Q8_0_MMA;  // same layout, scaled f16 copies
     if (type == AMV_ACT_Q8_K_DEQ) type = AMV_ACT_Q8_K_MMA;

@@ -658,15 +658,14 @@ struct Engine {
         const int64_t K = w->ne[0], M = nrows(x);
         // batched (M >= 8) MUL_MATs run on the matrix cores for Q4_0 / Q8_0 / Q4_K / Q6_K (the reference's switch at
         // AMEVA_QGEMM_MIN_M). Above 64 tokens the exact form (exact per-block integer sums, ggml's f32 epilogue: the
-        // reference's MMQ arithmetic) reads the plain Q8_0 / Q8_K layout (Q4_0: with room for its 6-bit digits); Q4_K
-        // batches of 8..32 tokens read the f16 copies of AMV_ACT_Q8_K_MMA; AMEVA_MMQ_FORM=scaled selects the scaled layouts (f16 q * d) above 64 tokens
+        // reference's MMQ arithmetic) reads the plain Q8_0 / Q8_K layout; Q4_K batches of 8..32 tokens read the f16
+        // copies of AMV_ACT_Q8_K_MMA; AMEVA_MMQ_FORM=scaled selects the scaled layouts (f16 q * d) above 64 tokens
         const bool mmq = M >= 8 && (w->type == GGML_TYPE_Q4_0 || w->type == GGML_TYPE_Q8_0 || w->type == GGML_TYPE_Q4_K ||
                                     w->type == GGML_TYPE_Q6_K);
         const bool kq = w->type == GGML_TYPE_Q4_K || w->type == GGML_TYPE_Q6_K;
         const bool deq = mmq && M > 64 && mmq_scaled() && w->type != GGML_TYPE_Q6_K;  // Q6_K: exact form only
         const int atype = deq ? (kq ? AMV_ACT_Q8_K_DEQ : AMV_ACT_Q8_0_DEQ)
                         : (mmq && w->type == GGML_TYPE_Q4_K && M <= 32) ? AMV_ACT_Q8_K_MMA
-                        : (mmq && w->type == GGML_TYPE_Q4_0 && M > 64) ? AMV_ACT_Q8_0_F6
                         : kq ? (int)GGML_TYPE_Q8_K : (int)GGML_TYPE_Q8_0;
         if (!mmq && !ep && raw_readable(w)) return mul_mat_raw(n, atype);
         const void* wp = weight_ptr(n);
@@ -911,8 +910,7 @@ struct Engine {
         for (int i = 0; i < g->n_nodes; ++i) {
             const ggml_tensor* n = g->nodes[i];
             if (n->op == GGML_OP_MUL_MAT) {
-                s += (size_t)std::max(amv_act_bytes(AMV_ACT_Q8_0_MMA, nrows(n->src[1]), n->src[1]->ne[0]),
-                                      amv_act_bytes(AMV_ACT_Q8_0_F6, nrows(n->src[1]), n->src[1]->ne[0])) + 4096;
+                s += (size_t)amv_act_bytes(AMV_ACT_Q8_0_MMA, nrows(n->src[1]), n->src[1]->ne[0]) + 4096;
                 s += (size_t)amv_act_bytes(AMV_ACT_Q8_K_MMA, nrows(n->src[1]), (n->src[1]->ne[0] + 255) / 256 * 256) + 4096;
                 if (n->src[0]->view_src) s += nbytes(n->src[0]->view_src) + nbytes(n->src[0]) + 512;
                 else if (n->src[0]->buffer->usage != GGML_BACKEND_BUFFER_USAGE_WEIGHTS) s += nbytes(n->src[0]) + 256;

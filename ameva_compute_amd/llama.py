@@ -204,7 +204,7 @@ class LlamaLayer:
                 "act_att": torch.empty(L.amv_act_bytes(at, n_tok, H), **u8),
                 "act_h2": torch.empty(L.amv_act_bytes(at, n_tok, H), **u8),
                 "act_ff": torch.empty(L.amv_act_bytes(at, n_tok, FF), **u8),
-                "h": torch.empty((n_tok, FF), **f32) if at not in (ops.Q8_0, ops.Q8_0_F6, ops.Q8_K) else None,
+                "h": torch.empty((n_tok, FF), **f32) if at not in (ops.Q8_0, ops.Q8_K) else None,
                 "pos": torch.zeros(n_tok, dtype=torch.int32, device=dev),
                 "idx": torch.zeros(n_tok, dtype=torch.int64, device=dev)}
         self._pf = sets[at] = bufs
@@ -242,15 +242,13 @@ class LlamaLayer:
             def mm_add(wt, w, nr, k, act, m, dst, ldd, add, what):
                 check(mm(wt, w, nr, k, act, m, dst, ldd, st), what)
                 check(L.amv_binary(0, dst, add, dst, m, nr, m, st), what + " residual")
-        # plain layouts (and the plain prefix of Q8_0_F6): the norms and SWIGLU write them directly
-        q8 = at in (ops.Q8_0, ops.Q8_0_F6, ops.Q8_K)
-        pt = ops.Q8_0 if at == ops.Q8_0_F6 else at
+        q8 = at in (ops.Q8_0, ops.Q8_K)  # plain layouts: the norms and SWIGLU write them directly
 
         def quant(src, k, act):
             check(L.amv_quantize_act(at, src, n, k, ops.Q8_X86, None, P(act), st), "quantize")
 
         check(L.amv_rms_norm_act(P(x), n, H, self.eps, P(self.attn_norm), None, None if q8 else P(b["t_o"]),
-                                 P(b["act_h"]) if q8 else None, pt, ops.Q8_X86, st), "rms_norm")
+                                 P(b["act_h"]) if q8 else None, at, ops.Q8_X86, st), "rms_norm")
         if not q8:
             quant(P(b["t_o"]), H, b["act_h"])
         nq = self.wqkv.n_rows
@@ -264,14 +262,14 @@ class LlamaLayer:
         quant(P(b["att"]), H, b["act_att"])
         mm_add(self.wo.type, P(self.wo.data), H, H, P(b["act_att"]), n, P(b["x1"]), H, P(x), "wo + residual")
         check(L.amv_rms_norm_act(P(b["x1"]), n, H, self.eps, P(self.ffn_norm), None, None if q8 else P(b["t_o2"]),
-                                 P(b["act_h2"]) if q8 else None, pt, ops.Q8_X86, st), "ffn norm")
+                                 P(b["act_h2"]) if q8 else None, at, ops.Q8_X86, st), "ffn norm")
         if not q8:
             quant(P(b["t_o2"]), H, b["act_h2"])
         ng = self.wgu.n_rows
         check(mm(self.wgu.type, P(self.wgu.data), ng, H, P(b["act_h2"]), n, P(b["gu"]), ng, st), "gate_up")
         if q8:
             check(L.amv_swiglu_rows_act(P(b["gu"]), ng, P(b["gu"]) + FF * 4, ng, None, FF, n, FF, P(b["act_ff"]),
-                                        pt, ops.Q8_X86, st), "swiglu + quant")
+                                        at, ops.Q8_X86, st), "swiglu + quant")
         else:
             check(L.amv_swiglu_rows(P(b["gu"]), ng, P(b["gu"]) + FF * 4, ng, P(b["h"]), FF, n, FF, None, ops.Q8_X86,
                                     st), "swiglu")

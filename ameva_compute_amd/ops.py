@@ -53,7 +53,7 @@ Q8_0_MMA = 1008
 # the same layouts with f16 q * d in place of f16 q: the scaled batched MUL_MAT (AMV_ACT_Q8_K_DEQ / AMV_ACT_Q8_0_DEQ)
 Q8_K_DEQ = 1115
 Q8_0_DEQ = 1108
-# Q8_0 activations with the scratch in which the batched Q4_0 MUL_MAT keeps their 6-bit digits (AMV_ACT_Q8_0_F6)
+# accepted as Q8_0 (AMV_ACT_Q8_0_F6)
 Q8_0_F6 = 1208
 
 
@@ -80,16 +80,13 @@ def act_type(wtype: int, m: int = 1, exact: bool | None = None) -> int:
 
 
 def gemm_act_type(wtype: int, m: int, n_rows: int | None = None, k: int | None = None) -> int:
-    """The activation layout the fastest MUL_MAT of m tokens in MMQ_FORM's arithmetic takes: act_type's, with the digits'
-    scratch for Q4_0 above MMQ16_MIN_M tokens in the exact form (the 6-bit matrix instruction), and for Q4_K without the
-    f16 copies above QGEMM_MIN_M tokens (the tiled kernel reads the plain prefix) and with them from Q4_K_SB_MIN_M (given
-    the weight's shape: where one launch is the faster there)."""
+    """The activation layout the fastest MUL_MAT of m tokens in MMQ_FORM's arithmetic takes: act_type's, but for Q4_K without
+    the f16 copies above QGEMM_MIN_M tokens (the tiled kernel reads the plain prefix) and with them from Q4_K_SB_MIN_M
+    (given the weight's shape: where one launch is the faster there)."""
     if wtype == Q4_K and QGEMM_MIN_M < m <= MMQ16_MIN_M:
         return Q8_K
     if wtype == Q4_K and Q4_K_SB_MIN_M <= m < MMQ_MIN_M and (k is None or _q4_k_few_batched(n_rows, k, m)):
         return Q8_K_MMA
-    if wtype == Q4_0 and m > MMQ16_MIN_M and MMQ_FORM == "exact":
-        return Q8_0_F6
     return act_type(wtype, m)
 
 

@@ -31,7 +31,7 @@ extern "C" {
 #define AMV_ACT_Q8_0_MMA 1008 /* Q8_0 activations with the f16 copies the batched Q4_0 / Q8_0 MUL_MAT reads */
 #define AMV_ACT_Q8_K_DEQ 1115 /* AMV_ACT_Q8_K_MMA's layout with f16 q * d in place of f16 q (the scaled batched form) */
 #define AMV_ACT_Q8_0_DEQ 1108 /* AMV_ACT_Q8_0_MMA's layout with f16 q * d in place of f16 q (the scaled batched form) */
-#define AMV_ACT_Q8_0_F6 1208  /* Q8_0 activations with room for the 6-bit digits the batched Q4_0 MUL_MAT makes of them */
+#define AMV_ACT_Q8_0_F6 1208  /* accepted as AMV_T_Q8_0 */
 #define AMV_Q8_X86 0
 #define AMV_Q8_ARM 1
 #define AMV_Q8_REF 2
@@ -74,11 +74,8 @@ int amv_unrepack(int type, const void* src, void* dst_ggml, int64_t n_rows, int6
  *           the batched Q4_0 / Q8_0 MUL_MAT reads.
  *           AMV_ACT_Q8_0_DEQ / AMV_ACT_Q8_K_DEQ: the same layouts (and sizes) with f16 of q * d (one rounding) in
  *           place of the f16 copies of q: the input of the scaled batched MUL_MAT.
- *           AMV_ACT_Q8_0_F6: the Q8_0 layout (which is all that amv_quantize_act writes), then scratch that
- *           amv_mul_mat_q_act fills for Q4_0 weights and m > 64; every other use reads the prefix. One such buffer
- *           feeds one product at a time (products that overlap on two streams need a buffer each).
  * type AMV_T Q8_0 (8), Q8_K (15), AMV_ACT_Q8_K_MMA, AMV_ACT_Q8_0_MMA, AMV_ACT_Q8_K_DEQ, AMV_ACT_Q8_0_DEQ or
- * AMV_ACT_Q8_0_F6; rule applies to the Q8_0 forms only.
+ * AMV_ACT_Q8_0_F6 (the plain Q8_0 layout); rule applies to the Q8_0 forms only.
  * ---------------------------------------------------------------------------------------------------------- */
 int64_t amv_act_bytes(int type, int64_t m, int64_t k);
 int amv_quantize_act(int type, const float* x, int64_t m, int64_t k, int rule, void* y_ggml, void* y_act,
@@ -233,9 +230,7 @@ int amv_mul_mat_q_block_sums(int wtype, const void* w, int64_t n_rows, int64_t k
  * m, k) bytes, which hold the quantized activations afterwards. */
 int amv_mul_mat_f32(int wtype, const void* w, int64_t n_rows, int64_t k, const float* x, int64_t m, int act_type, int rule,
                     int batched, void* act, float* dst, int64_t ldd, void* stream);
-/* amv_mul_mat_q with the activation layout named: act_type AMV_T_Q8_0, AMV_ACT_Q8_0_MMA, AMV_ACT_Q8_0_F6 (m > 64, Q4_0:
- * the 6-bit matrix instruction: the plain layout's block integers and f32 epilogue, k split where its own tiles leave CUs
- * idle; small launches run the plain layout's kernels) or AMV_ACT_Q8_0_DEQ for
+/* amv_mul_mat_q with the activation layout named: act_type AMV_T_Q8_0, AMV_ACT_Q8_0_MMA or AMV_ACT_Q8_0_DEQ for
  * Q4_0 / Q8_0 weights, AMV_T_Q8_K, AMV_ACT_Q8_K_MMA or AMV_ACT_Q8_K_DEQ for Q4_K (Q6_K: AMV_T_Q8_K or
  * AMV_ACT_Q8_K_MMA). With the plain or MMA layouts and m > 32 the product is the exact form on the int8 matrix cores
  * (one v_mfma_i32_32x32x32_i8 per 32-block: each block's ggml integer comes out exact, then ggml's f32 epilogue);
@@ -243,9 +238,6 @@ int amv_mul_mat_f32(int wtype, const void* w, int64_t n_rows, int64_t k, const f
  * activations' f16 q_a d_a and the matrix cores accumulate across all of k (no per-block epilogue; within ~3e-4
  * relative L2 of the exact form). Up to 32 tokens run the small-batch kernels (Q4_K on the MMA layout's f16 copies; a plain
  * Q8_K activation of Q4_K runs the tiled one).
- * act is read only, except for an AMV_ACT_Q8_0_F6 activation of Q4_0 weights and m > 64: the product writes that layout's
- * scratch part, so such an activation feeds one product at a time (overlapping products on two streams need one each; the
- * plain layout has no such limit).
  * Block sums need a plain or MMA layout. */
 int amv_mul_mat_q_act(int wtype, const void* w, int64_t n_rows, int64_t k, const void* act, int act_type, int64_t m,
                       float* dst, int64_t ldd, void* stream);
