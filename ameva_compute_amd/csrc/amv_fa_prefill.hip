@@ -250,9 +250,9 @@ __global__ __launch_bounds__(256) void k_fa_prefill(const float* __restrict__ q,
 // splitting a tile's keys further. 8 waves: 4 consecutive (query tile, head of the group) pairs of one KV head, head fastest,
 // so with 4 query heads per KV head a block of 32 keys is read from L2 once for 128 query rows (k_fa_prefill reads it once
 // per 32: 1 GB through L2 for 2048 causal tokens of 32 heads); each pair has two waves, which take the even and the odd
-// blocks and merge at the end (one wave per pair: 84 us against 75 before the next point, the longest tiles then run alone).
+// blocks and merge at the end (one wave per pair took 12 % longer: the longest tiles then run alone).
 // A block's exponentials run between the dependent products of the next block's scores. What bounds it: latency, at two
-// waves per SIMD (matrix cores 23 %, VALU 30 % busy).
+// waves per SIMD (2048 causal tokens: matrix cores 22 %, VALU 35 % of the SIMD cycles).
 // K and V rows go from memory to LDS without registers (global_load_lds), one step ahead, double-buffered. The loads write
 // the rows as they come, so pieces of a row are exchanged by an XOR with the key index on the memory side: K 16-byte pieces
 // by key % 16 (the fragment reads of 16 keys hit all banks once), V 32-byte pieces by key % 8 (so do the transposing reads

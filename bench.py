@@ -728,6 +728,33 @@ def pmc_fa(ops, torch, dev):
     print(json.dumps({"fa_dispatches": 20, "kv_bytes_each": 2 * CTX * NKV * D * 2}), flush=True)
 
 
+def pmc_prompt(ops, torch, dev):
+    """Dispatches for the counters of the prompt's kernels, 20 eager launches each: causal attention of 2048 tokens (32 / 8
+    heads of 128), the exact Q4_0 MUL_MAT of 512 tokens on 28672 x 4096, the exact Q8_0 one of 331 tokens on 4096 x 14336;
+    and the decode attention over 8192 Q8_0 keys."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(2048)
+    q = torch.randn((2048, 32, 128), generator=g, device=dev)
+    k, v = (torch.randn((2048, 8, 128), generator=g, device=dev).half().permute(1, 0, 2) for _ in "kv")
+    for _ in range(20):
+        ops.flash_attn_prefill(q, k, v, 128 ** -0.5, causal_pos0=0)
+    for wtype, n, kk, m in ((ops.Q4_0, 28672, 4096, 512), (ops.Q8_0, 4096, 14336, 331)):
+        w = make_weights(ops, torch, n, kk, 1, 300 + n, dev, wtype)[0]
+        act, _ = ops.quantize_act(torch.randn((m, kk), generator=g, device=dev), ops.Q8_0, ops.Q8_X86)
+        out = torch.empty((m, n), dtype=torch.float32, device=dev)
+        for _ in range(20):
+            ops.mul_mat_q(w, act, m, out, act_t=ops.Q8_0)
+    kv = [ops.quantize_act(torch.randn((8192 * 8, 128), generator=g, device=dev), ops.Q8_0, ggml=True)[1]
+          .view(8192, 8, -1).permute(1, 0, 2) for _ in "kv"]
+    ws = torch.empty(ops.lib().amv_flash_attn_workspace_bytes(32, 8, 8192, 128), dtype=torch.uint8, device=dev)
+    for _ in range(20):
+        ops.flash_attn_decode_kv(q[0], kv[0], kv[1], ops.Q8_0, 128 ** -0.5, workspace=ws)
+    torch.cuda.synchronize()
+    print(json.dumps({"dispatches": 20, "attn_flops": 4 * 32 * 128 * 2048 * 2049 // 2,
+                      "q4_0_ops": 2 * 512 * 28672 * 4096, "q8_0_ops": 2 * 331 * 4096 * 14336,
+                      "decode_kv_bytes": 2 * 8192 * 8 * 136}), flush=True)
+
+
 INT8_MFMA_PEAK_TOPS = 5000.0  # MI355X dense int8 matrix peak (5.0 POPS)
 
 
@@ -928,6 +955,9 @@ def main():
                     help="for rocprofv3 --pmc: 20 eager cold Q4_K and Q6_K MUL_MATs at M = 16 (14336 x 4096)")
     ap.add_argument("--pmc-i2s", action="store_true",
                     help="for rocprofv3 --pmc: 20 eager I2_S batch-128 MUL_MATs on each BitNet 2B shape")
+    ap.add_argument("--pmc-prompt", action="store_true",
+                    help="for rocprofv3 --pmc: 20 eager launches each of the prompt's attention and MUL_MAT kernels and of "
+                         "the decode attention over Q8_0 keys")
     ap.add_argument("--pmc-fa", action="store_true",
                     help="for rocprofv3 --pmc: 20 eager cold FA decodes at 4096 keys over an F16 cache")
     args = ap.parse_args()
@@ -953,6 +983,9 @@ def main():
         return
     if args.pmc_small:
         pmc_small(ops, torch, dev)
+        return
+    if args.pmc_prompt:
+        pmc_prompt(ops, torch, dev)
         return
     if args.pmc_fa:
         pmc_fa(ops, torch, dev)
