@@ -182,20 +182,21 @@ class LlamaLayer:
 
     def _prefill_buffers(self, n_tok: int) -> dict:
         """Per-token-count buffers of prefill (allocated on first use; a captured graph must see them allocated). A set
-        per activation layout is held, so that a captured graph keeps its own through prompts of another layout."""
+        per activation layout, and for prompts of up to MMQ16_MIN_M tokens one of their own, is held, so that a captured
+        graph keeps its own through prompts of another layout or, if it is short, through long ones."""
         bufs, at = getattr(self, "_pf", None), ops.gemm_act_type(self.wqkv.type, n_tok)
-        sets = self.__dict__.setdefault("_pf_sets", {})
+        sets, key = self.__dict__.setdefault("_pf_sets", {}), (at, n_tok > ops.MMQ16_MIN_M)
         if bufs is not None:
-            sets[bufs["at"]] = bufs
-        if at in sets and sets[at]["n"] >= n_tok:
-            self._pf = sets[at]
+            sets[bufs["key"]] = bufs
+        if key in sets and sets[key]["n"] >= n_tok:
+            self._pf = sets[key]
             return self._pf
         dev = self.attn_norm.device
         f32 = dict(dtype=torch.float32, device=dev)
         u8 = dict(dtype=torch.uint8, device=dev)
         L = lib()
         H, FF = self.H, self.FF
-        bufs = {"n": n_tok, "at": at,
+        bufs = {"n": n_tok, "at": at, "key": key,
                 "t_o": torch.empty((n_tok, H), **f32), "qkv": torch.empty((n_tok, self.wqkv.n_rows), **f32),
                 "att": torch.empty((n_tok, H), **f32),
                 "x1": torch.empty((n_tok, H), **f32), "t_o2": torch.empty((n_tok, H), **f32),
@@ -207,7 +208,7 @@ class LlamaLayer:
                 "h": torch.empty((n_tok, FF), **f32) if at not in (ops.Q8_0, ops.Q8_K) else None,
                 "pos": torch.zeros(n_tok, dtype=torch.int32, device=dev),
                 "idx": torch.zeros(n_tok, dtype=torch.int64, device=dev)}
-        self._pf = sets[at] = bufs
+        self._pf = sets[key] = bufs
         return bufs
 
     def set_prefill_position(self, pos0: int, n_tok: int) -> None:

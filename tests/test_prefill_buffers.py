@@ -20,6 +20,15 @@ def test_prefill_buffers_kept_per_layout(wtype):
         assert llama.LlamaLayer._prefill_buffers(lay, n) is b
 
 
+@pytest.mark.parametrize("wtype", [ops.Q4_0, ops.Q8_0, ops.Q4_K, ops.Q6_K])
+def test_short_prompt_keeps_its_buffers_through_a_long_one(wtype):
+    lay = types.SimpleNamespace(H=256, FF=512, attn_norm=torch.empty(1), wqkv=types.SimpleNamespace(type=wtype, n_rows=384),
+                                wgu=types.SimpleNamespace(n_rows=1024))
+    short = llama.LlamaLayer._prefill_buffers(lay, 20)
+    long = llama.LlamaLayer._prefill_buffers(lay, 300)
+    assert llama.LlamaLayer._prefill_buffers(lay, 20) is short and llama.LlamaLayer._prefill_buffers(lay, 300) is long
+
+
 @pytest.mark.parametrize("wtypes,n", [((ops.Q4_0, ops.Q8_0), 100), ((ops.Q4_K, ops.Q6_K), 5), ((ops.Q4_K, ops.Q6_K), 20),
                                      ((ops.Q4_K, ops.Q6_K, ops.Q4_K), 40), ((ops.Q8_0, ops.Q4_0, ops.Q8_0), 3)])
 def test_model_positions_reach_every_layer(wtypes, n):
