@@ -3,7 +3,7 @@
 ggml-impl.h): one C probe prints the size and every member offset of each struct and vtable the plugin fills or reads,
 every enum value ggml_abi.h declares and the limits, compiled once against each header set; the two outputs must be
 equal line for line. A header set that gave a vtable one more member, another GGML_MAX_NAME or a renumbered op fails
-here. CPU only; skipped where /root/reference is absent (the GPU box).
+here. CPU only; skipped where /root/reference is absent.
 
 ggml-impl.h includes gguf.h, which the reference does not vendor, so the two graph structs (and the bitset typedef
 of the hash set) are read out of ggml-impl.h's text and compiled after ggml.h (the probe takes nothing else from that
