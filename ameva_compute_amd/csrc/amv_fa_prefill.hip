@@ -408,8 +408,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
         mx = amv_max_x32(mx * f);
         // The weights' reference m: 14 below the running maximum, so that they reach 2^14 and f16 holds them in full down to
         // 2^-28 of the largest (from the maximum itself f16 loses bits 2^-14 below it: a key that outweighs all others, such
-        // as a prompt's first one, then cost the others theirs: one at 11 above the rest with V = 0, error against 64 bits
-        // 2.0e-4, from the maximum 7.7e-3, k_fa_prefill 5.4e-3).
+        // as a prompt's first one, then cost the others theirs: 2048 causal tokens, one key with a score 14 above 0 and V = 0,
+        // error against 64 bits 1.9e-4, from the maximum 5.3e-3).
         float mb = mx - 14.0f;
         if (__builtin_amdgcn_ballot_w64(fabsf(mx) > 0x1p20f)) {  // where no difference of 14 is exact
             // nor one of a score scaled in the fma below, unrounded, and the rounded maximum: it reached f16's infinity
